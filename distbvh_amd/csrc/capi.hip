@@ -1943,10 +1943,9 @@ bvh_status bvh_local_patches(bvh_object o, bvh_patch_info* out, size_t cap) {
   if (n > 0) {
     DevBuf dc;
     BVH_TRY(dc.ensure(3 * od * sizeof(double)));
-    const double* cpl = o->in.kind == kPoly ? o->centroid.as<double>() : nullptr;
-    const double* spl = o->in.kind == kSphere ? o->in.data : nullptr;
-    const double* cao = o->in.kind == kSnapshot ? o->in.centroids : nullptr;
-    HIP_TRY(launch_patch_centroids(cpl, spl, cao, o->ref_perm(), o->splits.as<uint32_t>(), n, od,
+    const double* planes = o->in.kind == kPoly ? o->centroid.as<double>() : o->in.data;  // spheres: x, y, z
+    if (o->in.kind == kSnapshot) planes = nullptr;
+    HIP_TRY(launch_patch_centroids(planes, o->in.centroids, o->ref_perm(), o->splits.as<uint32_t>(), n, od,
                                    dc.as<double>(), s));
     BVH_TRY(copy_out(cent.data(), dc.p, 3 * od * sizeof(double), BVH_MEM_HOST, s));
   }
@@ -2273,10 +2272,9 @@ bvh_status bvh_pack_patches(bvh_object o, void* out, uint64_t cap, uint64_t* byt
   double* cent = o->wire_cent.as<double>();
   HIP_TRY(launch_fill_u32(reinterpret_cast<uint32_t*>(cent), 6 * od, 0u, s));
   if (n > 0) {
-    const double* cpl = o->in.kind == kPoly ? o->centroid.as<double>() : nullptr;
-    const double* spl = o->in.kind == kSphere ? o->in.data : nullptr;
-    const double* cao = o->in.kind == kSnapshot ? o->in.centroids : nullptr;
-    HIP_TRY(launch_patch_centroids(cpl, spl, cao, o->ref_perm(), o->splits.as<uint32_t>(), n, od, cent, s));
+    const double* planes = o->in.kind == kPoly ? o->centroid.as<double>() : o->in.data;  // spheres: x, y, z
+    if (o->in.kind == kSnapshot) planes = nullptr;
+    HIP_TRY(launch_patch_centroids(planes, o->in.centroids, o->ref_perm(), o->splits.as<uint32_t>(), n, od, cent, s));
   }
   void* dst = out;
   if (mem == BVH_MEM_HOST) {

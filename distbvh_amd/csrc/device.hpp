@@ -468,6 +468,33 @@ __device__ __forceinline__ void to_fp32_outward(const double* kd, const double* 
 }
 
 
+// s + p[0] + ... + p[cnt - 1], added in that order (one serial chain).  p is
+// in LDS, read kOrderedBatch values ahead of the adds so that the chain waits
+// for nothing but itself.
+constexpr uint32_t kOrderedBatch = 16;
+__device__ __forceinline__ double ordered_sum(const double* p, uint32_t cnt, double s) {
+  uint32_t i = 0;
+  if (cnt >= kOrderedBatch) {
+    double a[kOrderedBatch];
+#pragma unroll
+    for (uint32_t j = 0; j < kOrderedBatch; ++j) a[j] = p[j];
+    for (; i + 2 * kOrderedBatch <= cnt; i += kOrderedBatch) {
+      double b[kOrderedBatch];
+#pragma unroll
+      for (uint32_t j = 0; j < kOrderedBatch; ++j) b[j] = p[i + kOrderedBatch + j];
+#pragma unroll
+      for (uint32_t j = 0; j < kOrderedBatch; ++j) s = s + a[j];
+#pragma unroll
+      for (uint32_t j = 0; j < kOrderedBatch; ++j) a[j] = b[j];
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < kOrderedBatch; ++j) s = s + a[j];
+    i += kOrderedBatch;
+  }
+  for (; i < cnt; ++i) s = s + p[i];
+  return s;
+}
+
 __device__ __forceinline__ uint32_t lane_id() { return __lane_id(); }
 __device__ __forceinline__ uint64_t lanemask_lt() { return (1ull << lane_id()) - 1ull; }
 
