@@ -233,7 +233,7 @@ struct bvh_object_s {
   DevBuf given;
   std::vector<uint64_t> given_h;
   DevBuf sp_rp, sp_rp_b, sp_scan, sp_tmpf, sp_tmpt, sp_seg, sp_seg_next, sp_k64, sp_acc, sp_axis, sp_flag, sp_lb,
-      sp_ctr, sp_key, key0, key_a, key_b, sp_hist, sp_x;
+      sp_ctr, sp_key, key0, key_a, key_b, sp_hist, sp_x, sp_blk;
   const uint32_t* ref_rp = nullptr;
   const uint32_t* ref_perm() const { return split == BVH_SPLIT_CLUSTERING ? perm.as<uint32_t>() : ref_rp; }
   // results
@@ -308,7 +308,7 @@ struct bvh_object_s {
                      &front_a, &front_b, &patch_k64, &patch_box32, &pairs, &pairs_a, &pairs_b, &records, &ppairs,
                      &sort_hist, &sort_ctl, &sort_lb, &count, &recheck, &digest, &sp_rp, &sp_rp_b,
                      &sp_scan, &sp_tmpf, &sp_tmpt, &sp_seg, &sp_seg_next, &sp_k64, &sp_acc, &sp_axis,
-                     &sp_flag, &sp_lb, &sp_ctr, &sp_key, &key0, &key_a, &key_b, &sp_hist, &sp_x,
+                     &sp_flag, &sp_lb, &sp_ctr, &sp_key, &key0, &key_a, &key_b, &sp_hist, &sp_x, &sp_blk,
                      &ex_flag, &ex_out, &ex_lb, &ex_ctr, &wire_cent, &wire_range, &wire_src, &wire_out,
                      &given};
     for (DevBuf* d : all) f(*d);
@@ -466,7 +466,7 @@ static bvh_status object_alloc(bvh_object_s* o) {
     BVH_TRY(o->sp_k64.ensure(od * kSlabs * 8));
     BVH_TRY(o->sp_acc.ensure(od * 5 * sizeof(double)));
     BVH_TRY(o->sp_axis.ensure(od * 4));
-    BVH_TRY(o->sp_flag.ensure(od * 2 * 4));
+    BVH_TRY(o->sp_flag.ensure(od * 4));
     BVH_TRY(o->sp_lb.ensure(sort_tiles(n1 + 1) * 8));
     BVH_TRY(o->sp_ctr.ensure(4));
     BVH_TRY(o->sp_key.ensure(n1 * 4));
@@ -475,6 +475,7 @@ static bvh_status object_alloc(bvh_object_s* o) {
     BVH_TRY(o->key_b.ensure(n1 * 4));
     BVH_TRY(o->sp_hist.ensure(2 * 256 * 4));
     BVH_TRY(o->sp_x.ensure(n1 * sizeof(double)));
+    BVH_TRY(o->sp_blk.ensure(split_blocks(n1) * sizeof(SplitBlock)));
   }
   return BVH_OK;
 }
@@ -508,6 +509,7 @@ static bvh_status split_and_order(bvh_object_s* o) {
   sb.scan_lb = o->sp_lb.as<uint64_t>();
   sb.scan_ctr = o->sp_ctr.as<uint32_t>();
   sb.xbuf = o->sp_x.as<double>();
+  sb.blk = o->sp_blk.as<SplitBlock>();
   uint32_t* rp = nullptr;
   uint32_t* patch_key = o->sp_key.as<uint32_t>();
   if (o->split == BVH_SPLIT_GIVEN)

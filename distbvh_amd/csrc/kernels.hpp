@@ -159,6 +159,18 @@ struct SplitInput {
   const double* caos;
   uint64_t n;
 };
+// blocks of consecutive positions of the exact split points (split.hip): the
+// sums of a block's projections, then how the block moves the rounded sum: d0
+// / d1 by the sum's parity, in units of the binade `key` names (2 x its
+// exponent, + 1 for negative sums), or kExactNone for serial adds
+constexpr uint32_t kExactBlock = 512;
+constexpr int32_t kExactNone = INT32_MIN;
+struct SplitBlock {
+  double sum, mag;
+  long long d0, d1;
+  int32_t key, pad;
+};
+inline uint64_t split_blocks(uint64_t n) { return (n + kExactBlock - 1) / kExactBlock; }
 struct SplitBufs {
   uint32_t* rp;        // n: position -> input index (the reference order)
   uint32_t* rp_b;      // n
@@ -170,10 +182,11 @@ struct SplitBufs {
   unsigned long long* seg_k64;  // od x 26: union of the range's element k-DOPs (ordered u64)
   double* seg_acc;     // od x 5: sum, sum of magnitudes, interval lo, hi, exact split point
   int32_t* seg_axis;   // od
-  uint32_t* seg_flag;  // od x 2: undecided elements, partition point (kEnd: nothing moves)
+  uint32_t* seg_flag;  // od: has undecided elements
   uint64_t* scan_lb;   // sort_tiles(n + 1) words
   uint32_t* scan_ctr;  // 1
-  double* xbuf;        // n: projections in range order (ranges that need the exact split point)
+  double* xbuf;        // n: projections in range order
+  SplitBlock* blk;     // split_blocks(n)
 };
 // The permutation (*result, one of sb.rp / sb.rp_b), the od - 1 split
 // offsets in the reference's order and the patch of every input element;

@@ -1,9 +1,13 @@
 """Sums that are rounded in element order, on the GPU: the patch centroids, at
-the sizes where the staged chunks end, against the same sums one by one."""
+the sizes where the staged chunks end, against the same sums one by one, and
+the splitters' split points, at the sizes where blocks of elements end, on
+inputs whose order-rounded sum decides where an element goes, against the
+oracle's permutations."""
 import numpy as np
 import pytest
 
-from distbvh_amd import GIVEN, CollisionWorld
+import oracle as O
+from distbvh_amd import GEOM_AXIS, GIVEN, ML_GEOM_AXIS, CollisionWorld
 from helpers import to_cuda
 
 pytestmark = pytest.mark.gpu
@@ -44,3 +48,41 @@ def test_patch_centroids_at_chunk_edges(kind):
         want = _ordered_mean(c[:, off[k]:off[k + 1]]) if m else np.zeros(3)
         assert got[k]["size"] == m
         assert np.array_equal(got[k]["centroid"], want), (k, m)
+
+
+def _split_line(kind, n, rng):
+    """x of n points whose mean is one of them, so that the rounded sum decides."""
+    k = np.arange(n) - (n - 1) // 2
+    if kind == "tenths":  # one sign, inexact steps
+        x = 1000.0 + 0.1 * k
+    elif kind == "negative":
+        x = -5.0 + 0.001 * k
+    elif kind == "mixed":  # partial sums through zero and many binades
+        x = 0.1 * k
+    elif kind == "ties":  # steps of a quarter ulp of the sum: halfway cases
+        x = 2.0 ** 40 + 2.0 ** -12 * k
+    else:  # one huge element first, then small ones against its ulp
+        x = 3.0 + rng.integers(0, 8, n) * 0.25
+        x[0] = 2.0 ** 52
+        return x
+    return x if kind == "mixed" else x[rng.permutation(n)]
+
+
+@pytest.mark.parametrize("ml", [False, True])
+@pytest.mark.parametrize("kind", ["tenths", "negative", "mixed", "ties", "huge"])
+@pytest.mark.parametrize("n", [1, 2, 3, 511, 512, 513, 1023, 1025, 1537, 4097, 33001])
+def test_split_points_at_block_edges(n, kind, ml):
+    rng = np.random.default_rng(n)
+    d = np.zeros((4, n))
+    d[0] = _split_line(kind, n, rng)
+    d[1] = 0.25 * rng.integers(0, 3, n)
+    d[3] = 0.125
+    kd, ce = O.elements_sphere(d)
+    od = 8
+    idx, sp = O.split_permutations(kd, ce, 3, ml=ml)
+    with CollisionWorld(od) as w:
+        o = w.create_collision_object()
+        o.set_entity_data_sphere(to_cuda(d), split_algorithm=ML_GEOM_AXIS if ml else GEOM_AXIS)
+        parts = [o.patch_elements(k) for k in range(od)]
+    assert np.array_equal(np.concatenate(parts).astype(np.uint32), idx)
+    assert np.array_equal(np.cumsum([len(p) for p in parts])[:-1].astype(np.uint64), sp)
