@@ -528,7 +528,7 @@ static bvh_status split_and_order(bvh_object_s* o) {
   SortArgs<uint32_t> a{};
   a.k0 = o->key0.as<uint32_t>(); a.ka = o->key_a.as<uint32_t>(); a.kb = o->key_b.as<uint32_t>();
   a.v0 = o->bb.perm; a.va = o->bb.perm_b; a.vb = sb.tmpf;  // tmpf is free once the splitter is done
-  a.n = n; a.ntiles = sort_tiles(n); a.ctl = o->bb.ctl + 1; a.lookback = o->bb.lookback;
+  a.n = n; a.ctl = o->bb.ctl + 1; a.lookback = o->bb.lookback;
   HIP_TRY(launch_sort_passes<uint32_t>(a, npass, o->sp_hist.as<uint32_t>(), s));
   HIP_TRY(launch_copy<uint32_t>(o->bb.perm, o->bb.perm_b, n, s));
   if (o->bits == 63)
@@ -573,14 +573,14 @@ static void object_build_steps(bvh_object_s* o, std::vector<BuildStep>& st) {
         SortArgs<uint64_t> a{};
         a.k0 = (const uint64_t*)o->bb.codes0; a.ka = (uint64_t*)o->bb.codes_a; a.kb = (uint64_t*)o->bb.codes_b;
         a.v0 = nullptr; a.va = o->bb.perm; a.vb = o->bb.perm_b;
-        a.n = n; a.ntiles = sort_tiles(n); a.ctl = o->bb.ctl; a.lookback = o->bb.lookback;
+        a.n = n; a.ctl = o->bb.ctl; a.lookback = o->bb.lookback;
         HIP_TRY(p < 0 ? launch_sort_plan<uint64_t>(a, npass, o->bb.hist, s, kHistCopies, kHistWords)
                       : launch_sort_pass<uint64_t>(a, p, s));
       } else {
         SortArgs<uint32_t> a{};
         a.k0 = (const uint32_t*)o->bb.codes0; a.ka = (uint32_t*)o->bb.codes_a; a.kb = (uint32_t*)o->bb.codes_b;
         a.v0 = nullptr; a.va = o->bb.perm; a.vb = o->bb.perm_b;
-        a.n = n; a.ntiles = sort_tiles(n); a.ctl = o->bb.ctl; a.lookback = o->bb.lookback;
+        a.n = n; a.ctl = o->bb.ctl; a.lookback = o->bb.lookback;
         HIP_TRY(p < 0 ? launch_sort_plan<uint32_t>(a, npass, o->bb.hist, s, kHistCopies, kHistWords)
                       : launch_sort_pass<uint32_t>(a, p, s));
       }
@@ -937,7 +937,7 @@ static bvh_status sort_results(bvh_object_s* o) {
   SortArgs<uint64_t> a{};
   a.k0 = o->pairs.as<uint64_t>(); a.ka = o->pairs_a.as<uint64_t>(); a.kb = o->pairs_b.as<uint64_t>();
   a.v0 = nullptr; a.va = nullptr; a.vb = nullptr;
-  a.n = n; a.ntiles = tiles; a.ctl = o->sort_ctl.as<SortCtl>(); a.lookback = o->sort_lb.as<uint32_t>();
+  a.n = n; a.ctl = o->sort_ctl.as<SortCtl>(); a.lookback = o->sort_lb.as<uint32_t>();
   HIP_TRY(launch_sort_passes<uint64_t>(a, 8, o->sort_hist.as<uint32_t>(), s));
   o->result_ptr = o->pairs_a.as<uint64_t>();
   return BVH_OK;
@@ -1232,7 +1232,7 @@ static bvh_status sort_in_place(bvh_world w, K* keys, uint32_t* vals, uint64_t n
   SortArgs<K> a{};
   a.k0 = keys; a.ka = static_cast<K*>(sc.ka); a.kb = static_cast<K*>(sc.kb);
   a.v0 = vals; a.va = vals ? sc.va : nullptr; a.vb = vals ? sc.vb : nullptr;
-  a.n = n; a.ntiles = tiles; a.ctl = sc.ctl; a.lookback = sc.lb;
+  a.n = n; a.ctl = sc.ctl; a.lookback = sc.lb;
   HIP_TRY(launch_sort_passes<K>(a, npass, sc.hist, s));
   HIP_TRY(hipMemcpyAsync(keys, a.ka, n * sizeof(K), hipMemcpyDeviceToDevice, s));
   if (vals) HIP_TRY(hipMemcpyAsync(vals, a.va, n * 4, hipMemcpyDeviceToDevice, s));

@@ -27,9 +27,9 @@ struct SortArgs {
   uint32_t* va;
   uint32_t* vb;
   uint64_t n;
-  uint64_t ntiles;
+  uint64_t ntiles;     // set by launch_sort_pass (the shape's tiles)
   SortCtl* ctl;
-  uint32_t* lookback;  // npass * ntiles * 256 words, zero before the sort
+  uint32_t* lookback;  // npass * sort_tiles(n) * 256 words, zero before the sort
 };
 
 uint64_t sort_tiles(uint64_t n);

@@ -5,11 +5,11 @@
 // split pass (3 dispatches) per key bit.  The result is the same stable
 // permutation: keys ascending, ties in input order.
 //
-// Per pass, a 256-thread workgroup takes a 4096-key tile (tile ids come from
-// an atomic counter, so a tile only ever waits on tiles already running):
-//  * keys are read coalesced (wave w, iteration j, lane l -> tile position
-//    w*1024 + j*64 + l) and ranked per wave with 8 ballots per iteration
-//    (the lanes holding the same digit) plus per-wave LDS digit counters;
+// Per pass, a workgroup takes a tile of 4,096 or 8,192 keys (tile ids come
+// from an atomic counter, so a tile only ever waits on tiles already running):
+//  * keys are read coalesced (a wave's items are consecutive runs of 64) and
+//    ranked per wave with 8 ballots per item (the lanes holding the same
+//    digit) plus per-wave LDS digit counters;
 //  * the tile's 256 digit counts are published as an aggregate, then each
 //    thread (= digit) walks back over earlier tiles until it meets an
 //    inclusive prefix (flag and count packed in one 32-bit word, agent-scope
@@ -24,12 +24,28 @@
 
 namespace dbvh {
 
-constexpr int kSortBlock = 256;
-constexpr int kSortItems = 16;
-constexpr int kSortTile = kSortBlock * kSortItems;  // 4096
+// The two shapes of a pass.  Narrow: 1,024 threads x 4 keys, keys and payloads
+// in LDS together; its tile's latency is the shortest (4 serial ranking steps
+// a wave), which is what bounds a sort of few tiles.  Wide: 512 threads x 16
+// keys, payloads after the keys through the same LDS, so that two workgroups
+// share a CU (72 KB each) and one's ranking hides the other's memory time,
+// and the digit runs written are twice as long.  Per 8-bit pass of u64 keys
+// with payloads, narrow / wide: 54,612 keys 9.1 / 13.8 us, 524,288 13.7 / 17.3,
+// 2,097,152 25.0 / 23.4, 12,000,017 104.9 / 81.3 (one shape of 256 threads x
+// 16 keys: 13.3, 18.0, 28.8, 118.7): the line lies between the last two of
+// these sizes where the wide one wins.
+template <bool WIDE>
+struct SortShape {
+  static constexpr int block = WIDE ? 512 : 1024;
+  static constexpr int items = WIDE ? 16 : 4;
+  static constexpr int tile = block * items;
+};
+constexpr uint64_t kSortWideMin = 3ull << 19;  // 1,572,864 keys
 constexpr uint32_t kFlagAgg = 1u << 30;
 constexpr uint32_t kFlagInc = 2u << 30;
 constexpr uint32_t kValMask = (1u << 30) - 1u;
+constexpr int kScanItems = 16;
+constexpr int kScanTile = 256 * kScanItems;
 constexpr int kLookWindow = 4;  // predecessors read per look-back round trip
 
 __device__ __forceinline__ uint32_t lb_load(const uint32_t* p) {
@@ -38,8 +54,6 @@ __device__ __forceinline__ uint32_t lb_load(const uint32_t* p) {
 __device__ __forceinline__ void lb_store(uint32_t* p, uint32_t v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-
-__device__ __forceinline__ uint64_t sort_tiles_dev(uint64_t n) { return (n + kSortTile - 1) / kSortTile; }
 
 // Exclusive scan of one value per thread over a 256-thread block.
 __device__ __forceinline__ uint32_t block_excl_scan256(uint32_t v, uint32_t* s_tmp /*4*/) {
@@ -169,8 +183,21 @@ __global__ __launch_bounds__(256) void k_sort_plan(const uint32_t* __restrict__ 
   }
 }
 
-template <typename K>
-__global__ __launch_bounds__(kSortBlock) void k_sort_pass(SortArgs<K> a, int pass) {
+// Keeps in (lo, hi), a lane mask, the lanes whose bit b of d equals this
+// lane's: m & ~(ballot ^ own bit), one three-input operation per half.
+__device__ __forceinline__ void match_bit(uint32_t d, int b, uint32_t& lo, uint32_t& hi) {
+  const int own = (int)(d << (31 - b)) >> 31;
+  const uint64_t bb = __ballot(own != 0);
+  lo = (uint32_t)__builtin_amdgcn_bitop3_b32((int)lo, (int)(uint32_t)bb, own, 0x90);
+  hi = (uint32_t)__builtin_amdgcn_bitop3_b32((int)hi, (int)(uint32_t)(bb >> 32), own, 0x90);
+}
+
+// One digit pass over one tile.  Bound by the VALU work of the ranking (about
+// 45 instructions a key) beside the memory time of 24 bytes a key.
+template <typename K, bool WIDE>
+__global__ __launch_bounds__(SortShape<WIDE>::block) void k_sort_pass(SortArgs<K> a, int pass) {
+  constexpr int kBlock = SortShape<WIDE>::block, kItems = SortShape<WIDE>::items, kTile = SortShape<WIDE>::tile;
+  constexpr int kWaves = kBlock / 64;
   const SortPassInfo pi = a.ctl->pass[pass];
   if (!pi.active) return;
   const K* __restrict__ kin = pi.in_sel == 0 ? a.k0 : (pi.in_sel == 1 ? a.ka : a.kb);
@@ -182,133 +209,158 @@ __global__ __launch_bounds__(kSortBlock) void k_sort_pass(SortArgs<K> a, int pas
   const uint64_t n = a.n;
 
   __shared__ uint32_t s_tile;
-  __shared__ uint32_t s_wcount[4][256];
+  __shared__ __align__(4) uint16_t s_wcount[kWaves][256];  // (a tile's counts fit 16 bits)
   __shared__ uint32_t s_texcl[256];
   __shared__ uint32_t s_gbase[256];
   __shared__ uint32_t s_tmp[4];
   __shared__ uint32_t s_hist[256];
-  __shared__ K s_keys[kSortTile];
-  __shared__ uint32_t s_vals[kSortTile];
+  __shared__ __align__(16) unsigned char s_buf[kTile * (WIDE ? sizeof(K) : sizeof(K) + 4)];
+  K* s_keys = (K*)s_buf;
+  uint32_t* s_vals = (uint32_t*)(WIDE ? s_buf : s_buf + kTile * sizeof(K));
 
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
   if (tid == 0) s_tile = atomicAdd(&a.ctl->tile_counter[pass], 1u);
-  for (int i = tid; i < 4 * 256; i += kSortBlock) (&s_wcount[0][0])[i] = 0;
-  s_hist[tid] = 0;
+  for (int i = tid; i < kWaves * 128; i += kBlock) ((uint32_t*)&s_wcount[0][0])[i] = 0;
+  if (tid < 256) s_hist[tid] = 0;
   __syncthreads();
   const uint32_t tile = s_tile;
   if (tile >= a.ntiles) return;  // uniform per block; no tile waits on it
-  const uint64_t base = (uint64_t)tile * kSortTile;
+  const uint64_t base = (uint64_t)tile * kTile;
+  const uint32_t cnt = (uint32_t)(n - base < (uint64_t)kTile ? n - base : (uint64_t)kTile);
 
-  K key[kSortItems];
-  uint32_t val[kSortItems];
-  uint32_t rank[kSortItems];
-  uint32_t dig[kSortItems];
+  // this thread's keys: tile positions p0 + 64 j
+  const uint32_t p0 = (uint32_t)(w * (kItems * 64) + lane);
+  K key[kItems];
+  uint32_t val[kItems];
+  uint32_t rank[kItems];
 #pragma unroll
-  for (int j = 0; j < kSortItems; ++j) {
-    uint64_t pos = base + (uint64_t)(w * (kSortItems * 64) + j * 64 + lane);
-    bool valid = pos < n;
+  for (int j = 0; j < kItems; ++j) {
+    const uint64_t pos = base + (p0 + j * 64);
+    const bool valid = pos < n;
     key[j] = valid ? kin[pos] : (K)0;
     if (has_vals) val[j] = valid ? (vin ? vin[pos] : (uint32_t)pos) : 0u;
-    dig[j] = valid ? (uint32_t)((key[j] >> shift) & 255) : 256u;
   }
+  auto valid = [&](int j) { return p0 + j * 64 < cnt; };
+  auto digit = [&](K k) { return (uint32_t)(k >> shift) & 255u; };
   // the tile's digit counts first, published as its aggregate before the
   // ranking, so that later tiles' look-backs find it sooner
 #pragma unroll
-  for (int j = 0; j < kSortItems; ++j)
-    if (dig[j] < 256u) atomicAdd(&s_hist[dig[j]], 1u);
+  for (int j = 0; j < kItems; ++j)
+    if (valid(j)) atomicAdd(&s_hist[digit(key[j])], 1u);
   __syncthreads();
   uint32_t* lb = a.lookback + ((uint64_t)pass * a.ntiles + tile) * 256;
-  {
-    const uint32_t tot = s_hist[tid];
-    if (tile == 0) lb_store(&lb[tid], kFlagInc | tot);
-    else lb_store(&lb[tid], kFlagAgg | tot);
+  uint32_t total = 0;
+  if (tid < 256) {
+    total = s_hist[tid];
+    lb_store(&lb[tid], (tile == 0 ? kFlagInc : kFlagAgg) | total);
   }
-  const uint64_t lt = lanemask_lt();
 #pragma unroll
-  for (int j = 0; j < kSortItems; ++j) {
-    const uint32_t d = dig[j];
-    const bool valid = d < 256u;
-    uint64_t m = __ballot(valid);
+  for (int j = 0; j < kItems; ++j) {
+    const uint32_t d = digit(key[j]);
+    const bool ok = valid(j);
+    const uint64_t m = __ballot(ok);
+    uint32_t lo = (uint32_t)m, hi = (uint32_t)(m >> 32);
 #pragma unroll
-    for (int b = 0; b < 8; ++b) {
-      const bool bit = (d >> b) & 1u;
-      const uint64_t bb = __ballot(bit);
-      m &= bit ? bb : ~bb;
-    }
-    const uint32_t before = __popcll(m & lt);
+    for (int b = 0; b < 8; ++b) match_bit(d, b, lo, hi);
+    const uint32_t before = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
+    const uint32_t same = (uint32_t)(__popc(lo) + __popc(hi));
     uint32_t old = 0;
-    if (valid) old = s_wcount[w][d];
+    if (ok) old = s_wcount[w][d];
     rank[j] = old + before;
     __builtin_amdgcn_wave_barrier();
-    if (valid && before == 0) s_wcount[w][d] = old + (uint32_t)__popcll(m);
+    if (ok && before == 0) s_wcount[w][d] = (uint16_t)(old + same);
     __builtin_amdgcn_wave_barrier();
   }
   __syncthreads();
 
-  // thread t owns digit t
-  const int t = tid;
-  uint32_t c0 = s_wcount[0][t], c1 = s_wcount[1][t], c2 = s_wcount[2][t], c3 = s_wcount[3][t];
-  const uint32_t total = c0 + c1 + c2 + c3;
+  // thread t < 256 owns digit t: exclusive scans over the waves and the digits
+  uint32_t x = total;
+  if (tid < 256) {
+    uint32_t run = 0;
+#pragma unroll
+    for (int v = 0; v < kWaves; ++v) {
+      const uint32_t c = s_wcount[v][tid];
+      s_wcount[v][tid] = (uint16_t)run;
+      run += c;
+    }
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t y = __shfl_up(x, o, 64);
+      if (lane >= o) x += y;
+    }
+    if (lane == 63) s_tmp[w] = x;
+  }
   __syncthreads();
-  s_wcount[0][t] = 0;
-  s_wcount[1][t] = c0;
-  s_wcount[2][t] = c0 + c1;
-  s_wcount[3][t] = c0 + c1 + c2;
-
-  const uint32_t texcl = block_excl_scan256(total, s_tmp);
-  s_texcl[t] = texcl;
-
-  uint32_t excl = 0;
-  if (tile > 0) {
-    // decoupled look-back over a window of kLookWindow predecessors whose
-    // words are loaded together (one round trip per window, not per tile):
-    // their aggregates are added in order up to the first inclusive prefix;
-    // a word not yet published is polled until it is (tile 0 publishes an
-    // inclusive prefix, so the walk ends by it)
-    const uint32_t* lb0 = a.lookback + (uint64_t)pass * a.ntiles * 256 + t;
-    int64_t prev = (int64_t)tile - 1;
-    bool done = false;
-    while (!done) {
-      uint32_t v[kLookWindow];
+  if (tid < 256) {
+    uint32_t texcl = x - total;
+    for (int i = 0; i < w; ++i) texcl += s_tmp[i];
+    s_texcl[tid] = texcl;
+    uint32_t excl = 0;
+    if (tile > 0) {
+      // decoupled look-back over a window of kLookWindow predecessors whose
+      // words are loaded together (one round trip per window, not per tile):
+      // their aggregates are added in order up to the first inclusive prefix;
+      // a word not yet published is polled until it is (tile 0 publishes an
+      // inclusive prefix, so the walk ends by it)
+      const uint32_t* lb0 = a.lookback + (uint64_t)pass * a.ntiles * 256 + tid;
+      int64_t prev = (int64_t)tile - 1;
+      bool done = false;
+      while (!done) {
+        uint32_t v[kLookWindow];
 #pragma unroll
-      for (int k = 0; k < kLookWindow; ++k) v[k] = prev - k >= 0 ? lb_load(lb0 + (uint64_t)(prev - k) * 256) : 0u;
+        for (int k = 0; k < kLookWindow; ++k) v[k] = prev - k >= 0 ? lb_load(lb0 + (uint64_t)(prev - k) * 256) : 0u;
 #pragma unroll
-      for (int k = 0; k < kLookWindow; ++k) {
-        if (done || prev - k < 0) break;
-        uint32_t x = v[k];
-        while ((x & ~kValMask) == 0) {
-          __builtin_amdgcn_s_sleep(1);
-          x = lb_load(lb0 + (uint64_t)(prev - k) * 256);
+        for (int k = 0; k < kLookWindow; ++k) {
+          if (done || prev - k < 0) break;
+          uint32_t y = v[k];
+          while ((y & ~kValMask) == 0) {
+            __builtin_amdgcn_s_sleep(1);
+            y = lb_load(lb0 + (uint64_t)(prev - k) * 256);
+          }
+          excl += y & kValMask;
+          done = (y & ~kValMask) == kFlagInc;
         }
-        excl += x & kValMask;
-        done = (x & ~kValMask) == kFlagInc;
+        prev -= kLookWindow;
       }
-      prev -= kLookWindow;
+      lb_store(&lb[tid], kFlagInc | (excl + total));
     }
-    lb_store(&lb[t], kFlagInc | (excl + total));
+    s_gbase[tid] = a.ctl->offsets[pass * 256 + tid] + excl - texcl;  // + tile-local place = output position
   }
-  s_gbase[t] = a.ctl->offsets[pass * 256 + t] + excl;
   __syncthreads();
 
 #pragma unroll
-  for (int j = 0; j < kSortItems; ++j) {
-    const uint32_t d = dig[j];
-    if (d < 256u) {
-      const uint32_t lp = s_texcl[d] + s_wcount[w][d] + rank[j];
-      s_keys[lp] = key[j];
-      if (has_vals) s_vals[lp] = val[j];
+  for (int j = 0; j < kItems; ++j) {
+    const uint32_t d = digit(key[j]);
+    rank[j] += s_texcl[d] + s_wcount[w][d];  // now the place in the tile's output
+    if (valid(j)) {
+      s_keys[rank[j]] = key[j];
+      if (!WIDE && has_vals) s_vals[rank[j]] = val[j];
     }
   }
   __syncthreads();
-  const uint32_t cnt = (uint32_t)((n - base) < (uint64_t)kSortTile ? (n - base) : (uint64_t)kSortTile);
-  for (uint32_t i = tid; i < cnt; i += kSortBlock) {
-    const K k = s_keys[i];
-    const uint32_t d = (uint32_t)((k >> shift) & 255);
-    const uint32_t op = s_gbase[d] + (i - s_texcl[d]);
-    if (op < n) {
-      kout[op] = k;
-      if (has_vals) vout[op] = s_vals[i];
+  uint32_t op[kItems];
+#pragma unroll
+  for (int j = 0; j < kItems; ++j) {
+    const uint32_t i = j * kBlock + tid;
+    op[j] = kEnd;
+    if (i < cnt) {
+      const K k = s_keys[i];
+      op[j] = s_gbase[digit(k)] + i;
+      if (op[j] < n) {
+        kout[op[j]] = k;
+        if (!WIDE && has_vals) vout[op[j]] = s_vals[i];
+      }
     }
+  }
+  if (WIDE && has_vals) {
+    __syncthreads();  // the keys in LDS have been read
+#pragma unroll
+    for (int j = 0; j < kItems; ++j)
+      if (valid(j)) s_vals[rank[j]] = val[j];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kItems; ++j)
+      if (op[j] < n) vout[op[j]] = s_vals[j * kBlock + tid];
   }
 }
 
@@ -332,7 +384,9 @@ __global__ void k_copy(T* __restrict__ dst, const T* __restrict__ src, uint64_t 
 }
 
 // ---- host launchers ----------------------------------------------------------------
-uint64_t sort_tiles(uint64_t n) { return (n + kSortTile - 1) / kSortTile; }
+// tiles of the narrow shape and of the scan: what callers size look-back
+// words by (the wide shape has fewer)
+uint64_t sort_tiles(uint64_t n) { return (n + kScanTile - 1) / kScanTile; }
 
 hipError_t launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t s) {
   if (n == 0) return hipSuccess;
@@ -387,7 +441,16 @@ hipError_t launch_sort_plan(const SortArgs<K>& a, int npass, const uint32_t* his
 template <typename K>
 hipError_t launch_sort_pass(const SortArgs<K>& a, int p, hipStream_t s) {
   if (a.n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_sort_pass<K>, dim3((unsigned)sort_tiles(a.n)), dim3(kSortBlock), 0, s, a, p);
+  SortArgs<K> b = a;
+  if (a.n >= kSortWideMin) {
+    using S = SortShape<true>;
+    b.ntiles = (a.n + S::tile - 1) / S::tile;
+    hipLaunchKernelGGL((k_sort_pass<K, true>), dim3((unsigned)b.ntiles), dim3(S::block), 0, s, b, p);
+  } else {
+    using S = SortShape<false>;
+    b.ntiles = (a.n + S::tile - 1) / S::tile;
+    hipLaunchKernelGGL((k_sort_pass<K, false>), dim3((unsigned)b.ntiles), dim3(S::block), 0, s, b, p);
+  }
   return hipGetLastError();
 }
 
@@ -424,12 +487,12 @@ __global__ __launch_bounds__(256) void k_scan_u32(uint32_t* __restrict__ v, uint
   if (tid == 0) s_tile = atomicAdd(counter, 1u);
   __syncthreads();
   const uint32_t tile = s_tile;
-  if ((uint64_t)tile >= sort_tiles_dev(n)) return;
-  const uint64_t base = (uint64_t)tile * kSortTile + (uint64_t)tid * kSortItems;
-  uint32_t x[kSortItems];
+  if ((uint64_t)tile * kScanTile >= n) return;
+  const uint64_t base = (uint64_t)tile * kScanTile + (uint64_t)tid * kScanItems;
+  uint32_t x[kScanItems];
   uint32_t sum = 0;
 #pragma unroll
-  for (int j = 0; j < kSortItems; ++j) {
+  for (int j = 0; j < kScanItems; ++j) {
     const uint64_t i = base + j;
     x[j] = i < n ? v[i] : 0u;
     sum += x[j];
@@ -460,7 +523,7 @@ __global__ __launch_bounds__(256) void k_scan_u32(uint32_t* __restrict__ v, uint
   __syncthreads();
   uint32_t run = (uint32_t)s_excl + texcl;
 #pragma unroll
-  for (int j = 0; j < kSortItems; ++j) {
+  for (int j = 0; j < kScanItems; ++j) {
     const uint64_t i = base + j;
     if (i < n) v[i] = run;
     run += x[j];
