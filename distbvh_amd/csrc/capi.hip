@@ -473,7 +473,7 @@ static bvh_status object_alloc(bvh_object_s* o) {
     BVH_TRY(o->key0.ensure(n1 * 4));
     BVH_TRY(o->key_a.ensure(n1 * 4));
     BVH_TRY(o->key_b.ensure(n1 * 4));
-    BVH_TRY(o->sp_hist.ensure(2 * 256 * 4));
+    BVH_TRY(o->sp_hist.ensure(kHistCopies * kSortHistWords * 4));
     BVH_TRY(o->sp_x.ensure(n1 * sizeof(double)));
     BVH_TRY(o->sp_blk.ensure(split_blocks(n1) * sizeof(SplitBlock)));
   }
@@ -520,16 +520,13 @@ static bvh_status split_and_order(bvh_object_s* o) {
   o->ref_rp = rp;
   // stable sort of the Morton order by patch
   HIP_TRY(launch_gather_by<uint32_t>(patch_key, o->bb.perm, n, o->key0.as<uint32_t>(), s));
-  const int npass = od <= 256 ? 1 : (od <= 65536 ? 2 : 4);
-  HIP_TRY(launch_fill_u32(o->sp_hist.as<uint32_t>(), 2 * 256, 0u, s));
-  HIP_TRY(launch_fill_u32(o->bb.lookback, (uint64_t)(npass > 2 ? 2 : npass) * sort_tiles(n) * 256, 0u, s));
-  if (npass > 2) return fail(BVH_E_UNSUPPORTED, "geom_axis splitting supports at most 65536 patches");
-  HIP_TRY(launch_sort_histogram<uint32_t>(o->key0.as<uint32_t>(), n, npass, o->sp_hist.as<uint32_t>(), s));
+  const int npass = od <= 256 ? 1 : 2;
+  if (od > 65536) return fail(BVH_E_UNSUPPORTED, "geom_axis splitting supports at most 65536 patches");
   SortArgs<uint32_t> a{};
   a.k0 = o->key0.as<uint32_t>(); a.ka = o->key_a.as<uint32_t>(); a.kb = o->key_b.as<uint32_t>();
   a.v0 = o->bb.perm; a.va = o->bb.perm_b; a.vb = sb.tmpf;  // tmpf is free once the splitter is done
   a.n = n; a.ctl = o->bb.ctl + 1; a.lookback = o->bb.lookback;
-  HIP_TRY(launch_sort_passes<uint32_t>(a, npass, o->sp_hist.as<uint32_t>(), s));
+  HIP_TRY(launch_sort<uint32_t>(a, npass, o->sp_hist.as<uint32_t>(), s));
   HIP_TRY(launch_copy<uint32_t>(o->bb.perm, o->bb.perm_b, n, s));
   if (o->bits == 63)
     HIP_TRY(launch_gather_by<uint64_t>((const uint64_t*)o->bb.codes0, o->bb.perm, n, (uint64_t*)o->bb.codes_a, s));
@@ -927,18 +924,14 @@ static bvh_status sort_results(bvh_object_s* o) {
   if (n >= (1ull << 30)) return fail(BVH_E_UNSUPPORTED, "sort_results holds at most 2^30 - 1 pairs");
   BVH_TRY(o->pairs_a.ensure(n * 8));
   BVH_TRY(o->pairs_b.ensure(n * 8));
-  BVH_TRY(o->sort_hist.ensure(8 * 256 * 4));
+  BVH_TRY(o->sort_hist.ensure(kHistCopies * kSortHistWords * 4));
   BVH_TRY(o->sort_ctl.ensure(sizeof(SortCtl)));
-  const uint64_t tiles = sort_tiles(n);
-  BVH_TRY(o->sort_lb.ensure(8 * tiles * 256 * 4));
-  HIP_TRY(launch_fill_u32(o->sort_hist.as<uint32_t>(), 8 * 256, 0u, s));
-  HIP_TRY(launch_fill_u32(o->sort_lb.as<uint32_t>(), 8 * tiles * 256, 0u, s));
-  HIP_TRY(launch_sort_histogram<uint64_t>(o->pairs.as<uint64_t>(), n, 8, o->sort_hist.as<uint32_t>(), s));
+  BVH_TRY(o->sort_lb.ensure(8 * sort_tiles(n) * 256 * 4));
   SortArgs<uint64_t> a{};
   a.k0 = o->pairs.as<uint64_t>(); a.ka = o->pairs_a.as<uint64_t>(); a.kb = o->pairs_b.as<uint64_t>();
   a.v0 = nullptr; a.va = nullptr; a.vb = nullptr;
   a.n = n; a.ctl = o->sort_ctl.as<SortCtl>(); a.lookback = o->sort_lb.as<uint32_t>();
-  HIP_TRY(launch_sort_passes<uint64_t>(a, 8, o->sort_hist.as<uint32_t>(), s));
+  HIP_TRY(launch_sort<uint64_t>(a, 8, o->sort_hist.as<uint32_t>(), s));
   o->result_ptr = o->pairs_a.as<uint64_t>();
   return BVH_OK;
 }
@@ -1206,8 +1199,8 @@ static bvh_status results_ready(bvh_object_s* o) {
 
 // ---- stand-alone primitives ------------------------------------------------------------------
 // Scratch of one stand-alone sort: key and value ping-pong buffers (n keys,
-// n values each), the digit histograms of every pass (8 x 256 words), the
-// sort control block and the look-back words (npass x tiles x 256 words).
+// n values each), the digit histograms (kHistCopies x kSortHistWords words),
+// the sort control block and the look-back words (npass x tiles x 256 words).
 struct SortScratch {
   void* ka;
   void* kb;
@@ -1218,24 +1211,17 @@ struct SortScratch {
   uint32_t* lb;
 };
 
-// Stable sort of n keys (with optional values) in place, in the scratch
-// `sc`; the histograms and look-back words are cleared here by fill kernels,
-// the control block by the sort's plan kernel.  Waits for the result.
+// Stable sort of n keys (with optional values) in place, in the scratch `sc`
+// (its last pass writes keys and vals themselves).  Waits for the result.
 template <typename K>
 static bvh_status sort_in_place(bvh_world w, K* keys, uint32_t* vals, uint64_t n, const SortScratch& sc) {
   hipStream_t s = w->stream;
-  const int npass = sizeof(K);
-  const uint64_t tiles = sort_tiles(n);
-  HIP_TRY(launch_fill_u32(sc.hist, 8 * 256, 0u, s));
-  HIP_TRY(launch_fill_u32(sc.lb, npass * tiles * 256, 0u, s));
-  HIP_TRY(launch_sort_histogram<K>(keys, n, npass, sc.hist, s));
   SortArgs<K> a{};
   a.k0 = keys; a.ka = static_cast<K*>(sc.ka); a.kb = static_cast<K*>(sc.kb);
   a.v0 = vals; a.va = vals ? sc.va : nullptr; a.vb = vals ? sc.vb : nullptr;
+  a.kout = keys; a.vout = vals;
   a.n = n; a.ctl = sc.ctl; a.lookback = sc.lb;
-  HIP_TRY(launch_sort_passes<K>(a, npass, sc.hist, s));
-  HIP_TRY(hipMemcpyAsync(keys, a.ka, n * sizeof(K), hipMemcpyDeviceToDevice, s));
-  if (vals) HIP_TRY(hipMemcpyAsync(vals, a.va, n * 4, hipMemcpyDeviceToDevice, s));
+  HIP_TRY(launch_sort<K>(a, sizeof(K), sc.hist, s));
   HIP_TRY(hipStreamSynchronize(s));
   return BVH_OK;
 }
@@ -1254,7 +1240,7 @@ static bvh_status prim_sort(bvh_world w, K* keys, uint32_t* vals, uint64_t n) {
   BVH_TRY(w->s_kb.ensure(n * sizeof(K)));
   BVH_TRY(w->s_va.ensure(n * 4));
   BVH_TRY(w->s_vb.ensure(n * 4));
-  BVH_TRY(w->s_hist.ensure(8 * 256 * 4));
+  BVH_TRY(w->s_hist.ensure(kHistCopies * kSortHistWords * 4));
   BVH_TRY(w->s_ctl.ensure(sizeof(SortCtl)));
   BVH_TRY(w->s_lb.ensure(npass * tiles * 256 * 4));
   const SortScratch sc{w->s_ka.p, w->s_kb.p, w->s_va.as<uint32_t>(), w->s_vb.as<uint32_t>(),
@@ -1278,7 +1264,7 @@ constexpr uint64_t kNaKb = kNaKa + na_align(kNoAllocMaxKeys * 8);
 constexpr uint64_t kNaVa = kNaKb + na_align(kNoAllocMaxKeys * 8);
 constexpr uint64_t kNaVb = kNaVa + na_align(kNoAllocMaxKeys * 4);
 constexpr uint64_t kNaHist = kNaVb + na_align(kNoAllocMaxKeys * 4);
-constexpr uint64_t kNaCtl = kNaHist + na_align(8 * 256 * 4);
+constexpr uint64_t kNaCtl = kNaHist + na_align(kHistCopies * kSortHistWords * 4);
 constexpr uint64_t kNaLb = kNaCtl + na_align(sizeof(SortCtl));
 constexpr uint64_t kNoAllocBytes = kNaLb + na_align(8 * kNoAllocTiles * 256 * 4);
 

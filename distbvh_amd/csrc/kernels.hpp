@@ -15,9 +15,10 @@ struct SortCtl {
   uint32_t tile_counter[8];
   uint32_t offsets[8 * 256];
 };
-// Buffers of one sort: keys in k0 (not modified), result in ka / va; kb / vb
-// are ping-pong scratch.  v0 == nullptr means payload = input index; va ==
-// nullptr means keys only.
+// Buffers of one sort: keys in k0, result in ka / va, kb / vb ping-pong
+// scratch; with kout (and vout) the result goes there instead, which may be k0
+// (v0), and ka / va are scratch too.  v0 == nullptr means payload = input
+// index; va == nullptr means keys only.
 template <typename K>
 struct SortArgs {
   const K* k0;
@@ -26,6 +27,8 @@ struct SortArgs {
   const uint32_t* v0;
   uint32_t* va;
   uint32_t* vb;
+  K* kout;
+  uint32_t* vout;
   uint64_t n;
   uint64_t ntiles;     // set by launch_sort_pass (the shape's tiles)
   SortCtl* ctl;
@@ -37,17 +40,21 @@ hipError_t launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t s);
 hipError_t launch_iota_u32(uint32_t* p, uint64_t n, hipStream_t s);
 template <typename T>
 hipError_t launch_copy(T* dst, const T* src, uint64_t n, hipStream_t s);
+// A whole sort of npass digits: the histograms (hist: kHistCopies x
+// kSortHistWords words; cleared here, as the look-back words), the plan and
+// the passes
 template <typename K>
-hipError_t launch_sort_histogram(const K* keys, uint64_t n, int npass, uint32_t* hist, hipStream_t s);
-template <typename K>
-hipError_t launch_sort_passes(const SortArgs<K>& a, int npass, const uint32_t* hist, hipStream_t s);
-// the same launches one at a time: the plan, then pass p (0 .. npass-1) in order
+hipError_t launch_sort(const SortArgs<K>& a, int npass, uint32_t* hist, hipStream_t s);
+// the plan and the passes one at a time, for a build whose Morton kernel made
+// the histograms and cleared the look-back words: the plan, then pass p
+// (0 .. npass-1) in order
 // The build's digit histograms (the Morton kernel's 8 x 256 words of sort
 // digits, then the 256 split depths of the cluster kernel): kHistCopies
 // copies, block b adding into copy b mod kHistCopies, so that the blocks'
 // global adds spread over more addresses; their readers sum the copies.
 constexpr int kHistCopies = 8;
 constexpr uint32_t kHistWords = 9 * 256;
+constexpr uint32_t kSortHistWords = 8 * 256;  // one copy of a stand-alone sort's histograms
 template <typename K>
 hipError_t launch_sort_plan(const SortArgs<K>& a, int npass, const uint32_t* hist, hipStream_t s, int copies = 1,
                             uint32_t copy_stride = 0);

@@ -72,27 +72,69 @@ __device__ __forceinline__ uint32_t block_excl_scan256(uint32_t v, uint32_t* s_t
   return wp + x - v;
 }
 
-// Histograms of all digit passes of `keys` (grid-stride).
+// Histograms of all digit passes of `keys` (grid-stride), and the sort's
+// look-back words cleared.  What bounds it is adds to one address: lanes of a
+// wave that share a digit serialise in LDS, and the blocks' sums on a digit's
+// word in memory.  So the LDS histograms are kept twice (lane mod 2,
+// interleaved over the banks; four copies cost a workgroup a place on the CU
+// and took 109 us where two take 85), a wave whose lanes all share a digit
+// adds once, and the blocks' sums go to kHistCopies copies (block b to copy b
+// mod kHistCopies) that the plan sums.  With one LDS histogram a block, a
+// block per 256 keys and one copy in memory it took 320 us on the 27 M pair
+// keys of a sphere cloud and 36 us on 420,000; now 110 and 10.
+constexpr unsigned kHistBlocks = 2048;
+constexpr int kHistLds = 2;
+constexpr uint64_t kHistKeys = 4;  // keys per thread and round, their loads together
 template <typename K>
-__global__ __launch_bounds__(256) void k_sort_histogram(const K* __restrict__ keys, uint64_t n, int npass,
-                                                        uint32_t* __restrict__ hist) {
-  __shared__ uint32_t sh[8 * 256];
-  for (int i = threadIdx.x; i < npass * 256; i += blockDim.x) sh[i] = 0;
+__global__ __launch_bounds__(256) void k_sort_histogram(const K* __restrict__ keys, uint64_t n,
+                                                        uint32_t* __restrict__ hist, uint32_t* __restrict__ lookback,
+                                                        uint64_t lb_words) {
+  constexpr int kPasses = sizeof(K);
+  __shared__ uint32_t sh[kPasses * 256 * kHistLds];
+  const uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (uint64_t)gridDim.x * blockDim.x;
+  for (int i = threadIdx.x; i < kPasses * 256 * kHistLds; i += 256) sh[i] = 0;
+  for (uint64_t i = gid; i < lb_words; i += stride) lookback[i] = 0;
   __syncthreads();
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (uint64_t)gridDim.x * blockDim.x) {
-    K k = keys[i];
-    for (int p = 0; p < npass; ++p) atomicAdd(&sh[p * 256 + (uint32_t)((k >> (8 * p)) & 255)], 1u);
+  const uint32_t copy = threadIdx.x % kHistLds;
+  for (uint64_t i0 = gid; i0 - threadIdx.x % 64 < n; i0 += kHistKeys * stride) {  // uniform per wave
+    K k[kHistKeys];
+#pragma unroll
+    for (uint64_t u = 0; u < kHistKeys; ++u) k[u] = i0 + u * stride < n ? keys[i0 + u * stride] : (K)0;
+#pragma unroll
+    for (uint64_t u = 0; u < kHistKeys; ++u) {
+      const bool valid = i0 + u * stride < n;
+      const uint64_t active = __ballot(valid);
+      if (active == 0) break;
+      const uint32_t leader = (uint32_t)(__ffsll((long long)active) - 1);
+#pragma unroll
+      for (int p = 0; p < kPasses; ++p) {
+        const uint32_t d = (uint32_t)(k[u] >> (8 * p)) & 255u;
+        const uint32_t d0 = __builtin_amdgcn_readlane(d, leader);
+        if (__ballot(valid & (d != d0)) == 0) {
+          if (lane_id() == leader) atomicAdd(&sh[(p * 256 + d0) * kHistLds], (uint32_t)__popcll(active));
+        } else if (valid) {
+          atomicAdd(&sh[(p * 256 + d) * kHistLds + copy], 1u);
+        }
+      }
+    }
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < npass * 256; i += blockDim.x)
-    if (sh[i]) atomicAdd(&hist[i], sh[i]);
+  uint32_t* h = hist + (blockIdx.x % kHistCopies) * kSortHistWords;
+  for (int i = threadIdx.x; i < kPasses * 256; i += 256) {
+    const uint32_t c = sh[kHistLds * i] + sh[kHistLds * i + 1];
+    if (c) atomicAdd(&h[i], c);
+  }
 }
 
 // One block: digit offsets (exclusive scan per pass), pass activity and the
-// ping-pong buffer selectors (the last active pass writes buffer A).
+// ping-pong buffer selectors: the last active pass writes buffer A, or the
+// result buffer with out_sel0 = kSelOut.  That buffer may be the input, so at
+// least two passes are then active (one more moves every key to its own
+// place): no pass reads what it writes.
+constexpr uint32_t kSelOut = 3;
 __global__ __launch_bounds__(256) void k_sort_plan(const uint32_t* __restrict__ hist, uint64_t n, int npass,
-                                                   SortCtl* __restrict__ ctl, int copies, uint32_t copy_stride) {
+                                                   SortCtl* __restrict__ ctl, int copies, uint32_t copy_stride,
+                                                   uint32_t out_sel0) {
   __shared__ uint32_t s_wtot[8][4];
   __shared__ uint32_t s_active[8];
   const int t = threadIdx.x;
@@ -150,13 +192,15 @@ __global__ __launch_bounds__(256) void k_sort_plan(const uint32_t* __restrict__ 
   if (t == 0) {
     int nact = 0;
     for (int p = 0; p < npass; ++p) nact += s_active[p];
-    if (nact == 0) {
-      s_active[0] = 1;
-      nact = 1;
-    }
-    // walk backwards: last active pass -> A (1), previous -> B (2), ...
+    const int need = out_sel0 == kSelOut ? 2 : 1;
+    for (int p = 0; p < npass && nact < need; ++p)
+      if (!s_active[p]) {
+        s_active[p] = 1;
+        ++nact;
+      }
+    // walk backwards: last active pass -> the result, previous -> A or B in turn
     uint32_t out_sel[8];
-    uint32_t cur = 1;
+    uint32_t cur = out_sel0;
     for (int p = npass - 1; p >= 0; --p) {
       if (s_active[p]) {
         out_sel[p] = cur;
@@ -201,9 +245,9 @@ __global__ __launch_bounds__(SortShape<WIDE>::block) void k_sort_pass(SortArgs<K
   const SortPassInfo pi = a.ctl->pass[pass];
   if (!pi.active) return;
   const K* __restrict__ kin = pi.in_sel == 0 ? a.k0 : (pi.in_sel == 1 ? a.ka : a.kb);
-  K* __restrict__ kout = pi.out_sel == 1 ? a.ka : a.kb;
+  K* __restrict__ kout = pi.out_sel == 1 ? a.ka : (pi.out_sel == 2 ? a.kb : a.kout);
   const uint32_t* __restrict__ vin = pi.in_sel == 0 ? a.v0 : (pi.in_sel == 1 ? a.va : a.vb);
-  uint32_t* __restrict__ vout = pi.out_sel == 1 ? a.va : a.vb;
+  uint32_t* __restrict__ vout = pi.out_sel == 1 ? a.va : (pi.out_sel == 2 ? a.vb : a.vout);
   const bool has_vals = a.va != nullptr;
   const int shift = 8 * pass;
   const uint64_t n = a.n;
@@ -417,15 +461,13 @@ template hipError_t launch_copy<uint32_t>(uint32_t*, const uint32_t*, uint64_t, 
 template hipError_t launch_copy<double>(double*, const double*, uint64_t, hipStream_t);
 
 template <typename K>
-hipError_t launch_sort_histogram(const K* keys, uint64_t n, int npass, uint32_t* hist, hipStream_t s) {
-  if (n == 0) return hipSuccess;
-  uint64_t blocks = (n + 255) / 256;
-  if (blocks > 2048) blocks = 2048;
-  hipLaunchKernelGGL(k_sort_histogram<K>, dim3((unsigned)blocks), dim3(256), 0, s, keys, n, npass, hist);
+static hipError_t launch_sort_histogram(const SortArgs<K>& a, uint32_t* hist, hipStream_t s) {
+  uint64_t blocks = (a.n + 2047) / 2048;
+  if (blocks > kHistBlocks) blocks = kHistBlocks;
+  hipLaunchKernelGGL(k_sort_histogram<K>, dim3((unsigned)blocks), dim3(256), 0, s, a.k0, a.n, hist, a.lookback,
+                     sizeof(K) * sort_tiles(a.n) * 256);
   return hipGetLastError();
 }
-template hipError_t launch_sort_histogram<uint64_t>(const uint64_t*, uint64_t, int, uint32_t*, hipStream_t);
-template hipError_t launch_sort_histogram<uint32_t>(const uint32_t*, uint64_t, int, uint32_t*, hipStream_t);
 
 // Sort after the histograms are in `hist` (npass * 256 counters) and the
 // look-back words are zero.  Result in a.ka (and a.va).
@@ -434,7 +476,8 @@ hipError_t launch_sort_plan(const SortArgs<K>& a, int npass, const uint32_t* his
                             uint32_t copy_stride) {
   if (a.n == 0) return hipSuccess;
   if (npass < 1 || npass > 8 || copies < 1 || copies > 8) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_sort_plan, dim3(1), dim3(256), 0, s, hist, a.n, npass, a.ctl, copies, copy_stride);
+  hipLaunchKernelGGL(k_sort_plan, dim3(1), dim3(256), 0, s, hist, a.n, npass, a.ctl, copies, copy_stride,
+                     a.kout ? kSelOut : 1u);
   return hipGetLastError();
 }
 
@@ -455,8 +498,11 @@ hipError_t launch_sort_pass(const SortArgs<K>& a, int p, hipStream_t s) {
 }
 
 template <typename K>
-hipError_t launch_sort_passes(const SortArgs<K>& a, int npass, const uint32_t* hist, hipStream_t s) {
-  hipError_t e = launch_sort_plan<K>(a, npass, hist, s);
+hipError_t launch_sort(const SortArgs<K>& a, int npass, uint32_t* hist, hipStream_t s) {
+  if (a.n == 0) return hipSuccess;
+  hipError_t e = launch_fill_u32(hist, (uint64_t)kHistCopies * kSortHistWords, 0u, s);
+  if (e == hipSuccess) e = launch_sort_histogram<K>(a, hist, s);
+  if (e == hipSuccess) e = launch_sort_plan<K>(a, npass, hist, s, kHistCopies, kSortHistWords);
   for (int p = 0; p < npass && e == hipSuccess; ++p) e = launch_sort_pass<K>(a, p, s);
   return e;
 }
@@ -466,8 +512,8 @@ template hipError_t launch_sort_plan<uint32_t>(const SortArgs<uint32_t>&, int, c
                                               uint32_t);
 template hipError_t launch_sort_pass<uint64_t>(const SortArgs<uint64_t>&, int, hipStream_t);
 template hipError_t launch_sort_pass<uint32_t>(const SortArgs<uint32_t>&, int, hipStream_t);
-template hipError_t launch_sort_passes<uint64_t>(const SortArgs<uint64_t>&, int, const uint32_t*, hipStream_t);
-template hipError_t launch_sort_passes<uint32_t>(const SortArgs<uint32_t>&, int, const uint32_t*, hipStream_t);
+template hipError_t launch_sort<uint64_t>(const SortArgs<uint64_t>&, int, uint32_t*, hipStream_t);
+template hipError_t launch_sort<uint32_t>(const SortArgs<uint32_t>&, int, uint32_t*, hipStream_t);
 
 
 // ---- exclusive scan (prefix_sum, util/prefix_sum.hpp:41-54) ---------------------------
