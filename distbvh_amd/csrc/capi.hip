@@ -540,9 +540,21 @@ static bvh_status object_build_tree(bvh_object_s* o);
 // steps of a deferred build launched by its set_entity_data call itself
 constexpr size_t kEagerSteps = 2;
 
+// One launch of a build's sort of its Morton codes: all of it (few elements),
+// else the plan (p < 0) or pass p.
+template <typename K>
+static hipError_t launch_build_sort(bvh_object_s* o, int npass, int p, bool small, hipStream_t s) {
+  SortArgs<K> a{};
+  a.k0 = (const K*)o->bb.codes0; a.ka = (K*)o->bb.codes_a; a.kb = (K*)o->bb.codes_b;
+  a.v0 = nullptr; a.va = o->bb.perm; a.vb = o->bb.perm_b;
+  a.n = o->in.n; a.ctl = o->bb.ctl; a.lookback = o->bb.lookback;
+  if (small) return launch_sort_small<K>(a, npass, s);
+  return p < 0 ? launch_sort_plan<K>(a, npass, o->bb.hist, s, kHistCopies, kHistWords) : launch_sort_pass<K>(a, p, s);
+}
+
 // The launches of a build up to (not including) its tree stage, as steps run
-// in order on the object's stream: the bounds, the Morton codes, the sort's
-// plan and each of its passes, the patch splits, the frame and the split
+// in order on the object's stream: the bounds, the Morton codes, the sort (its
+// plan and each of its passes, or one launch), the patch splits, the frame and the split
 // heights.  Host state that later calls read is set when the steps are made.
 static void object_build_steps(bvh_object_s* o, std::vector<BuildStep>& st) {
   bvh_world w = o->w;
@@ -563,25 +575,13 @@ static void object_build_steps(bvh_object_s* o, std::vector<BuildStep>& st) {
     return BVH_OK;
   });
   const int npass = o->bits == 63 ? 8 : 4;
-  for (int p = -1; p < npass; ++p) {
+  const bool small = sort_is_small(n);
+  for (int p = -1; p < (small ? 0 : npass); ++p) {
     st.push_back([=] {
       if (p < 0) w->stage_begin("sort");
-      if (o->bits == 63) {
-        SortArgs<uint64_t> a{};
-        a.k0 = (const uint64_t*)o->bb.codes0; a.ka = (uint64_t*)o->bb.codes_a; a.kb = (uint64_t*)o->bb.codes_b;
-        a.v0 = nullptr; a.va = o->bb.perm; a.vb = o->bb.perm_b;
-        a.n = n; a.ctl = o->bb.ctl; a.lookback = o->bb.lookback;
-        HIP_TRY(p < 0 ? launch_sort_plan<uint64_t>(a, npass, o->bb.hist, s, kHistCopies, kHistWords)
-                      : launch_sort_pass<uint64_t>(a, p, s));
-      } else {
-        SortArgs<uint32_t> a{};
-        a.k0 = (const uint32_t*)o->bb.codes0; a.ka = (uint32_t*)o->bb.codes_a; a.kb = (uint32_t*)o->bb.codes_b;
-        a.v0 = nullptr; a.va = o->bb.perm; a.vb = o->bb.perm_b;
-        a.n = n; a.ctl = o->bb.ctl; a.lookback = o->bb.lookback;
-        HIP_TRY(p < 0 ? launch_sort_plan<uint32_t>(a, npass, o->bb.hist, s, kHistCopies, kHistWords)
-                      : launch_sort_pass<uint32_t>(a, p, s));
-      }
-      if (p == npass - 1) w->stage_end();
+      if (o->bits == 63) HIP_TRY(launch_build_sort<uint64_t>(o, npass, p, small, s));
+      else HIP_TRY(launch_build_sort<uint32_t>(o, npass, p, small, s));
+      if (p == npass - 1 || small) w->stage_end();
       return BVH_OK;
     });
   }

@@ -40,6 +40,10 @@ hipError_t launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t s);
 hipError_t launch_iota_u32(uint32_t* p, uint64_t n, hipStream_t s);
 template <typename T>
 hipError_t launch_copy(T* dst, const T* src, uint64_t n, hipStream_t s);
+// sorts of few keys run as one launch, without histograms or look-back words
+bool sort_is_small(uint64_t n);
+template <typename K>
+hipError_t launch_sort_small(const SortArgs<K>& a, int npass, hipStream_t s);
 // A whole sort of npass digits: the histograms (hist: kHistCopies x
 // kSortHistWords words; cleared here, as the look-back words), the plan and
 // the passes

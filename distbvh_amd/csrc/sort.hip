@@ -408,6 +408,142 @@ __global__ __launch_bounds__(SortShape<WIDE>::block) void k_sort_pass(SortArgs<K
   }
 }
 
+// A whole sort of at most kSmallBlock * ITEMS keys in one workgroup: the keys
+// and payloads stay in registers between passes and change places through LDS,
+// digits that all keys share are skipped, and nothing is cleared or planned
+// beforehand.  Bound by its barriers and LDS latency: 1.5 us a pass of 512
+// pairs, 6 us of 8,192.  A whole sort of 512 / 4,096 / 8,192 pairs takes 13 /
+// 30 / 48 us so, 51 / 63 / 72 as passes of their own; at 16,384 keys the one
+// CU's work would pass the launches' 75 us.
+constexpr int kSmallBlock = 1024;
+constexpr uint64_t kSortSmallMax = 8 * kSmallBlock;
+template <typename K, int ITEMS>
+__global__ __launch_bounds__(kSmallBlock) void k_sort_small(SortArgs<K> a, int npass) {
+  constexpr int kWaves = kSmallBlock / 64;
+  __shared__ __align__(4) uint16_t s_wcount[kWaves][256];
+  __shared__ uint32_t s_texcl[256];
+  __shared__ uint32_t s_tmp[4];
+  __shared__ uint32_t s_diff[2];
+  __shared__ K s_first;
+  __shared__ __align__(16) unsigned char s_buf[kSmallBlock * ITEMS * (sizeof(K) + 4)];
+  K* s_keys = (K*)s_buf;
+  uint32_t* s_vals = (uint32_t*)(s_buf + kSmallBlock * ITEMS * sizeof(K));
+  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
+  const uint32_t n = (uint32_t)a.n;
+  const K* k0 = a.k0;
+  const uint32_t* v0 = a.v0;
+  K* kout = a.kout ? a.kout : a.ka;  // (may be the input)
+  uint32_t* vout = a.kout ? a.vout : a.va;
+  const bool has_vals = a.va != nullptr;
+  const uint32_t p0 = (uint32_t)(w * (ITEMS * 64) + lane);
+  auto valid = [&](int j) { return p0 + j * 64 < n; };
+  K key[ITEMS];
+  uint32_t val[ITEMS];
+#pragma unroll
+  for (int j = 0; j < ITEMS; ++j) {
+    const uint32_t pos = p0 + j * 64;
+    key[j] = valid(j) ? k0[pos] : (K)0;
+    if (has_vals) val[j] = valid(j) ? (v0 ? v0[pos] : pos) : 0u;
+  }
+  if (tid < 2) s_diff[tid] = 0;
+  if (tid == 0) s_first = key[0];
+  for (int i = lane; i < 128; i += 64) ((uint32_t*)&s_wcount[w][0])[i] = 0;
+  __syncthreads();
+  {  // the bits in which some key differs from the first
+    const K f = s_first;
+    K x = 0;
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j)
+      if (valid(j)) x |= key[j] ^ f;
+    uint32_t lo = (uint32_t)x, hi = sizeof(K) == 8 ? (uint32_t)((uint64_t)x >> 32) : 0u;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      lo |= __shfl_xor(lo, o, 64);
+      if (sizeof(K) == 8) hi |= __shfl_xor(hi, o, 64);
+    }
+    if (lane == 0) {
+      if (lo) atomicOr(&s_diff[0], lo);
+      if (hi) atomicOr(&s_diff[1], hi);
+    }
+  }
+  __syncthreads();
+  const uint64_t diff = ((uint64_t)s_diff[1] << 32) | s_diff[0];
+  for (int p = 0; p < npass; ++p) {
+    const int shift = 8 * p;
+    if (((diff >> shift) & 255u) == 0) continue;  // uniform
+    uint32_t rank[ITEMS];
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) {
+      const uint32_t d = (uint32_t)(key[j] >> shift) & 255u;
+      const bool ok = valid(j);
+      const uint64_t m = __ballot(ok);
+      uint32_t lo = (uint32_t)m, hi = (uint32_t)(m >> 32);
+#pragma unroll
+      for (int b = 0; b < 8; ++b) match_bit(d, b, lo, hi);
+      const uint32_t before = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
+      const uint32_t same = (uint32_t)(__popc(lo) + __popc(hi));
+      uint32_t old = 0;
+      if (ok) old = s_wcount[w][d];
+      rank[j] = old + before;
+      __builtin_amdgcn_wave_barrier();
+      if (ok && before == 0) s_wcount[w][d] = (uint16_t)(old + same);
+      __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    uint32_t run = 0, x = 0;
+    if (tid < 256) {
+#pragma unroll
+      for (int v = 0; v < kWaves; ++v) {
+        const uint32_t c = s_wcount[v][tid];
+        s_wcount[v][tid] = (uint16_t)run;
+        run += c;
+      }
+      x = run;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = __shfl_up(x, o, 64);
+        if (lane >= o) x += y;
+      }
+      if (lane == 63) s_tmp[w] = x;
+    }
+    __syncthreads();
+    if (tid < 256) {
+      uint32_t texcl = x - run;
+      for (int i = 0; i < w; ++i) texcl += s_tmp[i];
+      s_texcl[tid] = texcl;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) {
+      if (valid(j)) {
+        const uint32_t d = (uint32_t)(key[j] >> shift) & 255u;
+        const uint32_t at = s_texcl[d] + s_wcount[w][d] + rank[j];
+        s_keys[at] = key[j];
+        if (has_vals) s_vals[at] = val[j];
+      }
+    }
+    for (int i = lane; i < 128; i += 64) ((uint32_t*)&s_wcount[w][0])[i] = 0;  // (the wave's own counters)
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) {
+      const uint32_t pos = p0 + j * 64;
+      if (valid(j)) {
+        key[j] = s_keys[pos];
+        if (has_vals) val[j] = s_vals[pos];
+      }
+    }
+    // (the next writes to s_keys and s_vals come after two barriers)
+  }
+#pragma unroll
+  for (int j = 0; j < ITEMS; ++j) {
+    const uint32_t pos = p0 + j * 64;
+    if (valid(j)) {
+      kout[pos] = key[j];
+      if (has_vals) vout[pos] = val[j];
+    }
+  }
+}
+
 __global__ void k_fill_u32(uint32_t* __restrict__ p, uint64_t n, uint32_t v) {
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (uint64_t)gridDim.x * blockDim.x)
@@ -497,9 +633,26 @@ hipError_t launch_sort_pass(const SortArgs<K>& a, int p, hipStream_t s) {
   return hipGetLastError();
 }
 
+bool sort_is_small(uint64_t n) { return n <= kSortSmallMax; }
+
+template <typename K>
+hipError_t launch_sort_small(const SortArgs<K>& a, int npass, hipStream_t s) {
+  if (a.n == 0) return hipSuccess;
+  if (!sort_is_small(a.n) || npass < 1 || npass > (int)sizeof(K)) return hipErrorInvalidValue;
+  const dim3 g(1), b(kSmallBlock);
+  if (a.n <= 1 * kSmallBlock) hipLaunchKernelGGL((k_sort_small<K, 1>), g, b, 0, s, a, npass);
+  else if (a.n <= 2 * kSmallBlock) hipLaunchKernelGGL((k_sort_small<K, 2>), g, b, 0, s, a, npass);
+  else if (a.n <= 4 * kSmallBlock) hipLaunchKernelGGL((k_sort_small<K, 4>), g, b, 0, s, a, npass);
+  else hipLaunchKernelGGL((k_sort_small<K, 8>), g, b, 0, s, a, npass);
+  return hipGetLastError();
+}
+template hipError_t launch_sort_small<uint64_t>(const SortArgs<uint64_t>&, int, hipStream_t);
+template hipError_t launch_sort_small<uint32_t>(const SortArgs<uint32_t>&, int, hipStream_t);
+
 template <typename K>
 hipError_t launch_sort(const SortArgs<K>& a, int npass, uint32_t* hist, hipStream_t s) {
   if (a.n == 0) return hipSuccess;
+  if (sort_is_small(a.n)) return launch_sort_small<K>(a, npass, s);
   hipError_t e = launch_fill_u32(hist, (uint64_t)kHistCopies * kSortHistWords, 0u, s);
   if (e == hipSuccess) e = launch_sort_histogram<K>(a, hist, s);
   if (e == hipSuccess) e = launch_sort_plan<K>(a, npass, hist, s, kHistCopies, kSortHistWords);
