@@ -561,6 +561,15 @@ static void object_build_steps(bvh_object_s* o, std::vector<BuildStep>& st) {
   const hipStream_t s = w->stream;
   const uint64_t n = o->in.n;
   st.clear();
+  o->patch_slabs_ready = !o->fp32;
+  // (stage times are asked for stage by stage)
+  if (o->split == BVH_SPLIT_CLUSTERING && build_is_small(n) && !(w->cfg.flags & BVH_FLAG_TIMING)) {
+    st.push_back([=] {
+      HIP_TRY(launch_build_small(o->in, o->bb, o->bits, s));
+      return BVH_OK;
+    });
+    return;
+  }
   st.push_back([=] {
     // (the bounds kernel also clears the status words)
     w->stage_begin("bounds");
@@ -603,7 +612,6 @@ static void object_build_steps(bvh_object_s* o, std::vector<BuildStep>& st) {
     w->stage_end();
     return BVH_OK;
   });
-  o->patch_slabs_ready = !o->fp32;
 }
 
 // The whole object build, stream ordered, no host synchronization.  With

@@ -130,6 +130,11 @@ constexpr uint32_t kErrTree = 1u;      // inconsistent tree link during the buil
 constexpr uint32_t kErrTraverse = 2u;  // traversal exceeded its step bound
 constexpr uint32_t kErrIndex = 4u;     // element index out of range
 
+// the whole build of an object of few elements up to its tree stage (what
+// launch_prep, launch_morton, the sort, launch_cluster and launch_delta leave),
+// by the clustering splits, in one launch
+bool build_is_small(uint64_t n);
+hipError_t launch_build_small(const ElemInput& in, const BuildBufs& b, int bits, hipStream_t s);
 hipError_t launch_prep(const ElemInput& in, const BuildBufs& b, hipStream_t s);
 hipError_t launch_morton(const ElemInput& in, const BuildBufs& b, int bits, hipStream_t s);
 hipError_t launch_cluster(const BuildBufs& b, uint64_t n, int bits, uint64_t nsplits, hipStream_t s);

@@ -21,6 +21,7 @@
 // for every key is skipped on the device.
 #include "device.hpp"
 #include "kernels.hpp"
+#include "sort_block.hpp"
 
 namespace dbvh {
 
@@ -227,15 +228,6 @@ __global__ __launch_bounds__(256) void k_sort_plan(const uint32_t* __restrict__ 
   }
 }
 
-// Keeps in (lo, hi), a lane mask, the lanes whose bit b of d equals this
-// lane's: m & ~(ballot ^ own bit), one three-input operation per half.
-__device__ __forceinline__ void match_bit(uint32_t d, int b, uint32_t& lo, uint32_t& hi) {
-  const int own = (int)(d << (31 - b)) >> 31;
-  const uint64_t bb = __ballot(own != 0);
-  lo = (uint32_t)__builtin_amdgcn_bitop3_b32((int)lo, (int)(uint32_t)bb, own, 0x90);
-  hi = (uint32_t)__builtin_amdgcn_bitop3_b32((int)hi, (int)(uint32_t)(bb >> 32), own, 0x90);
-}
-
 // One digit pass over one tile.  Bound by the VALU work of the ranking (about
 // 45 instructions a key) beside the memory time of 24 bytes a key.
 template <typename K, bool WIDE>
@@ -415,129 +407,28 @@ __global__ __launch_bounds__(SortShape<WIDE>::block) void k_sort_pass(SortArgs<K
 // pairs, 6 us of 8,192.  A whole sort of 512 / 4,096 / 8,192 pairs takes 13 /
 // 30 / 48 us so, 51 / 63 / 72 as passes of their own; at 16,384 keys the one
 // CU's work would pass the launches' 75 us.
-constexpr int kSmallBlock = 1024;
-constexpr uint64_t kSortSmallMax = 8 * kSmallBlock;
 template <typename K, int ITEMS>
 __global__ __launch_bounds__(kSmallBlock) void k_sort_small(SortArgs<K> a, int npass) {
-  constexpr int kWaves = kSmallBlock / 64;
-  __shared__ __align__(4) uint16_t s_wcount[kWaves][256];
-  __shared__ uint32_t s_texcl[256];
-  __shared__ uint32_t s_tmp[4];
-  __shared__ uint32_t s_diff[2];
-  __shared__ K s_first;
-  __shared__ __align__(16) unsigned char s_buf[kSmallBlock * ITEMS * (sizeof(K) + 4)];
-  K* s_keys = (K*)s_buf;
-  uint32_t* s_vals = (uint32_t*)(s_buf + kSmallBlock * ITEMS * sizeof(K));
-  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
+  __shared__ SortBlockLds<K, ITEMS> L;
   const uint32_t n = (uint32_t)a.n;
   const K* k0 = a.k0;
   const uint32_t* v0 = a.v0;
   K* kout = a.kout ? a.kout : a.ka;  // (may be the input)
   uint32_t* vout = a.kout ? a.vout : a.va;
   const bool has_vals = a.va != nullptr;
-  const uint32_t p0 = (uint32_t)(w * (ITEMS * 64) + lane);
-  auto valid = [&](int j) { return p0 + j * 64 < n; };
   K key[ITEMS];
   uint32_t val[ITEMS];
 #pragma unroll
   for (int j = 0; j < ITEMS; ++j) {
-    const uint32_t pos = p0 + j * 64;
-    key[j] = valid(j) ? k0[pos] : (K)0;
-    if (has_vals) val[j] = valid(j) ? (v0 ? v0[pos] : pos) : 0u;
+    const uint32_t pos = small_pos<ITEMS>(j);
+    key[j] = pos < n ? k0[pos] : (K)0;
+    val[j] = has_vals && pos < n ? (v0 ? v0[pos] : pos) : 0u;
   }
-  if (tid < 2) s_diff[tid] = 0;
-  if (tid == 0) s_first = key[0];
-  for (int i = lane; i < 128; i += 64) ((uint32_t*)&s_wcount[w][0])[i] = 0;
-  __syncthreads();
-  {  // the bits in which some key differs from the first
-    const K f = s_first;
-    K x = 0;
-#pragma unroll
-    for (int j = 0; j < ITEMS; ++j)
-      if (valid(j)) x |= key[j] ^ f;
-    uint32_t lo = (uint32_t)x, hi = sizeof(K) == 8 ? (uint32_t)((uint64_t)x >> 32) : 0u;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      lo |= __shfl_xor(lo, o, 64);
-      if (sizeof(K) == 8) hi |= __shfl_xor(hi, o, 64);
-    }
-    if (lane == 0) {
-      if (lo) atomicOr(&s_diff[0], lo);
-      if (hi) atomicOr(&s_diff[1], hi);
-    }
-  }
-  __syncthreads();
-  const uint64_t diff = ((uint64_t)s_diff[1] << 32) | s_diff[0];
-  for (int p = 0; p < npass; ++p) {
-    const int shift = 8 * p;
-    if (((diff >> shift) & 255u) == 0) continue;  // uniform
-    uint32_t rank[ITEMS];
-#pragma unroll
-    for (int j = 0; j < ITEMS; ++j) {
-      const uint32_t d = (uint32_t)(key[j] >> shift) & 255u;
-      const bool ok = valid(j);
-      const uint64_t m = __ballot(ok);
-      uint32_t lo = (uint32_t)m, hi = (uint32_t)(m >> 32);
-#pragma unroll
-      for (int b = 0; b < 8; ++b) match_bit(d, b, lo, hi);
-      const uint32_t before = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
-      const uint32_t same = (uint32_t)(__popc(lo) + __popc(hi));
-      uint32_t old = 0;
-      if (ok) old = s_wcount[w][d];
-      rank[j] = old + before;
-      __builtin_amdgcn_wave_barrier();
-      if (ok && before == 0) s_wcount[w][d] = (uint16_t)(old + same);
-      __builtin_amdgcn_wave_barrier();
-    }
-    __syncthreads();
-    uint32_t run = 0, x = 0;
-    if (tid < 256) {
-#pragma unroll
-      for (int v = 0; v < kWaves; ++v) {
-        const uint32_t c = s_wcount[v][tid];
-        s_wcount[v][tid] = (uint16_t)run;
-        run += c;
-      }
-      x = run;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t y = __shfl_up(x, o, 64);
-        if (lane >= o) x += y;
-      }
-      if (lane == 63) s_tmp[w] = x;
-    }
-    __syncthreads();
-    if (tid < 256) {
-      uint32_t texcl = x - run;
-      for (int i = 0; i < w; ++i) texcl += s_tmp[i];
-      s_texcl[tid] = texcl;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < ITEMS; ++j) {
-      if (valid(j)) {
-        const uint32_t d = (uint32_t)(key[j] >> shift) & 255u;
-        const uint32_t at = s_texcl[d] + s_wcount[w][d] + rank[j];
-        s_keys[at] = key[j];
-        if (has_vals) s_vals[at] = val[j];
-      }
-    }
-    for (int i = lane; i < 128; i += 64) ((uint32_t*)&s_wcount[w][0])[i] = 0;  // (the wave's own counters)
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < ITEMS; ++j) {
-      const uint32_t pos = p0 + j * 64;
-      if (valid(j)) {
-        key[j] = s_keys[pos];
-        if (has_vals) val[j] = s_vals[pos];
-      }
-    }
-    // (the next writes to s_keys and s_vals come after two barriers)
-  }
+  sort_block<K, ITEMS>(L, key, val, has_vals, n, npass);
 #pragma unroll
   for (int j = 0; j < ITEMS; ++j) {
-    const uint32_t pos = p0 + j * 64;
-    if (valid(j)) {
+    const uint32_t pos = small_pos<ITEMS>(j);
+    if (pos < n) {
       kout[pos] = key[j];
       if (has_vals) vout[pos] = val[j];
     }
@@ -633,6 +524,7 @@ hipError_t launch_sort_pass(const SortArgs<K>& a, int p, hipStream_t s) {
   return hipGetLastError();
 }
 
+constexpr uint64_t kSortSmallMax = 8 * kSmallBlock;
 bool sort_is_small(uint64_t n) { return n <= kSortSmallMax; }
 
 template <typename K>
