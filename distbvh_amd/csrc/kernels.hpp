@@ -312,7 +312,10 @@ struct PairOut {
   // stripe w % kRecheckStripes through that stripe's counter,
   // rcount[stripe * kRecheckStride], so no single counter takes every
   // flush.  The re-check kernel adds rtotal[0] = sum and rtotal[1] = largest
-  // of the stripe counts (a stripe count above rcap is an overflow).
+  // of the stripe counts (a stripe count above rcap is an overflow).  The two
+  // words after a stripe's counter take its waves' visits and candidates: as
+  // two words of the query, every wave's end waited for one line (13 ns an
+  // addition).
   uint64_t* recheck;
   uint64_t rcap;
   unsigned long long* rcount;

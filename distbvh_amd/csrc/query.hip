@@ -497,9 +497,10 @@ __device__ __forceinline__ void walk32(const TreeView& q, const TreeView& t, uin
   recheck_flush(rbuf, rfill, out, rstripe);
   sink += pf;
   asm volatile("; record prefetch sink %0" ::"v"(sink));  // keeps the prefetch loads
-  if (lane == 0) {
-    if (out.visits) atomicAdd(out.visits, (unsigned long long)steps);
-    if (out.candidates) atomicAdd(out.candidates, (unsigned long long)ncand);
+  if (lane == 0) {  // in the stripe's line; k_recheck adds the stripes up
+    unsigned long long* line = out.rcount + (uint64_t)rstripe * kRecheckStride;
+    atomicAdd(line + 1, (unsigned long long)steps);
+    atomicAdd(line + 2, (unsigned long long)ncand);
   }
 }
 
@@ -893,7 +894,8 @@ __global__ __launch_bounds__(256) void k_narrow64s(TreeView q, TreeView t, int x
 // the two kernels.  The grid is kRecheckStripes x (blocks per stripe); block
 // b works on stripe b % kRecheckStripes.  Hits are staged per wave in LDS
 // (one atomic on the pair counter per flush, not per wave that hits).  Block
-// 0 also adds the stripe counts' sum and maximum to rtotal for the host.
+// 0 also adds the stripe counts' sum and maximum to rtotal, and the stripes'
+// visits and candidates to theirs, for the host.
 // KIND / NV: both objects' element type (the common case, with registers
 // sized for it); kGeneric: any mix, chosen at run time.
 constexpr int kGeneric = -1;
@@ -911,6 +913,8 @@ __global__ __launch_bounds__(256) void k_recheck(TreeView q, TreeView t, PairOut
     const unsigned long long c = out.rcount[(uint64_t)threadIdx.x * kRecheckStride];
     atomicAdd(out.rtotal, c);
     atomicMax(out.rtotal + 1, c);
+    if (out.visits) atomicAdd(out.visits, out.rcount[(uint64_t)threadIdx.x * kRecheckStride + 1]);
+    if (out.candidates) atomicAdd(out.candidates, out.rcount[(uint64_t)threadIdx.x * kRecheckStride + 2]);
   }
   const uint32_t stripe = blockIdx.x % kRecheckStripes;
   const uint32_t per = gridDim.x / kRecheckStripes;
