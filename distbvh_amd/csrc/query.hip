@@ -257,18 +257,18 @@ __device__ __forceinline__ void own_patch_range(const TreeView& q, uint32_t qa, 
   pe = (uint64_t)k + 1 >= q.od ? n : q.splits[k];
 }
 
-// The fp32-outward record walk of one tile of blockDim.x queries (the body of
+// The fp32-outward record walk of one wave's qper queries (the body of
 // k_narrow32 and of its batched form k_narrow32_batch); buf / rbuf / stk are
 // the wave's LDS pair staging, re-check staging and stack, rstripe the
 // wave's re-check stripe.  Leaf candidates with a gap above `inner` are
 // emitted, the rest queued for the fp64 re-check.
 template <bool SELF, bool CROSS>
-__device__ __forceinline__ void walk32(const TreeView& q, const TreeView& t, uint32_t tile, const PairOut& out,
-                                       int32_t inner, uint64_t* buf, uint64_t* rbuf, uint32_t* stk,
+__device__ __forceinline__ void walk32(const TreeView& q, const TreeView& t, uint32_t wave, uint32_t qper,
+                                       const PairOut& out, int32_t inner, uint64_t* buf, uint64_t* rbuf, uint32_t* stk,
                                        uint32_t rstripe) {
   uint32_t fill = 0, rfill = 0;
-  const uint64_t p = (uint64_t)tile * blockDim.x + threadIdx.x;
-  const bool valid = p < q.n;
+  const uint64_t p = (uint64_t)wave * qper + lane_id();
+  const bool valid = lane_id() < qper && p < q.n;
   if (q.origin != t.origin) inner = 0x7fffffff;
   int32_t qf[kSlabs];  // ord32 images of the query's outward fp32 slabs
   uint32_t qa = 0;
@@ -505,14 +505,15 @@ __device__ __forceinline__ void walk32(const TreeView& q, const TreeView& t, uin
 }
 
 template <bool SELF, bool CROSS = false>
-__global__ __launch_bounds__(256) void k_narrow32(TreeView q, TreeView t, int xcd, PairOut out, int32_t inner) {
+__global__ __launch_bounds__(256) void k_narrow32(TreeView q, TreeView t, int xcd, uint32_t qper, PairOut out,
+                                                  int32_t inner) {
   __shared__ uint64_t s_buf[256 / kWave][kWaveBuf];
   __shared__ uint64_t s_rbuf[256 / kWave][kRecheckBuf];
   __shared__ uint32_t s_stack[256 / kWave][kStack];
   const uint32_t wv = threadIdx.x / kWave;
   const uint32_t rstripe = (blockIdx.x * (blockDim.x / kWave) + wv) % kRecheckStripes;
   const uint32_t tile = xcd ? xcd_tile(blockIdx.x, gridDim.x) : blockIdx.x;
-  walk32<SELF, CROSS>(q, t, tile, out, inner, s_buf[wv], s_rbuf[wv], s_stack[wv], rstripe);
+  walk32<SELF, CROSS>(q, t, tile * (blockDim.x / kWave) + wv, qper, out, inner, s_buf[wv], s_rbuf[wv], s_stack[wv], rstripe);
 }
 
 // Several queries (object pairs) in one launch of the fp32-outward walk:
@@ -532,9 +533,9 @@ __global__ __launch_bounds__(256) void k_narrow32_batch(const BatchQuery* __rest
   }
   const BatchQuery& e = bq[lo];
   if (blockIdx.x - e.block0 >= e.blocks) return;
-  const uint32_t tile = blockIdx.x - e.block0;
-  const uint32_t rstripe = (tile * (blockDim.x / kWave) + wv) % kRecheckStripes;
-  walk32<false, false>(e.q, e.t, tile, e.out, inner, s_buf[wv], s_rbuf[wv], s_stack[wv], rstripe);
+  const uint32_t wave = (blockIdx.x - e.block0) * (256 / kWave) + wv;
+  const uint32_t rstripe = wave % kRecheckStripes;
+  walk32<false, false>(e.q, e.t, wave, kWave, e.out, inner, s_buf[wv], s_rbuf[wv], s_stack[wv], rstripe);
 }
 
 // Strict overlap of the lane's query slabs q with one box b whose 26 slabs
@@ -614,15 +615,15 @@ __device__ __forceinline__ void overlap_pair(const double* qk, const Rec64& r, b
 // set of visited nodes does not depend on K (a node is visited when some lane
 // overlaps it and its parent was visited), only the number of dependent
 // round trips does.  Leaf tests are exact, so hits are emitted directly.
-// The walk of one tile of blockDim.x queries (the body of k_narrow64 and of
-// its batched form k_narrow64_batch); buf / stk / R are the wave's LDS pair
+// The walk of one wave's qper queries (the body of k_narrow64 and of its
+// batched form k_narrow64_batch); buf / stk / R are the wave's LDS pair
 // staging, stack and record slots.
 template <bool SELF, int K, bool CROSS>
-__device__ __forceinline__ void walk64(const TreeView& q, const TreeView& t, uint32_t tile, const PairOut& out,
+__device__ __forceinline__ void walk64(const TreeView& q, const TreeView& t, uint32_t wave, uint32_t qper, const PairOut& out,
                                        uint64_t* buf, uint32_t* stk, Rec64* R) {
   uint32_t fill = 0;
-  const uint64_t p = (uint64_t)tile * blockDim.x + threadIdx.x;
-  const bool valid = p < q.n;
+  const uint64_t p = (uint64_t)wave * qper + lane_id();
+  const bool valid = lane_id() < qper && p < q.n;
   double qk[kSlabs];
   uint32_t qa = 0;
   if (valid) {
@@ -741,13 +742,13 @@ __device__ __forceinline__ void walk64(const TreeView& q, const TreeView& t, uin
 }
 
 template <bool SELF, int K, bool CROSS = false>
-__global__ __launch_bounds__(256) void k_narrow64(TreeView q, TreeView t, int xcd, PairOut out) {
+__global__ __launch_bounds__(256) void k_narrow64(TreeView q, TreeView t, int xcd, uint32_t qper, PairOut out) {
   __shared__ uint64_t s_buf[256 / kWave][kWaveBuf];
   __shared__ uint32_t s_stack[256 / kWave][kStack];
   __shared__ Rec64 s_rec[256 / kWave][K];
   const uint32_t wv = threadIdx.x / kWave;
   const uint32_t tile = xcd ? xcd_tile(blockIdx.x, gridDim.x) : blockIdx.x;
-  walk64<SELF, K, CROSS>(q, t, tile, out, s_buf[wv], s_stack[wv], s_rec[wv]);
+  walk64<SELF, K, CROSS>(q, t, tile * (blockDim.x / kWave) + wv, qper, out, s_buf[wv], s_stack[wv], s_rec[wv]);
 }
 
 // Several queries (object pairs) in one launch: block b walks tile
@@ -767,7 +768,7 @@ __global__ __launch_bounds__(256) void k_narrow64_batch(const BatchQuery* __rest
   }
   const BatchQuery& e = bq[lo];
   if (blockIdx.x - e.block0 >= e.blocks) return;
-  walk64<false, K, false>(e.q, e.t, blockIdx.x - e.block0, e.out, s_buf[wv], s_stack[wv], s_rec[wv]);
+  walk64<false, K, false>(e.q, e.t, (blockIdx.x - e.block0) * (256 / kWave) + wv, kWave, e.out, s_buf[wv], s_stack[wv], s_rec[wv]);
 }
 
 // fp64 form, one record per visit in scalar registers (batch 1): box 0
@@ -779,7 +780,7 @@ __global__ __launch_bounds__(256) void k_narrow64_batch(const BatchQuery* __rest
 typedef __attribute__((address_space(4))) const double CDbl;
 
 template <bool SELF, bool CROSS = false>
-__global__ __launch_bounds__(256) void k_narrow64s(TreeView q, TreeView t, int xcd, PairOut out) {
+__global__ __launch_bounds__(256) void k_narrow64s(TreeView q, TreeView t, int xcd, uint32_t qper, PairOut out) {
   __shared__ uint64_t s_buf[256 / kWave][kWaveBuf];
   __shared__ uint32_t s_stack[256 / kWave][kStack];
   const uint32_t wv = threadIdx.x / kWave;
@@ -787,8 +788,8 @@ __global__ __launch_bounds__(256) void k_narrow64s(TreeView q, TreeView t, int x
   uint32_t* stk = s_stack[wv];
   uint32_t fill = 0;
   const uint32_t tile = xcd ? xcd_tile(blockIdx.x, gridDim.x) : blockIdx.x;
-  const uint64_t p = (uint64_t)tile * blockDim.x + threadIdx.x;
-  const bool valid = p < q.n;
+  const uint64_t p = ((uint64_t)tile * (blockDim.x / kWave) + wv) * qper + lane_id();
+  const bool valid = lane_id() < qper && p < q.n;
   double qk[kSlabs];
   uint32_t qa = 0;
   if (valid) {
@@ -1116,11 +1117,28 @@ __global__ __launch_bounds__(256) void k_digest(const uint64_t* __restrict__ pai
 
 // ---- launchers ---------------------------------------------------------------------
 template <int K>
-static void narrow64_dispatch(const TreeView& q, const TreeView& t, int self, int xcd, unsigned blocks, unsigned bs,
+static void narrow64_dispatch(const TreeView& q, const TreeView& t, int self, int xcd, uint32_t qper, unsigned blocks, unsigned bs,
                               const PairOut& out, hipStream_t s) {
-  if (self == 2) hipLaunchKernelGGL((k_narrow64<true, K, true>), dim3(blocks), dim3(bs), 0, s, q, t, xcd, out);
-  else if (self) hipLaunchKernelGGL((k_narrow64<true, K>), dim3(blocks), dim3(bs), 0, s, q, t, xcd, out);
-  else hipLaunchKernelGGL((k_narrow64<false, K>), dim3(blocks), dim3(bs), 0, s, q, t, xcd, out);
+  if (self == 2) hipLaunchKernelGGL((k_narrow64<true, K, true>), dim3(blocks), dim3(bs), 0, s, q, t, xcd, qper, out);
+  else if (self) hipLaunchKernelGGL((k_narrow64<true, K>), dim3(blocks), dim3(bs), 0, s, q, t, xcd, qper, out);
+  else hipLaunchKernelGGL((k_narrow64<false, K>), dim3(blocks), dim3(bs), 0, s, q, t, xcd, qper, out);
+}
+
+// Queries per wave: 64, or fewer (down to 4) while the launch has less than two
+// waves for each of the GPU's 1,024 SIMDs, one for a self walk.  A wave visits
+// what any of its lanes overlaps, so fewer queries visit less, and a small
+// object's launch, which lasts as long as its longest wave, gets shorter as long as
+// idle SIMDs take the added waves.  A x B over sheets, at 64 queries a wave and
+// by this rule: 2,048 queries 114 -> 46 us, 8,192 228 -> 69, 32,768 205 -> 119,
+// 89,888 200 -> 160 (181,202 stay at 64: 187 us, 230 at 32); over fp64 records
+// 192 -> 79, 394 -> 121, 373 -> 209, 372 -> 279.  Self walks visit half as
+// much: 8,000 spheres 60 -> 27 us (fp64 records 102 -> 49), 30,000 88 -> 49
+// (148 -> 91; with 2,048 waves 58 and 122), 60,000 105 -> 75 (174 -> 131).  The
+// cross-patch walk keeps 64: few of its queries have work.
+static uint32_t queries_per_wave(uint64_t n, int self) {
+  uint32_t qper = kWave;
+  while (self != 2 && qper > 4 && n / qper < (self ? 1024u : 2048u)) qper >>= 1;
+  return qper;
 }
 
 hipError_t launch_narrowphase(const TreeView& q, const TreeView& t, int leaf_size, int self, int form,
@@ -1131,7 +1149,9 @@ hipError_t launch_narrowphase(const TreeView& q, const TreeView& t, int leaf_siz
   if (bs != 64 && bs != 128 && bs != 256) return hipErrorInvalidValue;
   if (!q.perm || !t.perm || !t.root || !t.status || !out.pairs || !out.count) return hipErrorInvalidValue;
   if (self == 2 && (!q.patch_of_input || (q.od > 1 && !q.splits))) return hipErrorInvalidValue;
-  const unsigned blocks = (unsigned)((q.n + bs - 1) / bs);
+  const uint32_t qper = queries_per_wave(q.n, self);
+  const uint64_t per_block = (uint64_t)(bs / kWave) * qper;
+  const unsigned blocks = (unsigned)((q.n + per_block - 1) / per_block);
   const int xcd = shape.xcd_remap ? 1 : 0;
   if (form == kFormFp32 || form == kFormMixed) {
     if (!q.rec32 || !q.rootbox32 || !q.delta || !t.rec32 || !t.rootbox32 || !q.origin || !t.origin)
@@ -1142,9 +1162,12 @@ hipError_t launch_narrowphase(const TreeView& q, const TreeView& t, int leaf_siz
     // applies to the fp64 walk).  Both forms keep the leaf candidates whose
     // fp32 gap proves the fp64 overlap and re-check the rest in fp64.
     const int32_t inner = kInnerUlps;
-    if (self == 2) hipLaunchKernelGGL((k_narrow32<true, true>), dim3(blocks), dim3(bs), 0, s, q, t, xcd, out, inner);
-    else if (self) hipLaunchKernelGGL(k_narrow32<true>, dim3(blocks), dim3(bs), 0, s, q, t, xcd, out, inner);
-    else hipLaunchKernelGGL(k_narrow32<false>, dim3(blocks), dim3(bs), 0, s, q, t, xcd, out, inner);
+    if (self == 2) hipLaunchKernelGGL((k_narrow32<true, true>), dim3(blocks), dim3(bs), 0, s, q, t, xcd, qper, out,
+                                     inner);
+    else if (self) hipLaunchKernelGGL(k_narrow32<true>, dim3(blocks), dim3(bs), 0, s, q, t, xcd, qper, out,
+                                     inner);
+    else hipLaunchKernelGGL(k_narrow32<false>, dim3(blocks), dim3(bs), 0, s, q, t, xcd, qper, out,
+                                     inner);
     // in self mode both keys index the one object (q == t)
     uint64_t per = (out.rcap + 255) / 256;  // blocks per stripe
     if (per > kRecheckBlocksPerStripe) per = kRecheckBlocksPerStripe;
@@ -1155,12 +1178,12 @@ hipError_t launch_narrowphase(const TreeView& q, const TreeView& t, int leaf_siz
   if (!q.rec64 || !q.rootbox64 || !q.delta || !t.rec64 || !t.rootbox64) return hipErrorInvalidValue;
   switch (shape.batch) {
     case 1:
-      if (self == 2) hipLaunchKernelGGL((k_narrow64s<true, true>), dim3(blocks), dim3(bs), 0, s, q, t, xcd, out);
-      else if (self) hipLaunchKernelGGL(k_narrow64s<true>, dim3(blocks), dim3(bs), 0, s, q, t, xcd, out);
-      else hipLaunchKernelGGL(k_narrow64s<false>, dim3(blocks), dim3(bs), 0, s, q, t, xcd, out);
+      if (self == 2) hipLaunchKernelGGL((k_narrow64s<true, true>), dim3(blocks), dim3(bs), 0, s, q, t, xcd, qper, out);
+      else if (self) hipLaunchKernelGGL(k_narrow64s<true>, dim3(blocks), dim3(bs), 0, s, q, t, xcd, qper, out);
+      else hipLaunchKernelGGL(k_narrow64s<false>, dim3(blocks), dim3(bs), 0, s, q, t, xcd, qper, out);
       break;
-    case 2: narrow64_dispatch<2>(q, t, self, xcd, blocks, bs, out, s); break;
-    case 4: narrow64_dispatch<4>(q, t, self, xcd, blocks, bs, out, s); break;
+    case 2: narrow64_dispatch<2>(q, t, self, xcd, qper, blocks, bs, out, s); break;
+    case 4: narrow64_dispatch<4>(q, t, self, xcd, qper, blocks, bs, out, s); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
