@@ -237,7 +237,7 @@ struct bvh_object_s {
   const uint32_t* ref_rp = nullptr;
   const uint32_t* ref_perm() const { return split == BVH_SPLIT_CLUSTERING ? perm.as<uint32_t>() : ref_rp; }
   // results
-  DevBuf pairs, pairs_a, pairs_b, records, ppairs, sort_hist, sort_ctl, sort_lb, count, recheck, digest;
+  DevBuf pairs, pairs_a, pairs_b, records, ppairs, sort_hist, sort_ctl, sort_lb, count, recheck, items, digest;
   // exact primitive filter of the results: flags / offsets, kept pairs, scan words
   DevBuf ex_flag, ex_out, ex_lb, ex_ctr;
   // wire formats: patch centroids, patch ranges, element sources, host staging
@@ -306,7 +306,7 @@ struct bvh_object_s {
                      &depth_idx_b, &splits, &delta, &patch_of_pos, &patch_of_input, &counters, &patch_root,
                      &root, &rec64, &rootbox64, &rec32, &rootbox32, &status, &frame, &slab_err,
                      &front_a, &front_b, &patch_k64, &patch_box32, &pairs, &pairs_a, &pairs_b, &records, &ppairs,
-                     &sort_hist, &sort_ctl, &sort_lb, &count, &recheck, &digest, &sp_rp, &sp_rp_b,
+                     &sort_hist, &sort_ctl, &sort_lb, &count, &recheck, &items, &digest, &sp_rp, &sp_rp_b,
                      &sp_scan, &sp_tmpf, &sp_tmpt, &sp_seg, &sp_seg_next, &sp_k64, &sp_acc, &sp_axis,
                      &sp_flag, &sp_lb, &sp_ctr, &sp_key, &key0, &key_a, &key_b, &sp_hist, &sp_x, &sp_blk,
                      &ex_flag, &ex_out, &ex_lb, &ex_ctr, &wire_cent, &wire_range, &wire_src, &wire_out,
@@ -889,11 +889,12 @@ static bvh_status set_entity_build(bvh_object_s* o, int kind, int nv, double eps
 // Counter words of a query (device, o->count): pairs, node visits, fp32
 // candidates, fp32 re-checks (sum and largest stripe), patch pairs; from word
 // kCntStripes on, the fp32 re-check list's stripe counters, one 128-byte line
-// each.
+// each, and a line for the length of the cross-patch walk's split list.
 constexpr int kCntPairs = 0, kCntVisits = 1, kCntCand = 2, kCntRecheck = 3, kCntRecheckMax = 4, kCntPatch = 5,
               kCntWords = 6;
 constexpr uint64_t kCntStripes = 16;
-constexpr uint64_t kCntTotal = kCntStripes + (uint64_t)kRecheckStripes * kRecheckStride;
+constexpr uint64_t kCntItems = kCntStripes + (uint64_t)kRecheckStripes * kRecheckStride;
+constexpr uint64_t kCntTotal = kCntItems + kRecheckStride;
 
 // Reads the counters of the last query of `o` and the device error words of
 // both objects (one synchronization).  Sets *overflow when a list outgrew
@@ -978,7 +979,8 @@ static bvh_status ensure_patch_pairs(bvh_object_s* o) {
   for (int attempt = 0; attempt < 2; ++attempt) {
     o->q_pcap = o->ppairs.bytes / 8;
     HIP_TRY(launch_fill_u32((uint32_t*)(dcount + kCntPatch), 2, 0u, s));
-    PairOut po{o->ppairs.as<uint64_t>(), o->q_pcap, dcount + kCntPatch, nullptr, nullptr, nullptr, 0, nullptr, nullptr};
+    PairOut po{o->ppairs.as<uint64_t>(), o->q_pcap, dcount + kCntPatch, nullptr, nullptr, nullptr, 0, nullptr, nullptr,
+               nullptr, 0, nullptr};
     HIP_TRY(launch_patch_broadphase(view_of(o), view_of(t), o->fp32, po, s));
     unsigned long long cnt = 0;
     BVH_TRY(copy_out(&cnt, dcount + kCntPatch, sizeof(cnt), BVH_MEM_HOST, s));
@@ -1013,7 +1015,8 @@ static bvh_status launch_query(bvh_object_s* o, bvh_object_s* other, bool self, 
     w->stage_begin("broadphase");
     BVH_TRY(ensure_patch_slabs(o));
     BVH_TRY(ensure_patch_slabs(other));
-    PairOut po{o->ppairs.as<uint64_t>(), o->q_pcap, dcount + kCntPatch, nullptr, nullptr, nullptr, 0, nullptr, nullptr};
+    PairOut po{o->ppairs.as<uint64_t>(), o->q_pcap, dcount + kCntPatch, nullptr, nullptr, nullptr, 0, nullptr, nullptr,
+               nullptr, 0, nullptr};
     HIP_TRY(launch_patch_broadphase(qv, tv, o->fp32, po, s));
     o->patch_pairs_ready = true;
     w->stage_end();
@@ -1021,7 +1024,8 @@ static bvh_status launch_query(bvh_object_s* o, bvh_object_s* other, bool self, 
   if (narrow) {
     w->stage_begin("narrowphase");
     PairOut po{o->pairs.as<uint64_t>(), o->q_cap, dcount + kCntPairs, dcount + kCntVisits, dcount + kCntCand,
-               o->recheck.as<uint64_t>(), o->q_rcap, dcount + kCntStripes, dcount + kCntRecheck};
+               o->recheck.as<uint64_t>(), o->q_rcap, dcount + kCntStripes, dcount + kCntRecheck,
+               o->items.as<uint64_t>(), o->items.bytes / 8, dcount + kCntItems};
     HIP_TRY(launch_narrowphase(qv, tv, (int)w->cfg.leaf_size, self ? (cross ? 2 : 1) : 0, o->form, w->shape, po, s));
     w->stage_end();
   }
@@ -1044,6 +1048,15 @@ static bvh_status grow_query_lists(bvh_object_s* o) {
   return BVH_OK;
 }
 
+// The fp32 walk's lists at their first sizes.  The split list is there from the
+// first query of any kind, so that a capture finds it.
+static bvh_status first_query_lists(bvh_object_s* o) {
+  if (!o->fp32) return BVH_OK;
+  const uint64_t bytes = std::max<uint64_t>(1u << 16, o->in.n) * 8;
+  BVH_TRY(o->recheck.ensure(bytes));
+  return o->items.ensure(bytes);
+}
+
 static bvh_status run_query(bvh_object_s* o, bvh_object_s* other, bool self, bool narrow = true, bool cross = false) {
   bvh_world w = o->w;
   if (!o->built || !other->built) return fail(BVH_E_STATE, "set_entity_data must precede broadphase");
@@ -1056,7 +1069,7 @@ static bvh_status run_query(bvh_object_s* o, bvh_object_s* other, bool self, boo
   BVH_TRY(o->ppairs.ensure(std::max<uint64_t>(1024, 4 * w->od) * 8));
   if (narrow) {
     BVH_TRY(ensure_pairs(o, std::max<uint64_t>(1u << 20, 8 * o->in.n)));
-    if (o->fp32) BVH_TRY(o->recheck.ensure(std::max<uint64_t>(1u << 16, o->in.n) * 8));
+    BVH_TRY(first_query_lists(o));
   }
   if (w->capturing) {
     BVH_TRY(launch_query(o, other, self, narrow, cross));
@@ -1102,7 +1115,7 @@ static bvh_status run_query_batch(bvh_object_s* const* os, bvh_object_s* const* 
     BVH_TRY(o->count.ensure(kCntTotal * sizeof(unsigned long long)));
     BVH_TRY(o->ppairs.ensure(std::max<uint64_t>(1024, 4 * w->od) * 8));
     BVH_TRY(ensure_pairs(o, std::max<uint64_t>(1u << 20, 8 * o->in.n)));
-    if (o->fp32) BVH_TRY(o->recheck.ensure(std::max<uint64_t>(1u << 16, o->in.n) * 8));
+    BVH_TRY(first_query_lists(o));
   }
   if (k > w->bq_host_cap) {
     if (w->bq_host) (void)hipHostFree(w->bq_host);
@@ -1138,11 +1151,14 @@ static bvh_status run_query_batch(bvh_object_s* const* os, bvh_object_s* const* 
     BatchQuery& e = w->bq_host[nq++];
     e.q = qv;
     e.t = tv;
-    e.out = o->fp32 ? PairOut{o->pairs.as<uint64_t>(), o->q_cap, dcount + kCntPairs, dcount + kCntVisits,
-                              dcount + kCntCand, o->recheck.as<uint64_t>(), o->q_rcap, dcount + kCntStripes,
-                              dcount + kCntRecheck}
-                    : PairOut{o->pairs.as<uint64_t>(), o->q_cap, dcount + kCntPairs, dcount + kCntVisits,
-                              dcount + kCntCand, nullptr, 0, nullptr, nullptr};
+    e.out = PairOut{o->pairs.as<uint64_t>(), o->q_cap, dcount + kCntPairs, dcount + kCntVisits, dcount + kCntCand,
+                    nullptr, 0, nullptr, nullptr, nullptr, 0, nullptr};
+    if (o->fp32) {
+      e.out.recheck = o->recheck.as<uint64_t>();
+      e.out.rcap = o->q_rcap;
+      e.out.rcount = dcount + kCntStripes;
+      e.out.rtotal = dcount + kCntRecheck;
+    }
     e.block0 = blocks;
     e.blocks = (uint32_t)((o->in.n + 255) / 256);
     blocks += e.blocks;

@@ -320,6 +320,11 @@ struct PairOut {
   uint64_t rcap;
   unsigned long long* rcount;
   unsigned long long* rtotal;
+  // fp32 cross-patch walk: the split list (subtrees that a wave leaves to a
+  // second launch) and its length, which may pass icap
+  uint64_t* items;
+  uint64_t icap;
+  unsigned long long* icount;
 };
 
 constexpr uint32_t kRecheckStripes = 64;

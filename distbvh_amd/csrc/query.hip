@@ -257,21 +257,19 @@ __device__ __forceinline__ void own_patch_range(const TreeView& q, uint32_t qa, 
   pe = (uint64_t)k + 1 >= q.od ? n : q.splits[k];
 }
 
-// The fp32-outward record walk of one wave's qper queries (the body of
-// k_narrow32 and of its batched form k_narrow32_batch); buf / rbuf / stk are
-// the wave's LDS pair staging, re-check staging and stack, rstripe the
-// wave's re-check stripe.  Leaf candidates with a gap above `inner` are
-// emitted, the rest queued for the fp64 re-check.
-template <bool SELF, bool CROSS>
-__device__ __forceinline__ void walk32(const TreeView& q, const TreeView& t, uint32_t wave, uint32_t qper,
-                                       const PairOut& out, int32_t inner, uint64_t* buf, uint64_t* rbuf, uint32_t* stk,
-                                       uint32_t rstripe) {
-  uint32_t fill = 0, rfill = 0;
-  const uint64_t p = (uint64_t)wave * qper + lane_id();
-  const bool valid = lane_id() < qper && p < q.n;
-  if (q.origin != t.origin) inner = 0x7fffffff;
-  int32_t qf[kSlabs];  // ord32 images of the query's outward fp32 slabs
-  uint32_t qa = 0;
+// A lane's query: the slabs (ord32 images, in the frame of the tree t), input
+// index and position of position p of the query object's order.
+struct Query32 {
+  int32_t s[kSlabs];
+  uint32_t elem, pos;  // (0 for a lane without a query, which hits nothing)
+  bool valid;
+};
+template <bool SELF>
+__device__ __forceinline__ void load_query32(const TreeView& q, const TreeView& t, uint64_t p, bool valid,
+                                             Query32& r) {
+  r.valid = valid;
+  r.elem = 0;
+  r.pos = valid ? (uint32_t)p : 0u;  // positions fit 32 bits
   if (valid) {
     // this leaf's slabs: its half of its parent's record (the root's array if n = 1)
     const int32_t* src = q.rootbox32;
@@ -284,31 +282,82 @@ __device__ __forceinline__ void walk32(const TreeView& q, const TreeView& t, uin
 #pragma unroll
     for (int a = 0; a < kAxes; ++a) {
       const int2 v = ((const int2*)src)[a];
-      qf[2 * a] = v.x;
-      qf[2 * a + 1] = v.y;
+      r.s[2 * a] = v.x;
+      r.s[2 * a + 1] = v.y;
     }
-    qa = q.perm[p];
+    r.elem = q.perm[p];
     // another object's tree has its own frame: the slabs moved to it, still
     // outward (their fp32 rounding then bounds nothing from the inside, so
     // every candidate of such a query is decided in fp64)
-    if (q.origin != t.origin)
-      reframe32(qf, q.origin[0], q.origin[1], q.origin[2], t.origin[0], t.origin[1], t.origin[2]);
+    if (!SELF && q.origin != t.origin)
+      reframe32(r.s, q.origin[0], q.origin[1], q.origin[2], t.origin[0], t.origin[1], t.origin[2]);
   } else {
 #pragma unroll
     for (int a = 0; a < kAxes; ++a) {  // the empty box overlaps nothing
-      qf[2 * a] = 0x7fffffff;
-      qf[2 * a + 1] = (int32_t)0x80000000;
+      r.s[2 * a] = 0x7fffffff;
+      r.s[2 * a + 1] = (int32_t)0x80000000;
     }
   }
+}
+
+// What a wave does with its queries: the whole walk; the walk's top, leaving
+// subtrees of at most kItemLeaves leaves to a second launch as items of the
+// split list ((wave << 32) | subtree root) once it has made kItemBudget visits;
+// or a run of such items.  The cross-patch walk is split: where meshes of
+// uneven sizes meet, a coarse element overlaps thousands of a fine mesh's, and
+// its wave alone (7,700 visits among 213 on average over 512 meshes of
+// lognormal size) held the launch for 4,577 us.  Split, it takes 1,465 + 1,092;
+// with 128 or 64 visits before the split, or 32 or 128 leaves an item, 2,536 to
+// 2,661 us.  Evenly loaded walks lose by it (contact of 2 x 2M triangles 1,158
+// -> 1,271 us: the split's registers cost every visit) and stay whole.
+constexpr int kWalkWhole = 0, kWalkTop = 1, kWalkItems = 2;
+constexpr uint32_t kItemBuf = 32;  // staged items per wave
+constexpr uint32_t kItemBudget = 256;
+constexpr uint32_t kItemLeaves = 64;
+constexpr unsigned kItemBlocks = 1792;  // seven a CU
+
+// Appends the wave's n staged subtree roots to the split list; returns how
+// many found room (the list is sized by the queries, not by the data: the wave
+// walks the others itself).
+__device__ __forceinline__ uint32_t items_flush(const uint32_t* ibuf, uint32_t n, uint32_t wave, const PairOut& out) {
+  if (n == 0) return 0;
+  __builtin_amdgcn_wave_barrier();
+  unsigned long long base = 0;
+  if (lane_id() == 0) base = atomicAdd(out.icount, (unsigned long long)n);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)base);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(base >> 32));
+  base = ((unsigned long long)hi << 32) | lo;
+  const uint32_t room = base >= out.icap ? 0u : (uint32_t)(out.icap - base < n ? out.icap - base : n);
+  if (lane_id() < room) out.items[base + lane_id()] = ((uint64_t)wave << 32) | ibuf[lane_id()];
+  __builtin_amdgcn_wave_barrier();
+  return room;
+}
+
+// The fp32-outward record walk of one wave (the body of k_narrow32 and of its
+// batched and item forms): the qper queries from position wave * qper on, one
+// lane each, or, as kWalkItems, the items [i0, i1) of the split list; buf /
+// rbuf / stk / ibuf are the wave's LDS pair staging, re-check staging, stack
+// and item staging, rstripe the wave's re-check stripe.  Leaf candidates with
+// a gap above `inner` are emitted, the rest queued for the fp64 re-check.
+template <bool SELF, bool CROSS, int MODE>
+__device__ __forceinline__ void walk32(const TreeView& q, const TreeView& t, uint32_t wave, uint32_t qper, uint64_t i0,
+                                       uint64_t i1, const PairOut& out, int32_t inner, uint64_t* buf, uint64_t* rbuf,
+                                       uint32_t* stk, uint32_t* ibuf, uint32_t rstripe) {
+  uint32_t fill = 0, rfill = 0;
+  if (!SELF && q.origin != t.origin) inner = 0x7fffffff;
+  uint64_t item = MODE == kWalkItems ? out.items[i0] : 0;
+  if (MODE == kWalkItems) wave = uniform((uint32_t)(item >> 32));
+  Query32 Q;
+  uint64_t p0 = (uint64_t)wave * qper + lane_id();
+  load_query32<SELF>(q, t, p0, lane_id() < qper && p0 < q.n, Q);
   const uint32_t n = (uint32_t)t.n;
   const uint32_t tleaf0 = n - 1;
   const uint32_t lane = lane_id();
-  const uint32_t p32 = valid ? (uint32_t)p : 0u;  // positions fit 32 bits; invalid lanes hit nothing
   uint32_t pb = 0, pe = 0;
-  if (CROSS) own_patch_range(q, qa, valid, n, pb, pe);
+  if (CROSS) own_patch_range(q, Q.elem, Q.valid, n, pb, pe);
   CRec32* recs = (CRec32*)t.rec32;
   uint32_t sink = 0, pf = 0;  // record prefetch (below)
-  uint32_t steps = 0;
+  uint32_t steps = 0, total = 0;
   uint32_t ncand = 0;
   // fp32 candidates at one (wave-uniform) leaf, gap g per lane: emit what
   // the inner bound proves, queue the rest for the fp64 re-check
@@ -317,7 +366,7 @@ __device__ __forceinline__ void walk32(const TreeView& q, const TreeView& t, uin
     if (m == 0) return;
     ncand += (uint32_t)__popcll(m);
     const bool sure = h & (g > inner);
-    const uint64_t key = pair_key(qa, elem, SELF);
+    const uint64_t key = pair_key(Q.elem, elem, SELF);
     wave_emit(buf, fill, out, sure, key);
     const bool unsure = h & !sure;
     const uint64_t mu = __ballot(unsure);
@@ -335,10 +384,10 @@ __device__ __forceinline__ void walk32(const TreeView& q, const TreeView& t, uin
   bool from_root = true;
   // (not in the cross-patch self walk: its workloads have many patches, and
   // the start's registers would cost that kernel a wave per SIMD)
-  if (!CROSS && t.patch_box32 != nullptr && n > 1 && od > 1 && od <= kFrontierMax) {
+  if (MODE != kWalkItems && !CROSS && t.patch_box32 != nullptr && n > 1 && od > 1 && od <= kFrontierMax) {
     // self: patches that end at or before the wave's first position hold no
     // pair of it
-    const uint32_t pmin = __builtin_amdgcn_readlane(p32, 0);
+    const uint32_t pmin = __builtin_amdgcn_readlane(Q.pos, 0);
     // lane l tests patches l, l + 64, ... (clamped to the last patch, with
     // the test off); the union is reduced one axis at a time, so that it
     // takes two scalar registers and each axis's loads go out together
@@ -353,7 +402,7 @@ __device__ __forceinline__ void walk32(const TreeView& q, const TreeView& t, uin
     }
 #pragma unroll
     for (int a = 0; a < kAxes; ++a) {
-      const int32_t ulo = wave_reduce_i32<false>(qf[2 * a]), uhi = wave_reduce_i32<true>(qf[2 * a + 1]);
+      const int32_t ulo = wave_reduce_i32<false>(Q.s[2 * a]), uhi = wave_reduce_i32<true>(Q.s[2 * a + 1]);
       const int32_t* plo = t.patch_box32 + (uint64_t)(2 * a) * od;  // this axis's slabs of every patch
       const int32_t* phi = plo + od;
 #pragma unroll
@@ -398,29 +447,55 @@ __device__ __forceinline__ void walk32(const TreeView& q, const TreeView& t, uin
           int32_t bx[kSlabs];
 #pragma unroll
           for (int a = 0; a < kSlabs; ++a) bx[a] = t.patch_box32[(uint64_t)a * od + k];
-          const int32_t g = min_gap(qf, bx);
+          const int32_t g = min_gap(Q.s, bx);
           bool hit = g > 0;
-          if (SELF) hit = hit & (pos > p32);
+          if (SELF) hit = hit & (pos > Q.pos);
           leaf_check(g, uniform(t.perm[pos]), hit);
         }
       }
     }
   }
-  if (from_root) {
-    const int32_t g = min_gap(qf, (CInt*)t.rootbox32);
+  if (MODE == kWalkItems) {
+    x = uniform((uint32_t)item);
+  } else if (from_root) {
+    const int32_t g = min_gap(Q.s, (CInt*)t.rootbox32);
     bool h = g > 0;
-    if (SELF) h = h & ((n - 1) > p32);  // the root's last position
+    if (SELF) h = h & ((n - 1) > Q.pos);  // the root's last position
     if (n == 1) {
       if (!SELF) leaf_check(g, uniform(t.perm[0]), h);
     } else if (__ballot(h) != 0) {
       x = uniform(*t.root);
     }
   }
+  // kWalkTop: staged items; once the list is full, the first of them left to
+  // this wave (else kEnd: still splitting)
+  uint32_t nitem = 0, kept = kEnd;
   for (;;) {
     if (x == kEnd) {
-      if (sp == 0) break;
-      x = uniform(stk[--sp]);
+      if (sp != 0) {
+        x = uniform(stk[--sp]);
+      } else if (MODE == kWalkItems) {
+        if (++i0 >= i1) break;
+        item = out.items[i0];
+        if (uniform((uint32_t)(item >> 32)) != wave) {  // another wave's queries
+          wave = uniform((uint32_t)(item >> 32));
+          p0 = (uint64_t)wave * qper + lane;
+          load_query32<SELF>(q, t, p0, lane < qper && p0 < q.n, Q);
+          if (CROSS) own_patch_range(q, Q.elem, Q.valid, n, pb, pe);
+        }
+        x = uniform((uint32_t)item);
+        steps = 0;  // (visits of earlier items: total)
+      } else if (MODE == kWalkTop && nitem != 0) {
+        if (kept == kEnd) {  // the walk is done but for its staged items
+          kept = items_flush(ibuf, nitem, wave, out);
+        }
+        if (kept >= nitem) break;
+        x = uniform(ibuf[kept++]);
+      } else {
+        break;
+      }
     }
+    if (MODE == kWalkItems) ++total;
     if (x >= tleaf0 || ++steps > n) {
       if (lane == 0) atomicOr(t.status, kErrTraverse);
       break;
@@ -458,8 +533,8 @@ __device__ __forceinline__ void walk32(const TreeView& q, const TreeView& t, uin
     // (self) and the own patch (cross), non-short-circuit &: no branch
     bool okl = true, okr = true;
     if (SELF) {
-      okl = x > p32;  // the left child ends at position x
-      okr = rlast > p32;
+      okl = x > Q.pos;  // the left child ends at position x
+      okr = rlast > Q.pos;
     }
     if (CROSS) {  // children [rfirst, x] and [x + 1, rlast] inside the lane's own patch
       okl = okl & !((rfirst >= pb) & (x < pe));
@@ -470,17 +545,34 @@ __device__ __forceinline__ void walk32(const TreeView& q, const TreeView& t, uin
     // also gets each lane's gap for the candidate test (both gaps before
     // either test, so the record's registers are free by then)
     int32_t gl = 0, gr = 0;
-    uint64_t ml = box_mask32(qf, rw), mr = box_mask32(qf, rw + 28);
+    uint64_t ml = box_mask32(Q.s, rw), mr = box_mask32(Q.s, rw + 28);
     if (SELF || CROSS) {
       ml &= __ballot(okl);
       mr &= __ballot(okr);
     }
-    if (leaf_l && ml != 0) gl = min_gap(qf, rw);
-    if (leaf_r && mr != 0) gr = min_gap(qf, rw + 28);
+    if (leaf_l && ml != 0) gl = min_gap(Q.s, rw);
+    if (leaf_r && mr != 0) gr = min_gap(Q.s, rw + 28);
     const bool any_l = ml != 0, any_r = mr != 0;
-    if (any_l && leaf_l) leaf_check(gl, el, (gl > 0) & okl & (!SELF || (cl - tleaf0 > p32)));
-    if (any_r && leaf_r) leaf_check(gr, er, (gr > 0) & okr & (!SELF || (cr - tleaf0 > p32)));
-    const bool go_l = any_l && !leaf_l, go_r = any_r && !leaf_r;
+    if (any_l && leaf_l) leaf_check(gl, el, (gl > 0) & okl & (!SELF || (cl - tleaf0 > Q.pos)));
+    if (any_r && leaf_r) leaf_check(gr, er, (gr > 0) & okr & (!SELF || (cr - tleaf0 > Q.pos)));
+    bool go_l = any_l && !leaf_l, go_r = any_r && !leaf_r;
+    if (MODE == kWalkTop && steps > kItemBudget && kept == kEnd) {
+      // children of few leaves become items (this node's range: half 0)
+      const uint32_t first = recs[x].h[0].first, last = recs[x].h[0].last;
+      if (go_l && x - first < kItemLeaves) {
+        ibuf[nitem++] = cl;
+        go_l = false;
+      }
+      if (go_r && last - x <= kItemLeaves) {
+        ibuf[nitem++] = cr;
+        go_r = false;
+      }
+      if (nitem + 2 > kItemBuf) {
+        const uint32_t room = items_flush(ibuf, nitem, wave, out);
+        if (room < nitem) kept = room;
+        else nitem = 0;
+      }
+    }
     // depth first: continue with the left child, keep the right one
     if (go_l && go_r) {
       if (sp >= kStack) {
@@ -499,21 +591,45 @@ __device__ __forceinline__ void walk32(const TreeView& q, const TreeView& t, uin
   asm volatile("; record prefetch sink %0" ::"v"(sink));  // keeps the prefetch loads
   if (lane == 0) {  // in the stripe's line; k_recheck adds the stripes up
     unsigned long long* line = out.rcount + (uint64_t)rstripe * kRecheckStride;
-    atomicAdd(line + 1, (unsigned long long)steps);
+    atomicAdd(line + 1, (unsigned long long)(MODE == kWalkItems ? total : steps));
     atomicAdd(line + 2, (unsigned long long)ncand);
   }
 }
 
-template <bool SELF, bool CROSS = false>
+// The LDS of a block of the walk, per wave (the split walk has items too).
+struct Walk32Lds {
+  uint64_t buf[256 / kWave][kWaveBuf];
+  uint64_t rbuf[256 / kWave][kRecheckBuf];
+  uint32_t stack[256 / kWave][kStack];
+};
+
+template <bool SELF, bool CROSS, int MODE = kWalkWhole>
 __global__ __launch_bounds__(256) void k_narrow32(TreeView q, TreeView t, int xcd, uint32_t qper, PairOut out,
                                                   int32_t inner) {
-  __shared__ uint64_t s_buf[256 / kWave][kWaveBuf];
-  __shared__ uint64_t s_rbuf[256 / kWave][kRecheckBuf];
-  __shared__ uint32_t s_stack[256 / kWave][kStack];
-  const uint32_t wv = threadIdx.x / kWave;
-  const uint32_t rstripe = (blockIdx.x * (blockDim.x / kWave) + wv) % kRecheckStripes;
+  __shared__ Walk32Lds L;
+  __shared__ uint32_t s_items[256 / kWave][MODE == kWalkTop ? kItemBuf : 1];
+  const uint32_t wv = threadIdx.x / kWave, nw = blockDim.x / kWave;
+  const uint32_t rstripe = (blockIdx.x * nw + wv) % kRecheckStripes;
   const uint32_t tile = xcd ? xcd_tile(blockIdx.x, gridDim.x) : blockIdx.x;
-  walk32<SELF, CROSS>(q, t, tile * (blockDim.x / kWave) + wv, qper, out, inner, s_buf[wv], s_rbuf[wv], s_stack[wv], rstripe);
+  walk32<SELF, CROSS, MODE>(q, t, tile * nw + wv, qper, 0, 0, out, inner, L.buf[wv], L.rbuf[wv], L.stack[wv],
+                            s_items[wv], rstripe);
+}
+
+// The split list of a query: a contiguous run of items per wave (items of one
+// wave's queries are neighbours, which share the loaded queries).
+template <bool SELF, bool CROSS>
+__global__ __launch_bounds__(256) void k_narrow32_items(TreeView q, TreeView t, uint32_t qper, PairOut out,
+                                                        int32_t inner) {
+  __shared__ Walk32Lds L;
+  const uint32_t wv = threadIdx.x / kWave, nw = blockDim.x / kWave;
+  const uint32_t wave = uniform(blockIdx.x * nw + wv);
+  const unsigned long long c = *out.icount;
+  const uint64_t cnt = c < out.icap ? c : out.icap;
+  const uint64_t per = (cnt + (uint64_t)gridDim.x * nw - 1) / ((uint64_t)gridDim.x * nw);
+  const uint64_t i0 = wave * per, i1 = i0 + per < cnt ? i0 + per : cnt;
+  if (i0 >= i1) return;
+  walk32<SELF, CROSS, kWalkItems>(q, t, 0, qper, i0, i1, out, inner, L.buf[wv], L.rbuf[wv], L.stack[wv], nullptr,
+                                  wave % kRecheckStripes);
 }
 
 // Several queries (object pairs) in one launch of the fp32-outward walk:
@@ -521,9 +637,7 @@ __global__ __launch_bounds__(256) void k_narrow32(TreeView q, TreeView t, int xc
 // blocks) holds b (a wave-uniform binary search over the table).
 __global__ __launch_bounds__(256) void k_narrow32_batch(const BatchQuery* __restrict__ bq, uint32_t nq,
                                                         int32_t inner) {
-  __shared__ uint64_t s_buf[256 / kWave][kWaveBuf];
-  __shared__ uint64_t s_rbuf[256 / kWave][kRecheckBuf];
-  __shared__ uint32_t s_stack[256 / kWave][kStack];
+  __shared__ Walk32Lds L;
   const uint32_t wv = threadIdx.x / kWave;
   uint32_t lo = 0, hi = nq;
   while (hi - lo > 1) {
@@ -534,8 +648,8 @@ __global__ __launch_bounds__(256) void k_narrow32_batch(const BatchQuery* __rest
   const BatchQuery& e = bq[lo];
   if (blockIdx.x - e.block0 >= e.blocks) return;
   const uint32_t wave = (blockIdx.x - e.block0) * (256 / kWave) + wv;
-  const uint32_t rstripe = wave % kRecheckStripes;
-  walk32<false, false>(e.q, e.t, wave, kWave, e.out, inner, s_buf[wv], s_rbuf[wv], s_stack[wv], rstripe);
+  walk32<false, false, kWalkWhole>(e.q, e.t, wave, kWave, 0, 0, e.out, inner, L.buf[wv], L.rbuf[wv], L.stack[wv],
+                                   nullptr, wave % kRecheckStripes);
 }
 
 // Strict overlap of the lane's query slabs q with one box b whose 26 slabs
@@ -1162,12 +1276,15 @@ hipError_t launch_narrowphase(const TreeView& q, const TreeView& t, int leaf_siz
     // applies to the fp64 walk).  Both forms keep the leaf candidates whose
     // fp32 gap proves the fp64 overlap and re-check the rest in fp64.
     const int32_t inner = kInnerUlps;
-    if (self == 2) hipLaunchKernelGGL((k_narrow32<true, true>), dim3(blocks), dim3(bs), 0, s, q, t, xcd, qper, out,
-                                     inner);
-    else if (self) hipLaunchKernelGGL(k_narrow32<true>, dim3(blocks), dim3(bs), 0, s, q, t, xcd, qper, out,
-                                     inner);
-    else hipLaunchKernelGGL(k_narrow32<false>, dim3(blocks), dim3(bs), 0, s, q, t, xcd, qper, out,
-                                     inner);
+    if (self == 2) {
+      if (!out.items || !out.icount) return hipErrorInvalidValue;
+      hipLaunchKernelGGL((k_narrow32<true, true, kWalkTop>), dim3(blocks), dim3(bs), 0, s, q, t, xcd, qper, out, inner);
+      hipLaunchKernelGGL((k_narrow32_items<true, true>), dim3(kItemBlocks), dim3(256), 0, s, q, t, qper, out, inner);
+    } else if (self) {
+      hipLaunchKernelGGL((k_narrow32<true, false>), dim3(blocks), dim3(bs), 0, s, q, t, xcd, qper, out, inner);
+    } else {
+      hipLaunchKernelGGL((k_narrow32<false, false>), dim3(blocks), dim3(bs), 0, s, q, t, xcd, qper, out, inner);
+    }
     // in self mode both keys index the one object (q == t)
     uint64_t per = (out.rcap + 255) / 256;  // blocks per stripe
     if (per > kRecheckBlocksPerStripe) per = kRecheckBlocksPerStripe;

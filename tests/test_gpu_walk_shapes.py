@@ -38,3 +38,29 @@ def test_queries_per_wave(n, precision):
         if n <= 8193:
             oa.self_collision()
             assert np.array_equal(sort_pairs(oa.pairs()), sort_pairs(O.brute_self(ka)))
+
+
+@pytest.mark.parametrize("precision", FORMS)
+@pytest.mark.parametrize("na,nb,every", [(63, 65, 1), (300, 500, 7), (2000, 9000, 40), (9000, 2000, 640),
+                                         (14000, 20000, 40)])
+def test_cross_patch_uneven(na, nb, every, precision):
+    """Two meshes as patches, every `every`-th element of one overlapping all
+    of the other: waves of many times the usual visits, and in the largest case
+    more left-over subtrees than their list holds (65,536)."""
+    from distbvh_amd import GIVEN
+    rng = np.random.default_rng(na)
+    a, b = _spheres(na, rng), _spheres(nb, rng)
+    b[0] += 2.0  # apart but for the big ones
+    a[3] *= 0.1
+    b[3] *= 0.1
+    big = rng.permutation(na)[: max(1, na // every)]
+    a[3, big] = 6.0
+    with CollisionWorld(2, precision=precision) as w:
+        o = w.create_collision_object()
+        o.set_patch_offsets([na])
+        o.set_entity_data_sphere(to_cuda(np.concatenate([a, b], axis=1)), split_algorithm=GIVEN)
+        o.init_broadphase()
+        o.self_collision_cross_patch()
+        got = sort_pairs(o.pairs())
+    want = np.stack([np.repeat(np.sort(big), nb), np.tile(np.arange(na, na + nb), len(big))], axis=1)
+    assert np.array_equal(got.astype(np.int64), want)
