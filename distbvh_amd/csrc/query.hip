@@ -183,7 +183,10 @@ __device__ __forceinline__ int32_t min_gap(const int32_t* q, P b) {
 // children of the fp32 walk (a leaf child needs the gap, min_gap).  Returns
 // the mask of the lanes that hit (EXEC after the chain; every lane of the
 // wave is active in the walk), which stays in scalar registers: an internal
-// child only needs to know whether any lane hits it.
+// child only needs to know whether any lane hits it.  Every second box is missed
+// by all lanes, mostly on x, y or z: the chain ends there if no lane is left
+// (walk of 2 x 2M triangles 1,149 -> 1,086 us; leaving after one axis, or at more
+// places, gains less or nothing).
 __device__ __forceinline__ uint64_t box_mask32(const int32_t* q, const int32_t* b) {
   unsigned long long res, save, m;
   asm volatile(
@@ -194,6 +197,8 @@ __device__ __forceinline__ uint64_t box_mask32(const int32_t* q, const int32_t* 
       "v_cmpx_lt_i32_e64 %[m], %[b2], %[q3]\n\t"
       "v_cmpx_lt_i32_e64 %[m], %[q4], %[b5]\n\t"
       "v_cmpx_lt_i32_e64 %[m], %[b4], %[q5]\n\t"
+      "s_nop 4\n\t"
+      "s_cbranch_execz .Lmiss%=\n\t"
       "v_cmpx_lt_i32_e64 %[m], %[q6], %[b7]\n\t"
       "v_cmpx_lt_i32_e64 %[m], %[b6], %[q7]\n\t"
       "v_cmpx_lt_i32_e64 %[m], %[q8], %[b9]\n\t"
@@ -214,7 +219,8 @@ __device__ __forceinline__ uint64_t box_mask32(const int32_t* q, const int32_t* 
       "v_cmpx_lt_i32_e64 %[m], %[b22], %[q23]\n\t"
       "v_cmpx_lt_i32_e64 %[m], %[q24], %[b25]\n\t"
       "v_cmpx_lt_i32_e64 %[m], %[b24], %[q25]\n\t"
-      "s_nop 4\n\t"
+      "s_nop 4\n"
+      ".Lmiss%=:\n\t"
       "s_mov_b64 %[res], exec\n\t"
       "s_mov_b64 exec, %[save]\n\t"
       : [res] "=&s"(res), [save] "=&s"(save), [m] "=&s"(m)
@@ -704,20 +710,72 @@ __device__ __forceinline__ uint64_t box_hits(const double* q, const double* b, u
   return res;
 }
 
-// Both boxes of an LDS-staged fp64 record against the lane's query slabs,
-// one axis at a time: the scheduling barrier after each axis keeps four of
-// the record's doubles in registers, which holds the walk at 88-94 VGPRs
-// (5 waves per SIMD) where loading both boxes at once needs over 128.
-__device__ __forceinline__ void overlap_pair(const double* qk, const Rec64& r, bool& h0, bool& h1) {
-  bool o0 = true, o1 = true;
-#pragma unroll
-  for (int a = 0; a < kAxes; ++a) {
-    o0 = o0 & (qk[2 * a] < r.box[0][2 * a + 1]) & (r.box[0][2 * a] < qk[2 * a + 1]);
-    o1 = o1 & (qk[2 * a] < r.box[1][2 * a + 1]) & (r.box[1][2 * a] < qk[2 * a + 1]);
-    __builtin_amdgcn_sched_barrier(0);
+// N axes of a box in LDS against the lane's query slabs, for the lanes in
+// `mask`: the v_cmpx chain of box_hits.  Returns the lanes that hit.
+template <int N>
+__device__ __forceinline__ uint64_t box_part64(const double* q, const double* b, uint64_t mask);
+template <>
+__device__ __forceinline__ uint64_t box_part64<3>(const double* q, const double* b, uint64_t mask) {
+  unsigned long long save, m, res = mask;
+  asm volatile(
+      "s_mov_b64 %[save], exec\n\t"
+      "s_mov_b64 exec, %[res]\n\t"
+      "v_cmpx_lt_f64_e64 %[m], %[q0], %[b1]\n\t"
+      "v_cmpx_lt_f64_e64 %[m], %[b0], %[q1]\n\t"
+      "v_cmpx_lt_f64_e64 %[m], %[q2], %[b3]\n\t"
+      "v_cmpx_lt_f64_e64 %[m], %[b2], %[q3]\n\t"
+      "v_cmpx_lt_f64_e64 %[m], %[q4], %[b5]\n\t"
+      "v_cmpx_lt_f64_e64 %[m], %[b4], %[q5]\n\t"
+      "s_nop 4\n\t"
+      "s_mov_b64 %[res], exec\n\t"
+      "s_mov_b64 exec, %[save]\n\t"
+      : [res] "+s"(res), [save] "=&s"(save), [m] "=&s"(m)
+      : [q0] "v"(q[0]), [q1] "v"(q[1]), [q2] "v"(q[2]), [q3] "v"(q[3]), [q4] "v"(q[4]), [q5] "v"(q[5]),
+        [b0] "v"(b[0]), [b1] "v"(b[1]), [b2] "v"(b[2]), [b3] "v"(b[3]), [b4] "v"(b[4]), [b5] "v"(b[5]));
+  return res;
+}
+template <>
+__device__ __forceinline__ uint64_t box_part64<5>(const double* q, const double* b, uint64_t mask) {
+  unsigned long long save, m, res = mask;
+  asm volatile(
+      "s_mov_b64 %[save], exec\n\t"
+      "s_mov_b64 exec, %[res]\n\t"
+      "v_cmpx_lt_f64_e64 %[m], %[q0], %[b1]\n\t"
+      "v_cmpx_lt_f64_e64 %[m], %[b0], %[q1]\n\t"
+      "v_cmpx_lt_f64_e64 %[m], %[q2], %[b3]\n\t"
+      "v_cmpx_lt_f64_e64 %[m], %[b2], %[q3]\n\t"
+      "v_cmpx_lt_f64_e64 %[m], %[q4], %[b5]\n\t"
+      "v_cmpx_lt_f64_e64 %[m], %[b4], %[q5]\n\t"
+      "v_cmpx_lt_f64_e64 %[m], %[q6], %[b7]\n\t"
+      "v_cmpx_lt_f64_e64 %[m], %[b6], %[q7]\n\t"
+      "v_cmpx_lt_f64_e64 %[m], %[q8], %[b9]\n\t"
+      "v_cmpx_lt_f64_e64 %[m], %[b8], %[q9]\n\t"
+      "s_nop 4\n\t"
+      "s_mov_b64 %[res], exec\n\t"
+      "s_mov_b64 exec, %[save]\n\t"
+      : [res] "+s"(res), [save] "=&s"(save), [m] "=&s"(m)
+      : [q0] "v"(q[0]), [q1] "v"(q[1]), [q2] "v"(q[2]), [q3] "v"(q[3]), [q4] "v"(q[4]), [q5] "v"(q[5]), [q6] "v"(q[6]), [q7] "v"(q[7]), [q8] "v"(q[8]), [q9] "v"(q[9]),
+        [b0] "v"(b[0]), [b1] "v"(b[1]), [b2] "v"(b[2]), [b3] "v"(b[3]), [b4] "v"(b[4]), [b5] "v"(b[5]), [b6] "v"(b[6]), [b7] "v"(b[7]), [b8] "v"(b[8]), [b9] "v"(b[9]));
+  return res;
+}
+// Both boxes of an LDS-staged fp64 record against the lane's query slabs.
+// Every second box is missed by all lanes, mostly on x, y or z, so the other
+// axes are read only if these leave a lane; in parts of five axes, so that ten
+// doubles of the record are in registers at a time (92 VGPRs; parts of three or
+// four axes take fewer, 86, but no more waves fit).  With all 13 axes read, and
+// the compares ANDed in scalar registers, the walk of 2 x 524k triangles took
+// 614 us instead of 474, of 2 x 8,192 121 instead of 92.
+__device__ __forceinline__ void overlap_pair(const double* qk, const Rec64& r, uint64_t& m0, uint64_t& m1) {
+  m0 = box_part64<3>(qk, r.box[0], ~0ull);
+  m1 = box_part64<3>(qk, r.box[1], ~0ull);
+  if (m0 != 0) {
+    m0 = box_part64<5>(qk + 6, r.box[0] + 6, m0);
+    if (m0 != 0) m0 = box_part64<5>(qk + 16, r.box[0] + 16, m0);
   }
-  h0 = o0;
-  h1 = o1;
+  if (m1 != 0) {
+    m1 = box_part64<5>(qk + 6, r.box[1] + 6, m1);
+    if (m1 != 0) m1 = box_part64<5>(qk + 16, r.box[1] + 16, m1);
+  }
 }
 
 // fp64 form: the same record walk, K records per memory round trip.  Two
@@ -814,26 +872,35 @@ __device__ __forceinline__ void walk64(const TreeView& q, const TreeView& t, uin
         const Rec64& Rk = R[k];
         const uint32_t cl = uniform(Rk.child[0]), cr = uniform(Rk.child[1]);
         const uint32_t el = uniform(Rk.elem[0]), er = uniform(Rk.elem[1]);
-        bool hl, hr;
-        overlap_pair(qk, Rk, hl, hr);
+        uint64_t ml, mr;
+        overlap_pair(qk, Rk, ml, mr);
+        bool okl = true, okr = true;
         if (SELF) {
           // position bounds (non-short-circuit &: no divergent branch)
-          hl = hl & (xs[k] > p32);  // the left child ends at position x
-          hr = hr & (uniform(Rk.last) > p32);
+          okl = xs[k] > p32;  // the left child ends at position x
+          okr = uniform(Rk.last) > p32;
         }
         if (CROSS) {  // children inside the lane's own patch
           const uint32_t f = uniform(Rk.first), l = uniform(Rk.last);
-          hl = hl & !((f >= pb) & (xs[k] < pe));
-          hr = hr & !((xs[k] + 1 >= pb) & (l < pe));
+          okl = okl & !((f >= pb) & (xs[k] < pe));
+          okr = okr & !((xs[k] + 1 >= pb) & (l < pe));
         }
-        // ballots and readfirstlane values: every branch below is wave-uniform,
+        if (SELF) {
+          ml &= __ballot(okl);
+          mr &= __ballot(okr);
+        }
+        // masks and readfirstlane values: every branch below is wave-uniform,
         // so the stack pointer and counters stay in scalar registers
-        const bool any_l = __ballot(hl) != 0, any_r = __ballot(hr) != 0;
+        const bool any_l = ml != 0, any_r = mr != 0;
         const bool leaf_l = cl >= tleaf0, leaf_r = cr >= tleaf0;
-        if (any_l && leaf_l)
+        if (any_l && leaf_l) {
+          const bool hl = (ml >> lane) & 1;
           wave_emit(buf, fill, out, SELF ? (hl & (cl - tleaf0 > p32)) : hl, pair_key(qa, el, SELF));
-        if (any_r && leaf_r)
+        }
+        if (any_r && leaf_r) {
+          const bool hr = (mr >> lane) & 1;
           wave_emit(buf, fill, out, SELF ? (hr & (cr - tleaf0 > p32)) : hr, pair_key(qa, er, SELF));
+        }
         // the left child ends on top of the stack
         if (sp + 2 > kStack) {
           bad = true;
