@@ -171,6 +171,14 @@ __device__ __forceinline__ uint32_t xcd_tile(uint32_t b, uint32_t nb) {
   return x * per + (x < rem ? x : rem) + j;
 }
 
+// The same, `group` tiles in a row per XCD, in turn: the XCDs then share a part
+// of the order whose tiles take longer (the last nb % (8 * group) tiles as they
+// come).
+__device__ __forceinline__ uint32_t xcd_group_tile(uint32_t b, uint32_t nb, uint32_t group) {
+  const uint32_t turn = 8 * group, g = b / turn, r = b % turn;
+  return (uint64_t)(g + 1) * turn <= nb ? g * turn + (r & 7u) * group + (r >> 3) : b;
+}
+
 // ---- tree records ---------------------------------------------------------------
 // Internal node k (k in [0, n-2]) is the split between sorted positions k and
 // k+1; leaf p is node n-1+p.

@@ -365,8 +365,8 @@ struct BatchQuery {
   uint32_t block0;
   uint32_t blocks;
 };
-// the pair walks of nq queries (no self, no XCD remap) in one launch of
-// `blocks` blocks of 256 threads; bq in device memory; batch 2 or 4 for the
+// the pair walks of nq queries (no self) in one launch of `blocks` blocks of 256
+// threads (the fp32-outward walk: four of one wave each); bq in device memory; batch 2 or 4 for the
 // walk over fp64 records.  The fp32-outward forms leave their re-check
 // lists to launch_recheck_query, one launch per query.
 // a query's ncount counter words, then the two objects' status words (4 x

@@ -249,6 +249,15 @@ __device__ __forceinline__ void recheck_flush(uint64_t* buf, uint32_t& fill, con
   fill = 0;
 }
 
+// Queries in a row per XCD.  One eighth of them for each XCD left some XCDs
+// idle while others still walked: work differs between parts of a scene, and
+// the start of a self walk meets more than its end.  With 1,024 queries in turn
+// the 2 x 2M walk takes 933 us instead of 1,038 (931 / 947 with 4,096 / 16,384 in
+// a row), the 512-mesh walk 1,215 instead of 1,259 (1,256 / 1,310), the 2 x 524k
+// walk over fp64 records 568 instead of 612; tiles that share lines still run on
+// one XCD.
+constexpr uint32_t kXcdQueries = 1024;
+
 // The self walks take CROSS = true for cross-patch self collision: a lane
 // skips every child whose position range lies inside its own patch's range
 // [pb, pe) (patches are contiguous position ranges of the tree order), so
@@ -320,7 +329,7 @@ constexpr int kWalkWhole = 0, kWalkTop = 1, kWalkItems = 2;
 constexpr uint32_t kItemBuf = 32;  // staged items per wave
 constexpr uint32_t kItemBudget = 256;
 constexpr uint32_t kItemLeaves = 64;
-constexpr unsigned kItemBlocks = 1792;  // seven a CU
+constexpr unsigned kItemBlocks = 4 * 1792;  // seven waves a SIMD
 
 // Appends the wave's n staged subtree roots to the split list; returns how
 // many found room (the list is sized by the queries, not by the data: the wave
@@ -602,60 +611,58 @@ __device__ __forceinline__ void walk32(const TreeView& q, const TreeView& t, uin
   }
 }
 
-// The LDS of a block of the walk, per wave (the split walk has items too).
+// One wave per block: a wave's slot is free for the next one as soon as it
+// ends, not when the slowest of its block does (walk of 2 x 2M triangles
+// 1,085 -> 1,040 us, of 512 meshes across patches 1,440 -> 1,260).
 struct Walk32Lds {
-  uint64_t buf[256 / kWave][kWaveBuf];
-  uint64_t rbuf[256 / kWave][kRecheckBuf];
-  uint32_t stack[256 / kWave][kStack];
+  uint64_t buf[kWaveBuf];
+  uint64_t rbuf[kRecheckBuf];
+  uint32_t stack[kStack];
 };
 
 template <bool SELF, bool CROSS, int MODE = kWalkWhole>
-__global__ __launch_bounds__(256) void k_narrow32(TreeView q, TreeView t, int xcd, uint32_t qper, PairOut out,
-                                                  int32_t inner) {
+__global__ __launch_bounds__(kWave) void k_narrow32(TreeView q, TreeView t, int xcd, uint32_t qper, PairOut out,
+                                                    int32_t inner) {
   __shared__ Walk32Lds L;
-  __shared__ uint32_t s_items[256 / kWave][MODE == kWalkTop ? kItemBuf : 1];
-  const uint32_t wv = threadIdx.x / kWave, nw = blockDim.x / kWave;
-  const uint32_t rstripe = (blockIdx.x * nw + wv) % kRecheckStripes;
-  const uint32_t tile = xcd ? xcd_tile(blockIdx.x, gridDim.x) : blockIdx.x;
-  walk32<SELF, CROSS, MODE>(q, t, tile * nw + wv, qper, 0, 0, out, inner, L.buf[wv], L.rbuf[wv], L.stack[wv],
-                            s_items[wv], rstripe);
+  __shared__ uint32_t s_items[MODE == kWalkTop ? kItemBuf : 1];
+  const uint32_t wave = xcd ? xcd_group_tile(blockIdx.x, gridDim.x, kXcdQueries / qper) : blockIdx.x;
+  walk32<SELF, CROSS, MODE>(q, t, wave, qper, 0, 0, out, inner, L.buf, L.rbuf, L.stack, s_items,
+                            blockIdx.x % kRecheckStripes);
 }
 
 // The split list of a query: a contiguous run of items per wave (items of one
 // wave's queries are neighbours, which share the loaded queries).
 template <bool SELF, bool CROSS>
-__global__ __launch_bounds__(256) void k_narrow32_items(TreeView q, TreeView t, uint32_t qper, PairOut out,
-                                                        int32_t inner) {
+__global__ __launch_bounds__(kWave) void k_narrow32_items(TreeView q, TreeView t, uint32_t qper, PairOut out,
+                                                          int32_t inner) {
   __shared__ Walk32Lds L;
-  const uint32_t wv = threadIdx.x / kWave, nw = blockDim.x / kWave;
-  const uint32_t wave = uniform(blockIdx.x * nw + wv);
   const unsigned long long c = *out.icount;
   const uint64_t cnt = c < out.icap ? c : out.icap;
-  const uint64_t per = (cnt + (uint64_t)gridDim.x * nw - 1) / ((uint64_t)gridDim.x * nw);
-  const uint64_t i0 = wave * per, i1 = i0 + per < cnt ? i0 + per : cnt;
+  const uint64_t per = (cnt + gridDim.x - 1) / gridDim.x;
+  const uint64_t i0 = blockIdx.x * per, i1 = i0 + per < cnt ? i0 + per : cnt;
   if (i0 >= i1) return;
-  walk32<SELF, CROSS, kWalkItems>(q, t, 0, qper, i0, i1, out, inner, L.buf[wv], L.rbuf[wv], L.stack[wv], nullptr,
-                                  wave % kRecheckStripes);
+  walk32<SELF, CROSS, kWalkItems>(q, t, 0, qper, i0, i1, out, inner, L.buf, L.rbuf, L.stack, nullptr,
+                                  blockIdx.x % kRecheckStripes);
 }
 
-// Several queries (object pairs) in one launch of the fp32-outward walk:
-// block b walks tile b - block0 of the query whose [block0, block0 +
-// blocks) holds b (a wave-uniform binary search over the table).
-__global__ __launch_bounds__(256) void k_narrow32_batch(const BatchQuery* __restrict__ bq, uint32_t nq,
-                                                        int32_t inner) {
+// Several queries (object pairs) in one launch of the fp32-outward walk: four
+// waves for each of the table's blocks of 256 queries, in the order above;
+// block b belongs to the query whose [block0, block0 + blocks) holds it (a
+// wave-uniform binary search over the table).
+__global__ __launch_bounds__(kWave) void k_narrow32_batch(const BatchQuery* __restrict__ bq, uint32_t nq,
+                                                          int32_t inner) {
   __shared__ Walk32Lds L;
-  const uint32_t wv = threadIdx.x / kWave;
+  const uint32_t tile = xcd_group_tile(blockIdx.x, gridDim.x, kXcdQueries / kWave), b = tile / 4;
   uint32_t lo = 0, hi = nq;
   while (hi - lo > 1) {
     const uint32_t mid = (lo + hi) >> 1;
-    if (bq[mid].block0 <= blockIdx.x) lo = mid;
+    if (bq[mid].block0 <= b) lo = mid;
     else hi = mid;
   }
   const BatchQuery& e = bq[lo];
-  if (blockIdx.x - e.block0 >= e.blocks) return;
-  const uint32_t wave = (blockIdx.x - e.block0) * (256 / kWave) + wv;
-  walk32<false, false, kWalkWhole>(e.q, e.t, wave, kWave, 0, 0, e.out, inner, L.buf[wv], L.rbuf[wv], L.stack[wv],
-                                   nullptr, wave % kRecheckStripes);
+  if (b - e.block0 >= e.blocks) return;
+  walk32<false, false, kWalkWhole>(e.q, e.t, tile - 4 * e.block0, kWave, 0, 0, e.out, inner, L.buf, L.rbuf, L.stack,
+                                   nullptr, blockIdx.x % kRecheckStripes);
 }
 
 // Strict overlap of the lane's query slabs q with one box b whose 26 slabs
@@ -928,7 +935,8 @@ __global__ __launch_bounds__(256) void k_narrow64(TreeView q, TreeView t, int xc
   __shared__ uint32_t s_stack[256 / kWave][kStack];
   __shared__ Rec64 s_rec[256 / kWave][K];
   const uint32_t wv = threadIdx.x / kWave;
-  const uint32_t tile = xcd ? xcd_tile(blockIdx.x, gridDim.x) : blockIdx.x;
+  const uint32_t group = kXcdQueries * kWave / (qper * blockDim.x);
+  const uint32_t tile = xcd ? xcd_group_tile(blockIdx.x, gridDim.x, group) : blockIdx.x;
   walk64<SELF, K, CROSS>(q, t, tile * (blockDim.x / kWave) + wv, qper, out, s_buf[wv], s_stack[wv], s_rec[wv]);
 }
 
@@ -968,7 +976,8 @@ __global__ __launch_bounds__(256) void k_narrow64s(TreeView q, TreeView t, int x
   uint64_t* buf = s_buf[wv];
   uint32_t* stk = s_stack[wv];
   uint32_t fill = 0;
-  const uint32_t tile = xcd ? xcd_tile(blockIdx.x, gridDim.x) : blockIdx.x;
+  const uint32_t group = kXcdQueries * kWave / (qper * blockDim.x);
+  const uint32_t tile = xcd ? xcd_group_tile(blockIdx.x, gridDim.x, group) : blockIdx.x;
   const uint64_t p = ((uint64_t)tile * (blockDim.x / kWave) + wv) * qper + lane_id();
   const bool valid = lane_id() < qper && p < q.n;
   double qk[kSlabs];
@@ -1331,8 +1340,8 @@ hipError_t launch_narrowphase(const TreeView& q, const TreeView& t, int leaf_siz
   if (!q.perm || !t.perm || !t.root || !t.status || !out.pairs || !out.count) return hipErrorInvalidValue;
   if (self == 2 && (!q.patch_of_input || (q.od > 1 && !q.splits))) return hipErrorInvalidValue;
   const uint32_t qper = queries_per_wave(q.n, self);
-  const uint64_t per_block = (uint64_t)(bs / kWave) * qper;
-  const unsigned blocks = (unsigned)((q.n + per_block - 1) / per_block);
+  const unsigned waves = (unsigned)((q.n + qper - 1) / qper), bw = bs / kWave;
+  const unsigned blocks = (waves + bw - 1) / bw;  // of the walks over fp64 records
   const int xcd = shape.xcd_remap ? 1 : 0;
   if (form == kFormFp32 || form == kFormMixed) {
     if (!q.rec32 || !q.rootbox32 || !q.delta || !t.rec32 || !t.rootbox32 || !q.origin || !t.origin)
@@ -1343,14 +1352,15 @@ hipError_t launch_narrowphase(const TreeView& q, const TreeView& t, int leaf_siz
     // applies to the fp64 walk).  Both forms keep the leaf candidates whose
     // fp32 gap proves the fp64 overlap and re-check the rest in fp64.
     const int32_t inner = kInnerUlps;
+    const dim3 g(waves), bl(kWave);
     if (self == 2) {
       if (!out.items || !out.icount) return hipErrorInvalidValue;
-      hipLaunchKernelGGL((k_narrow32<true, true, kWalkTop>), dim3(blocks), dim3(bs), 0, s, q, t, xcd, qper, out, inner);
-      hipLaunchKernelGGL((k_narrow32_items<true, true>), dim3(kItemBlocks), dim3(256), 0, s, q, t, qper, out, inner);
+      hipLaunchKernelGGL((k_narrow32<true, true, kWalkTop>), g, bl, 0, s, q, t, xcd, qper, out, inner);
+      hipLaunchKernelGGL((k_narrow32_items<true, true>), dim3(kItemBlocks), bl, 0, s, q, t, qper, out, inner);
     } else if (self) {
-      hipLaunchKernelGGL((k_narrow32<true, false>), dim3(blocks), dim3(bs), 0, s, q, t, xcd, qper, out, inner);
+      hipLaunchKernelGGL((k_narrow32<true, false>), g, bl, 0, s, q, t, xcd, qper, out, inner);
     } else {
-      hipLaunchKernelGGL((k_narrow32<false, false>), dim3(blocks), dim3(bs), 0, s, q, t, xcd, qper, out, inner);
+      hipLaunchKernelGGL((k_narrow32<false, false>), g, bl, 0, s, q, t, xcd, qper, out, inner);
     }
     // in self mode both keys index the one object (q == t)
     uint64_t per = (out.rcap + 255) / 256;  // blocks per stripe
@@ -1398,7 +1408,7 @@ hipError_t launch_narrowphase_batch(const BatchQuery* bq, uint32_t nq, uint32_t 
                                     hipStream_t s) {
   if (nq == 0 || blocks == 0) return hipSuccess;
   if (form == kFormFp32 || form == kFormMixed) {
-    hipLaunchKernelGGL(k_narrow32_batch, dim3(blocks), dim3(256), 0, s, bq, nq, kInnerUlps);
+    hipLaunchKernelGGL(k_narrow32_batch, dim3(4 * blocks), dim3(kWave), 0, s, bq, nq, kInnerUlps);
   } else if (batch == 4) {
     hipLaunchKernelGGL(k_narrow64_batch<4>, dim3(blocks), dim3(256), 0, s, bq, nq);
   } else {

@@ -433,8 +433,8 @@ bvh_status bvh_unpack_results(bvh_world w, const void *in, uint64_t bytes, uint3
 typedef struct bvh_tuning {
   uint32_t batch;       /* fp64 walk: 1 = one record per visit in scalar registers, 2 (default)
                            or 4 = that many records per memory round trip loaded into LDS */
-  uint32_t block_size;  /* narrowphase threads per block: 64, 128 or 256 */
-  uint32_t xcd_remap;   /* 1: each XCD walks a contiguous range of query tiles */
+  uint32_t block_size;  /* fp64 walk: threads per block, 64, 128 or 256 (the fp32 walk: one wave) */
+  uint32_t xcd_remap;   /* 1: neighbouring queries walk on one XCD, the XCDs take turns */
   uint32_t tried;       /* configurations timed (entries of tried_ms) */
   double ms;            /* best query time */
   double tried_ms[24];  /* in the order batch (1, 2, 4) x block (64, 128, 256) x remap (off, on) */
