@@ -577,14 +577,11 @@ __device__ __forceinline__ uint32_t patch_end(const uint32_t* splits, uint64_t o
 //    whose sibling extends past the chunk leaves its arrival word in global
 //    memory.
 //  * phase k >= 2 (k_tree_up): chunks kTreeChunk times larger; a workgroup
-//    continues the handed-over nodes of its kTreeChunk sub-chunks.  An arrival is one
-//    workgroup-scope atomic exchange on the parent's arrival word: the first
-//    arriver deposits its far end (l for a left child, r for a right child)
-//    and its patch, so the second learns the parent's range and patch from
-//    the exchange itself and reads only the two slab halves.  No other
-//    workgroup touches those words in that launch; earlier launches are
-//    ordered by the kernel boundary.  The last phase is one chunk and finds
-//    the root.
+//    continues the handed-over nodes of its kTreeChunk sub-chunks, counting
+//    this launch's arrivals in LDS and taking an earlier launch's from the
+//    words.  No other workgroup touches those words in that launch; earlier
+//    launches are ordered by the kernel boundary.  The last phase is one
+//    chunk and finds the root.
 //
 // Both forms store one record per internal node with both children's slabs
 // (Rec32 / Rec64).  Each node writes its slabs into its half of the parent's
@@ -695,65 +692,95 @@ __device__ __forceinline__ bool is_patch_root(uint32_t patch, uint32_t l, uint32
 // 612 us per 2M-triangle tree instead of 653 at 256)
 constexpr uint32_t kTreeChunk = kTreeLeafChunk;
 
+// LDS of an upper phase's workgroup: per thread (slot) the node it has
+// deposited at its parent, the node's far end and the delta beyond it; the
+// arrivals, slot + 1, at the boundaries of the sub-chunks and inside them.
+template <bool FP32>
+struct UpLds {
+  SlabT<FP32> slab[2 * kTreeChunk][kSlabs];
+  uint32_t far[2 * kTreeChunk];
+  uint32_t delta[2 * kTreeChunk];
+  uint32_t arrived[2 * kTreeChunk];  // [j]: at the last position of sub-chunk j; [kTreeChunk + j]: inside it
+  FrontNode front[2];
+  uint32_t nfront;
+};
+
+// Word of a node that waits for its sibling from one launch to the next: its
+// far end (n < 2^30) and the delta beyond it; 0 for none.
+__device__ __forceinline__ unsigned long long arrival_word(uint32_t far, uint32_t delta) {
+  return ((unsigned long long)far + 1) << 8 | delta;
+}
+
 // Upper-phase climb (phases >= 2), one thread per handed-over node of the
-// workgroup's chunk [c0, c1).  Node [l, r] of patch `mypatch` with slabs kd
-// (its half of its parent's record is written); dl = delta[l-1] and dr =
-// delta[r] (0 at the ends).  Every arrival deposits the node's slabs, far end
-// and patch in the thread's LDS slot, then exchanges the parent's arrival
-// word for bit 63 | slot: the first arriver stops; the second finds its
-// sibling in that LDS slot, or, for a word left by phase 1 (far end + 1 in
-// the high half, patch in the low half; below 2^62 since n < 2^30), in the
-// sibling's half of the parent's record, written by an earlier launch.  So a
-// level costs one workgroup-scope atomic and LDS latency; record halves are
-// stored for the queries and the next phase, and nothing in this launch
-// waits for those stores.  The climb stops at the root or at a child whose
-// parent splits on the chunk boundary (handed to the next phase).  A first
-// arrival returns its parent in *pend (else kEnd): if its sibling arrives
-// only in a later launch, k_tree_up rewrites the word in the phase-1 format.
+// workgroup's chunk [c0, c1) of sub-chunks of 2^shift positions.  Node [l, r]
+// of patch `mypatch` with slabs kd (its half of its parent's record is
+// written); dl = delta[l-1] and dr = delta[r] (0 at the ends).  What a parent
+// inside a sub-chunk needs is mostly there from an earlier launch: the
+// sibling's word and its half of the parent's record, loaded together.  Else
+// the node is deposited in the thread's LDS slot and the slot exchanged for
+// the parent's arrival: the first arriver stops, the second finds its sibling
+// in that slot.  A sub-chunk has one arrival entry for its last position and
+// one for its inside: a parent inside it neither of whose children lies in it
+// is the split of the largest delta of the sub-chunk, so there is one such.
+// The climb is a chain of dependent accesses, a few dozen levels in a few
+// workgroups: a level costs one memory round trip, or LDS latency at the
+// boundaries (with the arrivals exchanged in memory, the sibling's half loaded
+// after the exchange and the new neighbour's delta after that, three: 66 us a
+// phase instead of 58 over 2M spheres, 54 instead of 46 over 512 meshes, 28
+// instead of 22 over 54,612 hexes).  The
+// patch needs no word: a node lies in one patch if the delta it splits at says so.
+// The climb stops at the root or at a child whose parent splits on the chunk
+// boundary (handed to the next phase).  A first arrival returns its parent in
+// *pend (else kEnd) and its entry in *pidx: if its sibling arrives only in a
+// later launch, k_tree_up leaves the word.
 template <bool FP32>
 __device__ __forceinline__ void climb(const BuildBufs& b, uint64_t n, uint32_t l, uint32_t r, uint32_t mypatch,
                                       uint32_t dl, uint32_t dr, SlabT<FP32>* kd, uint32_t c0, uint32_t c1,
-                                      uint32_t slot, SlabT<FP32> (*s_slab)[kSlabs], uint32_t* s_far,
-                                      uint32_t* s_patch, FrontNode* s_front, uint32_t* s_nfront, uint32_t* pend) {
+                                      uint32_t shift, uint32_t slot, UpLds<FP32>& L, uint32_t* pend, uint32_t* pidx) {
   *pend = kEnd;
+  *pidx = 0;
   RecT<FP32>* recs = recs_of<FP32>(b);
   for (;;) {
     const bool is_left = (l == 0) || (r != n - 1 && dr < dl);
     const uint32_t parent = is_left ? r : l - 1;
     if (parent < c0 || parent + 1 >= c1) {
-      const uint32_t k = atomicAdd(s_nfront, 1u);
-      if (k < 2) s_front[k] = FrontNode{l, r, mypatch, dl | (dr << 8)};
+      const uint32_t k = atomicAdd(&L.nfront, 1u);
+      if (k < 2) L.front[k] = FrontNode{l, r, mypatch, dl | (dr << 8)};
       else atomicOr(b.status, kErrTree);
       return;
     }
-#pragma unroll
-    for (int i = 0; i < kSlabs; ++i) s_slab[slot][i] = kd[i];
-    s_far[slot] = is_left ? l : r;
-    s_patch[slot] = mypatch;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    const unsigned long long old = __hip_atomic_exchange(&b.counters[parent], (1ull << 63) | slot,
-                                                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-    if (old == 0) {  // first arriver: the sibling finishes the parent
-      *pend = parent;
-      return;
-    }
-    uint32_t far, spatch;
+    if ((is_left ? dr : dl) >= 128) mypatch = kMixed;
+    const uint32_t j = (parent - c0) >> shift;
+    const bool inside = (parent + 1 - c0) & ((1u << shift) - 1);
+    uint32_t far, fd;
+    unsigned long long word = 0;
     SlabT<FP32> ks[kSlabs];
-    if (old >> 63) {
-      const uint32_t ss = (uint32_t)old & 0x7fffffffu;
-      if (ss >= 2 * kTreeChunk) {
-        atomicOr(b.status, kErrTree);
+    if (inside) {
+      word = b.counters[parent];
+      rec_load_half<FP32>(b, parent, is_left ? 1 : 0, ks);  // (used only if the word says it is there)
+    }
+    if (word != 0) {
+      far = (uint32_t)(word >> 8) - 1u;
+      fd = (uint32_t)word & 0xffu;
+    } else {
+#pragma unroll
+      for (int i = 0; i < kSlabs; ++i) L.slab[slot][i] = kd[i];
+      L.far[slot] = is_left ? l : r;
+      L.delta[slot] = is_left ? dl : dr;
+      const uint32_t idx = inside ? kTreeChunk + j : j;
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+      const uint32_t old =
+          __hip_atomic_exchange(&L.arrived[idx], slot + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+      if (old == 0) {  // first arriver: the sibling finishes the parent
+        *pend = parent;
+        *pidx = idx;
         return;
       }
-      far = s_far[ss];
-      spatch = s_patch[ss];
+      far = L.far[old - 1];
+      fd = L.delta[old - 1];
 #pragma unroll
-      for (int i = 0; i < kSlabs; ++i) ks[i] = s_slab[ss][i];
-    } else {
-      far = (uint32_t)(old >> 32) - 1u;
-      spatch = (uint32_t)old;
-      rec_load_half<FP32>(b, parent, is_left ? 1 : 0, ks);
+      for (int i = 0; i < kSlabs; ++i) ks[i] = L.slab[old - 1][i];
     }
     // a left child's sibling ends past r, a right child's starts before l
     if (is_left ? (far <= r || far >= n) : (far >= l)) {
@@ -762,13 +789,12 @@ __device__ __forceinline__ void climb(const BuildBufs& b, uint64_t n, uint32_t l
     }
     if (is_left) {
       r = far;
-      dr = (r != n - 1) ? b.delta[r] : 0u;
+      dr = fd;
     } else {
       l = far;
-      dl = l ? b.delta[l - 1] : 0u;
+      dl = fd;
     }
     slab_union(kd, ks);
-    mypatch = (mypatch == spatch) ? mypatch : kMixed;
     rec_set_range(recs[parent], l, r, mypatch);
     if (is_patch_root(mypatch, l, r, n, dl, dr)) {
       b.patch_root[mypatch] = parent;
@@ -898,15 +924,13 @@ __global__ void k_patch_k64_init(unsigned long long* pk64, uint64_t count) {
 // finished node whose range starts at position c0 + j (its slabs, last
 // position, patch); endslot[j] is the slot of the newest finished node that
 // ends at c0 + j.  A parent is written to its first position's slot, so a
-// slot is only overwritten by the thread that has just read it.  far[j] and
-// fpatch[j] are the far end and patch of the first child to arrive at
-// internal node c0 + j.
+// slot is only overwritten by the thread that has just read it.  far[j] is
+// the far end of the first child to arrive at internal node c0 + j.
 template <bool FP32>
 struct ChunkLds {
   SlabT<FP32> slab[kSlabs][kTreeChunk + 1];  // SoA, rows padded: conflict-free stores, and column reads
   uint32_t cnt[kTreeChunk];      // arrivals at internal node c0 + j
   uint32_t far[kTreeChunk];
-  uint32_t fpatch[kTreeChunk];
   uint32_t last[kTreeChunk];
   uint32_t patch[kTreeChunk];
   uint32_t endslot[kTreeChunk];
@@ -955,7 +979,6 @@ __device__ __forceinline__ void climb_chunk(const BuildBufs& b, uint64_t n, uint
       // first arriver: the sibling finishes the parent, in this phase or,
       // through the parent's arrival word, in a later one
       L.far[parent - c0] = is_left ? l : r;
-      L.fpatch[parent - c0] = mypatch;
       return;
     }
     if (old != 1) {
@@ -1072,8 +1095,7 @@ __device__ __forceinline__ void climb_chunk32(const BuildBufs& b, uint64_t n, bo
           // first arriver: the sibling finishes the parent, in this phase or,
           // through the parent's arrival word, in a later one
           L.far[parent - c0] = is_left ? l : r;
-          L.fpatch[parent - c0] = mypatch;
-          alive = false;
+              alive = false;
         } else if (old != 1 || ss >= kTreeChunk) {
           atomicOr(b.status, kErrTree);
           alive = false;
@@ -1337,31 +1359,34 @@ __global__ __launch_bounds__(kTreeChunk) void k_tree_leaves(ElemInput in, BuildB
   else if (act && n > 1) climb_chunk<FP32>(b, n, p, p, pk, c0, c1, L, own);
   __syncthreads();
   // a first arrival whose sibling lies outside the chunk leaves its arrival word
-  if (c0 + t + 1 < c1 && L.cnt[t] == 1)
-    b.counters[c0 + t] = ((unsigned long long)(L.far[t] + 1u) << 32) | L.fpatch[t];
+  if (c0 + t + 1 < c1 && L.cnt[t] == 1) {
+    // (the far end's neighbour: left of a left child's first position, right
+    // of a right child's last)
+    const uint32_t f = L.far[t] - c0;
+    b.counters[c0 + t] = arrival_word(c0 + f, L.delta[f <= t ? f : f + 1]);
+  }
   if (t < 2) b.front_a[2 * chunk + t] = (t < L.nfront) ? L.front[t] : FrontNode{kEnd, kEnd, kEnd, 0u};
 }
 
-// Upper phase: a block of 2 x kTreeChunk threads per chunk of kTreeChunk sub-chunks, one
-// thread per handed-over node (two per sub-chunk).  A handed-over node's
-// slabs are in its half of its parent's record; thread t's LDS slot is t.
+// Upper phase: a block of 2 x kTreeChunk threads per chunk of kTreeChunk
+// sub-chunks of 2^shift positions, one thread per handed-over node (two per
+// sub-chunk).  A handed-over node's slabs are in its half of its parent's
+// record; thread t's LDS slot is t.
 template <bool FP32>
-__global__ __launch_bounds__(2 * kTreeChunk) void k_tree_up(BuildBufs b, uint64_t n, uint64_t chunk, uint64_t nsub,
+__global__ __launch_bounds__(2 * kTreeChunk) void k_tree_up(BuildBufs b, uint64_t n, uint32_t shift, uint64_t nsub,
                                                             const FrontNode* __restrict__ front_in,
                                                             FrontNode* __restrict__ front_out) {
-  __shared__ SlabT<FP32> s_slab[2 * kTreeChunk][kSlabs];
-  __shared__ uint32_t s_far[2 * kTreeChunk];
-  __shared__ uint32_t s_patch[2 * kTreeChunk];
-  __shared__ FrontNode s_front[2];
-  __shared__ uint32_t s_nfront;
+  __shared__ UpLds<FP32> L;
   const uint32_t t = threadIdx.x;
+  const uint64_t chunk = (uint64_t)kTreeChunk << shift;
   const uint64_t c0l = (uint64_t)blockIdx.x * chunk;
   const uint32_t c0 = (uint32_t)c0l;
   const uint32_t c1 = (uint32_t)(c0l + chunk < n ? c0l + chunk : n);
-  if (t == 0) s_nfront = 0;
+  L.arrived[t] = 0;
+  if (t == 0) L.nfront = 0;
   __syncthreads();
   const uint64_t slot = (uint64_t)blockIdx.x * (2 * kTreeChunk) + t;  // = 2 * sub + i
-  uint32_t pend = kEnd;
+  uint32_t pend = kEnd, pidx = 0;
   if (slot < 2 * nsub) {
     const FrontNode f = front_in[slot];
     if (f.l != kEnd) {
@@ -1372,21 +1397,16 @@ __global__ __launch_bounds__(2 * kTreeChunk) void k_tree_up(BuildBufs b, uint64_
         const bool is_left = (f.l == 0) || (f.r != n - 1 && dr < dl);
         SlabT<FP32> kd[kSlabs];
         rec_load_half<FP32>(b, is_left ? f.r : f.l - 1, is_left ? 0 : 1, kd);
-        climb<FP32>(b, n, f.l, f.r, f.patch, dl, dr, kd, c0, c1, t, s_slab, s_far, s_patch, s_front, &s_nfront,
-                    &pend);
+        climb<FP32>(b, n, f.l, f.r, f.patch, dl, dr, kd, c0, c1, shift, t, L, &pend, &pidx);
       }
     }
   }
   __syncthreads();
-  // a first arrival whose deposit is still in the word: its sibling arrives in
-  // a later launch, which needs the far end and patch from the word itself
-  // (the slabs are in the record half)
-  if (pend != kEnd) {
-    const unsigned long long w =
-        __hip_atomic_load(&b.counters[pend], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    if (w == ((1ull << 63) | t)) b.counters[pend] = ((unsigned long long)(s_far[t] + 1u) << 32) | s_patch[t];
-  }
-  if (t < 2) front_out[2 * blockIdx.x + t] = (t < s_nfront) ? s_front[t] : FrontNode{kEnd, kEnd, kEnd, 0u};
+  // a first arrival whose sibling has not come: it arrives in a later launch,
+  // which needs the far end and the delta beyond it (the slabs are in the
+  // record half)
+  if (pend != kEnd && L.arrived[pidx] == t + 1) b.counters[pend] = arrival_word(L.far[t], L.delta[t]);
+  if (t < 2) front_out[2 * blockIdx.x + t] = (t < L.nfront) ? L.front[t] : FrontNode{kEnd, kEnd, kEnd, 0u};
 }
 
 // fp64 form: leaf p's slabs from its parent's record (n x 26, sorted order)
@@ -1630,21 +1650,23 @@ hipError_t launch_tree_leaves(const ElemInput& in, const BuildBufs& b, uint64_t 
 hipError_t launch_tree_up(uint64_t n, const BuildBufs& b, int fp32, hipStream_t s) {
   hipError_t e = hipSuccess;
   // upper phases: chunks kTreeChunk times larger until one chunk holds every leaf
-  uint64_t chunk = kTreeChunk;
+  uint32_t shift = 0;
+  while ((1u << shift) < kTreeChunk) ++shift;
+  const uint32_t step = shift;  // log2 of kTreeChunk
   FrontNode* fin = b.front_a;
   FrontNode* fout = b.front_b;
-  while (chunk < n) {
+  while ((1ull << shift) < n) {
+    const uint64_t chunk = 1ull << shift, next = chunk * kTreeChunk;
     const uint64_t nsub = (n + chunk - 1) / chunk;
-    const uint64_t next = chunk * kTreeChunk;
     const unsigned blocks = (unsigned)((n + next - 1) / next);
-    if (fp32) hipLaunchKernelGGL(k_tree_up<true>, dim3(blocks), dim3(2 * kTreeChunk), 0, s, b, n, next, nsub, fin, fout);
-    else hipLaunchKernelGGL(k_tree_up<false>, dim3(blocks), dim3(2 * kTreeChunk), 0, s, b, n, next, nsub, fin, fout);
+    if (fp32) hipLaunchKernelGGL(k_tree_up<true>, dim3(blocks), dim3(2 * kTreeChunk), 0, s, b, n, shift, nsub, fin, fout);
+    else hipLaunchKernelGGL(k_tree_up<false>, dim3(blocks), dim3(2 * kTreeChunk), 0, s, b, n, shift, nsub, fin, fout);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
     FrontNode* tmp = fin;
     fin = fout;
     fout = tmp;
-    chunk = next;
+    shift += step;
   }
   return hipSuccess;
 }
