@@ -156,7 +156,7 @@ struct bvh_world_s {
   bool capturing = false;
   std::vector<CapturedQuery> captured;
   std::vector<bvh_graph> graphs;  // live graphs captured on this world
-  unsigned long long* h_count = nullptr;  // pinned, 16 words: query counters and status words
+  unsigned long long* h_count = nullptr;  // pinned, 32 words: query counters and status words; a root box
   bool iteration_open = false;
   // allocation generation of this world's buffers (its objects' and its own)
   std::atomic<uint64_t> alloc_gen{0};
@@ -164,6 +164,7 @@ struct bvh_world_s {
   DevBuf bq_dev;
   BatchQuery* bq_host = nullptr;
   size_t bq_host_cap = 0;
+  bool bq_busy = false;  // the table may still be on its way to the device
 
   // Only buffers that captured work can reference count on the world's
   // generation (its objects' buffers).  The stand-alone primitives' and the
@@ -903,7 +904,7 @@ static bvh_status read_counts(bvh_object_s* o, bvh_object_s* other, bool* overfl
   bvh_world w = o->w;
   hipStream_t s = w->stream;
   const unsigned long long* dcount = o->count.as<unsigned long long>();
-  HIP_TRY(launch_readback(dcount, kCntWords, o->status.as<uint32_t>(), other->status.as<uint32_t>(), w->h_count, s));
+  HIP_TRY(launch_readback(dcount, kCntWords, o->status.p, 2, other->status.p, 2, w->h_count, s));
   HIP_TRY(hipStreamSynchronize(s));
   o->npairs = o->q_narrow ? w->h_count[kCntPairs] : 0;
   o->nvisits = w->h_count[kCntVisits];
@@ -1117,18 +1118,20 @@ static bvh_status run_query_batch(bvh_object_s* const* os, bvh_object_s* const* 
     BVH_TRY(ensure_pairs(o, std::max<uint64_t>(1u << 20, 8 * o->in.n)));
     BVH_TRY(first_query_lists(o));
   }
+  // (a batch ends synchronized, unless it failed)
+  if (w->bq_busy) HIP_TRY(hipStreamSynchronize(s));
+  w->bq_busy = false;
   if (k > w->bq_host_cap) {
     if (w->bq_host) (void)hipHostFree(w->bq_host);
     w->bq_host = nullptr;
     w->bq_host_cap = 0;
-    void* hp = nullptr;
-    HIP_TRY(hipHostMalloc(&hp, k * sizeof(BatchQuery), hipHostMallocDefault));
+    void* hp = nullptr;  // the table, then kReadbackWords words for each query
+    HIP_TRY(hipHostMalloc(&hp, k * (sizeof(BatchQuery) + kReadbackWords * sizeof(unsigned long long)),
+                          hipHostMallocDefault));
     w->bq_host = static_cast<BatchQuery*>(hp);
     w->bq_host_cap = k;
   }
   BVH_TRY(w->bq_dev.ensure(k * sizeof(BatchQuery)));
-  // the previous batch's table may still be in flight to the device
-  HIP_TRY(hipStreamSynchronize(s));
   uint32_t blocks = 0;
   uint32_t nq = 0;
   for (uint64_t i = 0; i < k; ++i) {
@@ -1144,13 +1147,10 @@ static bvh_status run_query_batch(bvh_object_s* const* os, bvh_object_s* const* 
     o->result_ptr = o->pairs.as<uint64_t>();
     o->result_other = t;
     o->self_result = false;
-    HIP_TRY(launch_fill_u32((uint32_t*)dcount, 2 * kCntTotal, 0u, s));
-    const TreeView qv = view_of(o), tv = view_of(t);
     o->patch_pairs_ready = false;  // computed when asked for (ensure_patch_pairs)
-    if (o->in.n == 0 || t->in.n == 0) continue;
     BatchQuery& e = w->bq_host[nq++];
-    e.q = qv;
-    e.t = tv;
+    e.q = view_of(o);
+    e.t = view_of(t);
     e.out = PairOut{o->pairs.as<uint64_t>(), o->q_cap, dcount + kCntPairs, dcount + kCntVisits, dcount + kCntCand,
                     nullptr, 0, nullptr, nullptr, nullptr, 0, nullptr};
     if (o->fp32) {
@@ -1160,12 +1160,16 @@ static bvh_status run_query_batch(bvh_object_s* const* os, bvh_object_s* const* 
       e.out.rtotal = dcount + kCntRecheck;
     }
     e.block0 = blocks;
-    e.blocks = (uint32_t)((o->in.n + 255) / 256);
+    e.blocks = t->in.n ? (uint32_t)((o->in.n + 255) / 256) : 0;  // none: nothing to walk
     blocks += e.blocks;
   }
-  if (nq) {
+  unsigned long long* const h = (unsigned long long*)(w->bq_host + w->bq_host_cap);
+  {
     w->stage_begin("narrowphase_batch");
+    w->bq_busy = true;
     HIP_TRY(hipMemcpyAsync(w->bq_dev.p, w->bq_host, nq * sizeof(BatchQuery), hipMemcpyHostToDevice, s));
+    for (uint32_t j = 0; j < nq; j += 65535)  // (the grid's second dimension)
+      HIP_TRY(launch_batch_clear(w->bq_dev.as<BatchQuery>() + j, std::min<uint32_t>(nq - j, 65535), (uint32_t)kCntTotal, s));
     HIP_TRY(launch_narrowphase_batch(w->bq_dev.as<BatchQuery>(), nq, blocks, w->shape.batch == 4 ? 4 : 2,
                                      os[0]->form, s));
     // the fp32-outward forms: each query's re-check list, decided in fp64
@@ -1174,17 +1178,12 @@ static bvh_status run_query_batch(bvh_object_s* const* os, bvh_object_s* const* 
     w->stage_end();
   }
   // every pair's counters and both objects' error words, one synchronization
-  std::vector<unsigned long long> h(12 * k);
-  for (uint64_t i = 0; i < k; ++i) {
-    HIP_TRY(hipMemcpyAsync(&h[12 * i], os[i]->count.p, kCntWords * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipMemcpyAsync(&h[12 * i + kCntWords], os[i]->status.p, 4 * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipMemcpyAsync(&h[12 * i + kCntWords + 2], others[i]->status.p, 4 * sizeof(uint32_t),
-                           hipMemcpyDeviceToHost, s));
-  }
+  HIP_TRY(launch_batch_readback(w->bq_dev.as<BatchQuery>(), nq, kCntWords, h, s));
   HIP_TRY(hipStreamSynchronize(s));
+  w->bq_busy = false;
   for (uint64_t i = 0; i < k; ++i) {
     bvh_object_s* o = os[i];
-    const unsigned long long* c = &h[12 * i];
+    const unsigned long long* c = h + kReadbackWords * i;
     o->npairs = c[kCntPairs];
     o->nvisits = c[kCntVisits];
     o->ncandidates = c[kCntCand];
@@ -1404,7 +1403,7 @@ bvh_status bvh_world_create(size_t od, const bvh_world_config* cfg, bvh_world* o
   }
   BVH_TRY(noalloc_setup_current());  // the device address of bvh_sort_u64_noalloc's scratch
   void* hc = nullptr;
-  HIP_TRY(hipHostMalloc(&hc, 16 * sizeof(unsigned long long), hipHostMallocDefault));
+  HIP_TRY(hipHostMalloc(&hc, 32 * sizeof(unsigned long long), hipHostMallocDefault));
   w->h_count = (unsigned long long*)hc;
   *out = w.release();
   return BVH_OK;
@@ -1580,15 +1579,20 @@ bvh_status bvh_object_root_kdop(bvh_object o, double* kdop) {
   for (int i = 0; i < 26; ++i) kdop[i] = (i & 1) ? -1.7976931348623157e308 : 1.7976931348623157e308;
   if (o->in.n == 0) return BVH_OK;
   hipStream_t s = o->w->stream;
+  // 26 slabs and, in fp32, the frame they are in
+  if (o->fp32) HIP_TRY(launch_readback(o->rootbox32.p, kSlabs / 2, o->frame.p, 3, nullptr, 0, o->w->h_count, s));
+  else HIP_TRY(launch_readback(o->rootbox64.p, kSlabs, nullptr, 0, nullptr, 0, o->w->h_count, s));
+  HIP_TRY(hipStreamSynchronize(s));
   if (o->fp32) {
     int32_t ko[kSlabs];
     double org[3];
-    BVH_TRY(copy_out(ko, o->rootbox32.p, sizeof(ko), BVH_MEM_HOST, s));
-    BVH_TRY(copy_out(org, o->frame.p, sizeof(org), BVH_MEM_HOST, s));
+    std::memcpy(ko, o->w->h_count, sizeof(ko));
+    std::memcpy(org, o->w->h_count + kSlabs / 2, sizeof(org));
     decode_box32(ko, org, kdop);
-    return BVH_OK;
+  } else {
+    std::memcpy(kdop, o->w->h_count, kSlabs * sizeof(double));
   }
-  return copy_out(kdop, o->rootbox64.p, 26 * sizeof(double), BVH_MEM_HOST, s);
+  return BVH_OK;
 }
 
 bvh_status bvh_object_overdecomposition(bvh_object o, size_t* od) {

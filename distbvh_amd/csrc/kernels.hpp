@@ -369,10 +369,17 @@ struct BatchQuery {
 // threads (the fp32-outward walk: four of one wave each); bq in device memory; batch 2 or 4 for the
 // walk over fp64 records.  The fp32-outward forms leave their re-check
 // lists to launch_recheck_query, one launch per query.
-// a query's ncount counter words, then the two objects' status words (4 x
-// u32 each, 8-byte aligned), into host (pinned, device-accessible) memory
-hipError_t launch_readback(const unsigned long long* count, int ncount, const uint32_t* st_a, const uint32_t* st_b,
+// na, nb and nc 8-byte words of device memory (at most 64, 8-byte aligned), one
+// run after the other, into host (pinned, device-accessible) memory
+hipError_t launch_readback(const void* a, int na, const void* b, int nb, const void* c, int nc,
                            unsigned long long* host, hipStream_t s);
+// every query's first `words` words from out.count on set to zero
+hipError_t launch_batch_clear(const BatchQuery* bq, uint32_t nq, uint32_t words, hipStream_t s);
+// every query's ncount counter words, then its two objects' status words (4 x
+// u32 each), at host + kReadbackWords * query
+constexpr uint32_t kReadbackWords = 16;
+hipError_t launch_batch_readback(const BatchQuery* bq, uint32_t nq, int ncount, unsigned long long* host,
+                                 hipStream_t s);
 hipError_t launch_narrowphase_batch(const BatchQuery* bq, uint32_t nq, uint32_t blocks, int batch, int form,
                                     hipStream_t s);
 hipError_t launch_recheck_query(const TreeView& q, const TreeView& t, const PairOut& out, hipStream_t s);

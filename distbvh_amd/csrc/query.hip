@@ -1383,24 +1383,58 @@ hipError_t launch_narrowphase(const TreeView& q, const TreeView& t, int leaf_siz
   return hipGetLastError();
 }
 
-// The counters of a query and both objects' status words (4 x u32 each) in
-// one launch, straight into pinned host memory: one small kernel instead of
-// three device-to-host copies.
-__global__ void k_readback(const unsigned long long* __restrict__ count, int ncount,
-                           const unsigned long long* __restrict__ st_a, const unsigned long long* __restrict__ st_b,
+// Three short runs of 8-byte words (a query's counters and both objects' status
+// words, a root box and its frame) in one launch, straight into pinned host
+// memory: one small kernel instead of a device-to-host copy for each.
+__global__ void k_readback(const unsigned long long* __restrict__ a, int na, const unsigned long long* __restrict__ b,
+                           int nb, const unsigned long long* __restrict__ c, int nc,
                            unsigned long long* __restrict__ host) {
   const int i = (int)threadIdx.x;
-  if (i < ncount) host[i] = count[i];
-  else if (i < ncount + 2) host[i] = st_a[i - ncount];
-  else if (i < ncount + 4) host[i] = st_b[i - ncount - 2];
+  if (i < na) host[i] = a[i];
+  else if (i < na + nb) host[i] = b[i - na];
+  else if (i < na + nb + nc) host[i] = c[i - na - nb];
   __threadfence_system();  // the words are in host memory before the kernel ends
 }
 
-hipError_t launch_readback(const unsigned long long* count, int ncount, const uint32_t* st_a, const uint32_t* st_b,
+hipError_t launch_readback(const void* a, int na, const void* b, int nb, const void* c, int nc,
                            unsigned long long* host, hipStream_t s) {
-  if (ncount < 0 || ncount + 4 > 64) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_readback, dim3(1), dim3(64), 0, s, count, ncount, (const unsigned long long*)st_a,
-                     (const unsigned long long*)st_b, host);
+  if (na < 0 || nb < 0 || nc < 0 || na + nb + nc > 64) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_readback, dim3(1), dim3(64), 0, s, (const unsigned long long*)a, na,
+                     (const unsigned long long*)b, nb, (const unsigned long long*)c, nc, host);
+  return hipGetLastError();
+}
+
+// A batch's counters, `words` of each query, set to zero (a block row per query).
+__global__ __launch_bounds__(256) void k_batch_clear(const BatchQuery* __restrict__ bq, uint32_t words) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i < words) bq[blockIdx.y].out.count[i] = 0;
+}
+
+// The first ncount counters of every query of a batch and its objects' status
+// words, kReadbackWords words each, into pinned host memory: one launch and one
+// synchronization, where three copies for each query took 30 us apiece.
+__global__ void k_batch_readback(const BatchQuery* __restrict__ bq, int ncount, unsigned long long* __restrict__ host) {
+  const BatchQuery& e = bq[blockIdx.x];
+  const int i = (int)threadIdx.x;
+  unsigned long long* h = host + (uint64_t)blockIdx.x * kReadbackWords;
+  if (i < ncount) h[i] = e.out.count[i];
+  else if (i < ncount + 2) h[i] = ((const unsigned long long*)e.q.status)[i - ncount];
+  else if (i < ncount + 4) h[i] = ((const unsigned long long*)e.t.status)[i - ncount - 2];
+  __threadfence_system();  // the words are in host memory before the kernel ends
+}
+
+hipError_t launch_batch_clear(const BatchQuery* bq, uint32_t nq, uint32_t words, hipStream_t s) {
+  if (nq == 0 || words == 0) return hipSuccess;
+  if (nq > 65535) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_batch_clear, dim3((words + 255) / 256, nq), dim3(256), 0, s, bq, words);
+  return hipGetLastError();
+}
+
+hipError_t launch_batch_readback(const BatchQuery* bq, uint32_t nq, int ncount, unsigned long long* host,
+                                 hipStream_t s) {
+  if (nq == 0) return hipSuccess;
+  if (ncount < 0 || (uint32_t)ncount + 4 > kReadbackWords) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_batch_readback, dim3(nq), dim3(64), 0, s, bq, ncount, host);
   return hipGetLastError();
 }
 

@@ -64,3 +64,36 @@ def test_cross_patch_uneven(na, nb, every, precision):
         got = sort_pairs(o.pairs())
     want = np.stack([np.repeat(np.sort(big), nb), np.tile(np.arange(na, na + nb), len(big))], axis=1)
     assert np.array_equal(got.astype(np.int64), want)
+
+
+@pytest.mark.parametrize("precision", FORMS)
+def test_batch_with_empty_objects(precision):
+    """Batches of growing and shrinking sizes with objects of no element as
+    query and as tree, first, between and last: every pair's results, and the
+    root boxes of the objects."""
+    sizes = [0, 1, 300, 0, 257, 64, 0]
+    rng = np.random.default_rng(5)
+    data = [(_spheres(max(1, n), rng)[:, :n], _spheres(200, rng)[:, :(0 if n == 64 else 200)])
+            for n in sizes]
+    with CollisionWorld(4, precision=precision) as w:
+        objs = []
+        for a, b in data:
+            pair = []
+            for d in (a, b):
+                o = w.create_collision_object()
+                o.set_entity_data_sphere(to_cuda(np.ascontiguousarray(d)))
+                o.init_broadphase()
+                pair.append(o)
+            objs.append(pair)
+        for take in ([0], [2, 4], [0, 1, 2, 3, 4, 5, 6], [6, 2, 0], [3, 5]):
+            w.broadphase_batch([objs[i][0] for i in take], [objs[i][1] for i in take])
+            for i in take:
+                (ka, _), (kb, _) = O.elements_sphere(data[i][0]), O.elements_sphere(data[i][1])
+                want = sort_pairs(O.brute_pairs(ka, kb)) if len(ka) and len(kb) else np.zeros((0, 2), np.uint64)
+                assert np.array_equal(sort_pairs(objs[i][0].pairs()), want), (take, i)
+        for (a, _), (o, _) in zip(data, objs):
+            if a.shape[1]:
+                k = O.elements_sphere(a)[0].reshape(-1, 13, 2)
+                root = np.asarray(o.root_kdop()).reshape(13, 2)
+                assert np.allclose(root[:, 0], k[:, :, 0].min(0), atol=1e-6) and (root[:, 0] <= k[:, :, 0].min(0)).all()
+                assert np.allclose(root[:, 1], k[:, :, 1].max(0), atol=1e-6) and (root[:, 1] >= k[:, :, 1].max(0)).all()
