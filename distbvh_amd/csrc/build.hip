@@ -920,34 +920,61 @@ __global__ void k_patch_k64_init(unsigned long long* pk64, uint64_t count) {
   if (i < count) pk64[i] = (i & 1) ? 0ull : ~0ull;
 }
 
-// Phase-1 state of one chunk of kTreeChunk leaves, all in LDS.  Slot j holds the newest
-// finished node whose range starts at position c0 + j (its slabs, last
-// position, patch); endslot[j] is the slot of the newest finished node that
-// ends at c0 + j.  A parent is written to its first position's slot, so a
-// slot is only overwritten by the thread that has just read it.  far[j] is
-// the far end of the first child to arrive at internal node c0 + j.
+// Phase-1 state of one chunk of kTreeChunk leaves, all in LDS.  Slot j holds the slabs
+// of the newest finished node whose range starts at position c0 + j: a parent is
+// written to its first position's slot, which only the thread that has just read
+// it overwrites.  far[j] is the far end of the first child to arrive at internal
+// node c0 + j, plus one (0: none yet).  What else a sibling needs to know follows
+// from it, so the slabs are most of this: 14.6 KB (fp32), 11 chunks a CU.
 template <bool FP32>
 struct ChunkLds {
   SlabT<FP32> slab[kSlabs][kTreeChunk + 1];  // SoA, rows padded: conflict-free stores, and column reads
-  uint32_t cnt[kTreeChunk];      // arrivals at internal node c0 + j
   uint32_t far[kTreeChunk];
-  uint32_t last[kTreeChunk];
-  uint32_t patch[kTreeChunk];
-  uint32_t endslot[kTreeChunk];
   uint8_t delta[kTreeChunk + 1];  // delta[c0 - 1 + j]
+  uint8_t order[kTreeChunk];      // fp32 climb: per wave, the lanes that formed a node at this level
   FrontNode front[2];
   uint32_t nfront;
-  uint32_t order[kTreeChunk];  // fp32 climb: per wave, the lanes that formed a node at this level
 };
 
 template <bool FP32>
-__device__ __forceinline__ void publish(ChunkLds<FP32>& L, uint32_t slot, uint32_t endslot, const SlabT<FP32>* kd,
-                                        uint32_t last, uint32_t patch) {
+__device__ __forceinline__ void publish(ChunkLds<FP32>& L, uint32_t slot, const SlabT<FP32>* kd) {
 #pragma unroll
   for (int i = 0; i < kSlabs; ++i) L.slab[i][slot] = kd[i];
-  L.last[slot] = last;
-  L.patch[slot] = patch;
-  L.endslot[endslot] = slot;
+}
+
+// One step of the phase-1 climb of node [l, r] inside the chunk [c0, c1): its
+// arrival at its parent.  Returns the sibling's slot when the sibling was there
+// (far is then the parent's other end), else kEnd: handed to the next phase,
+// first to arrive (its sibling finishes the parent, in this phase or, through
+// the parent's arrival word, in a later one), or an error.
+template <bool FP32>
+__device__ __forceinline__ uint32_t arrive(const BuildBufs& b, uint64_t n, uint32_t l, uint32_t r, uint32_t mypatch,
+                                           uint32_t c0, uint32_t c1, ChunkLds<FP32>& L, uint32_t& parent,
+                                           bool& is_left, uint32_t& far) {
+  // delta[l - 1] = L.delta[l - c0], delta[r] = L.delta[r - c0 + 1] (0 at the ends)
+  const uint32_t dl = L.delta[l - c0], dr = L.delta[r - c0 + 1];
+  is_left = (l == 0) || (r != n - 1 && dr < dl);
+  parent = is_left ? r : l - 1;
+  if (parent < c0 || parent + 1 >= c1) {
+    const uint32_t k = atomicAdd(&L.nfront, 1u);
+    if (k < 2) L.front[k] = FrontNode{l, r, mypatch, dl | (dr << 8)};
+    else atomicOr(b.status, kErrTree);
+    return kEnd;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  const uint32_t old = __hip_atomic_exchange(&L.far[parent - c0], (is_left ? l : r) + 1u, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_WORKGROUP);
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  if (old == 0) return kEnd;
+  far = old - 1;
+  // a left child's sibling starts at r + 1 and ends past r, a right child's
+  // starts before l
+  if (is_left ? (far <= r || far >= c1) : (far >= l || far < c0)) {
+    atomicOr(b.status, kErrTree);
+    return kEnd;
+  }
+  L.far[parent - c0] = 0;  // both have arrived
+  return (is_left ? r + 1 : far) - c0;
 }
 
 // Phase-1 climb inside the chunk [c0, c1) from node [l, r] of patch
@@ -957,70 +984,40 @@ __device__ __forceinline__ void publish(ChunkLds<FP32>& L, uint32_t slot, uint32
 // from the two children's LDS slots, so no slabs are carried from one level
 // to the next (which keeps the register count down); record halves go to
 // global memory with stores that nothing in this kernel waits for.
-template <bool FP32>
-__device__ __forceinline__ void climb_chunk(const BuildBufs& b, uint64_t n, uint32_t l, uint32_t r, uint32_t mypatch,
-                                            uint32_t c0, uint32_t c1, ChunkLds<FP32>& L, SlabT<FP32>* own) {
-  RecT<FP32>* recs = recs_of<FP32>(b);
+__device__ __forceinline__ void climb_chunk64(const BuildBufs& b, uint64_t n, uint32_t l, uint32_t r, uint32_t mypatch,
+                                              uint32_t c0, uint32_t c1, ChunkLds<false>& L) {
+  Rec64* recs = b.rec64;
   for (;;) {
-    // delta[l - 1] = L.delta[l - c0], delta[r] = L.delta[r - c0 + 1] (0 at the ends)
-    const uint32_t dl = L.delta[l - c0], dr = L.delta[r - c0 + 1];
-    const bool is_left = (l == 0) || (r != n - 1 && dr < dl);
-    const uint32_t parent = is_left ? r : l - 1;
-    if (parent < c0 || parent + 1 >= c1) {
-      const uint32_t k = atomicAdd(&L.nfront, 1u);
-      if (k < 2) L.front[k] = FrontNode{l, r, mypatch, dl | (dr << 8)};
-      else atomicOr(b.status, kErrTree);
-      return;
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    const uint32_t old = __hip_atomic_fetch_add(&L.cnt[parent - c0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-    if (old == 0) {
-      // first arriver: the sibling finishes the parent, in this phase or,
-      // through the parent's arrival word, in a later one
-      L.far[parent - c0] = is_left ? l : r;
-      return;
-    }
-    if (old != 1) {
-      atomicOr(b.status, kErrTree);
-      return;
-    }
-    // the sibling starts at r + 1 (left child) or ends at l - 1 (right child)
-    const uint32_t ss = is_left ? (r + 1 - c0) : L.endslot[l - 1 - c0];
-    if (ss >= kTreeChunk) {
-      atomicOr(b.status, kErrTree);
-      return;
-    }
+    uint32_t parent, far;
+    bool is_left;
+    const uint32_t ss = arrive<false>(b, n, l, r, mypatch, c0, c1, L, parent, is_left, far);
+    if (ss == kEnd) return;
     const uint32_t ms = l - c0;
-    const uint32_t slast = L.last[ss], spatch = L.patch[ss];
-    // fp32 slabs (32-bit images) stay in registers from one level to the
-    // next; the fp64 ones are read back from the node's own slot
-    SlabT<FP32> kdl[FP32 ? 1 : kSlabs];
-    SlabT<FP32>* kd = FP32 ? own : kdl;
+    double kd[kSlabs];
 #pragma unroll
     for (int a = 0; a < kAxes; ++a) {
-      const SlabT<FP32> lo0 = FP32 ? own[2 * a] : L.slab[2 * a][ms], lo1 = L.slab[2 * a][ss];
-      const SlabT<FP32> hi0 = FP32 ? own[2 * a + 1] : L.slab[2 * a + 1][ms], hi1 = L.slab[2 * a + 1][ss];
+      const double lo0 = L.slab[2 * a][ms], lo1 = L.slab[2 * a][ss];
+      const double hi0 = L.slab[2 * a + 1][ms], hi1 = L.slab[2 * a + 1][ss];
       kd[2 * a] = (lo0 < lo1) ? lo0 : lo1;
       kd[2 * a + 1] = (hi0 > hi1) ? hi0 : hi1;
     }
-    if (is_left) r = slast;
-    else l = c0 + ss;
-    mypatch = (mypatch == spatch) ? mypatch : kMixed;
+    if (L.delta[parent - c0 + 1] >= 128) mypatch = kMixed;
+    if (is_left) r = far;
+    else l = far;
     rec_set_range(recs[parent], l, r, mypatch);
     const uint32_t ndl = L.delta[l - c0], ndr = L.delta[r - c0 + 1];
     if (is_patch_root(mypatch, l, r, n, ndl, ndr)) {
       b.patch_root[mypatch] = parent;
-      store_patch_box<FP32>(b, mypatch, kd);
+      store_patch_box<false>(b, mypatch, kd);
     }
     if (l == 0 && r == n - 1) {
       *b.root = parent;
-      store_rootbox<FP32>(b, kd);
+      store_rootbox<false>(b, kd);
       return;
     }
     const bool up_left = (l == 0) || (r != n - 1 && ndr < ndl);
-    rec_store_half<FP32>(b, up_left ? r : l - 1, up_left ? 0 : 1, kd, parent, kEnd);
-    publish<FP32>(L, l - c0, r - c0, kd, r, mypatch);
+    rec_store_half<false>(b, up_left ? r : l - 1, up_left ? 0 : 1, kd, parent, kEnd);
+    publish<false>(L, l - c0, kd);
   }
 }
 
@@ -1035,12 +1032,12 @@ __device__ __forceinline__ void climb_chunk(const BuildBufs& b, uint64_t n, uint
 // than one piece of up to 64 scattered nodes.  Called by all lanes of the
 // wave, after the forming lanes published their slabs in their LDS slots.
 __device__ __forceinline__ void store_level32(const BuildBufs& b, ChunkLds<true>& L, uint32_t c0, uint32_t node,
-                                              uint32_t half, uint32_t sl) {
+                                              uint32_t half, uint32_t sl, uint32_t last, uint32_t patch) {
   const uint64_t mask = __ballot(node != kEnd);
   if (mask == 0) return;
   int4* base = (int4*)b.rec32;
   const uint32_t lane = lane_id(), w0 = threadIdx.x - lane;
-  if (node != kEnd) L.order[w0 + (uint32_t)__popcll(mask & lanemask_lt())] = lane;
+  if (node != kEnd) L.order[w0 + (uint32_t)__popcll(mask & lanemask_lt())] = (uint8_t)lane;
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
@@ -1052,9 +1049,10 @@ __device__ __forceinline__ void store_level32(const BuildBufs& b, ChunkLds<true>
     const uint32_t nd = (uint32_t)__shfl((int)node, src, kWave);
     const uint32_t hf = (uint32_t)__shfl((int)half, src, kWave);
     const uint32_t s = (uint32_t)__shfl((int)sl, src, kWave);
+    const int32_t la = __shfl((int)last, src, kWave), pa = __shfl((int)patch, src, kWave);
     if (k >= pieces) continue;
     if (q == 7) {  // this node's range and patch (its record's half 0)
-      base[(uint64_t)nd * 16u + 7u] = make_int4((int32_t)(c0 + s), (int32_t)L.last[s], (int32_t)L.patch[s], 0);
+      base[(uint64_t)nd * 16u + 7u] = make_int4((int32_t)(c0 + s), la, pa, 0);
     } else if (hf != kEnd) {
       // piece q of the half: slabs 4q .. 4q+3; piece 6: slabs 24, 25, node, no element
       const uint32_t r0 = 4u * q;
@@ -1062,6 +1060,7 @@ __device__ __forceinline__ void store_level32(const BuildBufs& b, ChunkLds<true>
       const int32_t z = q < 6 ? L.slab[q < 6 ? r0 + 2 : 0][s] : (int32_t)nd;
       const int32_t w = q < 6 ? L.slab[q < 6 ? r0 + 3 : 0][s] : (int32_t)kEnd;
       base[(uint64_t)hf * 8u + q] = make_int4(x, y, z, w);
+      if (q == 6 && (hf & 1u)) base[(uint64_t)hf * 8u + 7u] = make_int4(0, 0, 0, 0);  // (whole sectors)
     }
   }
 }
@@ -1076,59 +1075,39 @@ __device__ __forceinline__ void climb_chunk32(const BuildBufs& b, uint64_t n, bo
   while (__ballot(alive) != 0) {
     uint32_t node = kEnd, half = kEnd;
     if (alive) {
-      const uint32_t dl = L.delta[l - c0], dr = L.delta[r - c0 + 1];
-      const bool is_left = (l == 0) || (r != n - 1 && dr < dl);
-      const uint32_t parent = is_left ? r : l - 1;
-      if (parent < c0 || parent + 1 >= c1) {
-        const uint32_t k = atomicAdd(&L.nfront, 1u);
-        if (k < 2) L.front[k] = FrontNode{l, r, mypatch, dl | (dr << 8)};
-        else atomicOr(b.status, kErrTree);
+      uint32_t parent, far;
+      bool is_left;
+      const uint32_t ss = arrive<true>(b, n, l, r, mypatch, c0, c1, L, parent, is_left, far);
+      if (ss == kEnd) {
         alive = false;
       } else {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-        const uint32_t old =
-            __hip_atomic_fetch_add(&L.cnt[parent - c0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-        // the sibling starts at r + 1 (left child) or ends at l - 1 (right child)
-        const uint32_t ss = (old == 1) ? (is_left ? (r + 1 - c0) : L.endslot[l - 1 - c0]) : 0u;
-        if (old == 0) {
-          // first arriver: the sibling finishes the parent, in this phase or,
-          // through the parent's arrival word, in a later one
-          L.far[parent - c0] = is_left ? l : r;
-              alive = false;
-        } else if (old != 1 || ss >= kTreeChunk) {
-          atomicOr(b.status, kErrTree);
+#pragma unroll
+        for (int a = 0; a < kAxes; ++a) {
+          const int32_t lo1 = L.slab[2 * a][ss], hi1 = L.slab[2 * a + 1][ss];
+          own[2 * a] = (own[2 * a] < lo1) ? own[2 * a] : lo1;
+          own[2 * a + 1] = (own[2 * a + 1] > hi1) ? own[2 * a + 1] : hi1;
+        }
+        if (L.delta[parent - c0 + 1] >= 128) mypatch = kMixed;
+        if (is_left) r = far;
+        else l = far;
+        const uint32_t ndl = L.delta[l - c0], ndr = L.delta[r - c0 + 1];
+        if (is_patch_root(mypatch, l, r, n, ndl, ndr)) {
+          b.patch_root[mypatch] = parent;
+          store_patch_box<true>(b, mypatch, own);
+        }
+        node = parent;
+        if (l == 0 && r == n - 1) {
+          *b.root = parent;
+          store_rootbox<true>(b, own);
           alive = false;
         } else {
-          const uint32_t slast = L.last[ss], spatch = L.patch[ss];
-#pragma unroll
-          for (int a = 0; a < kAxes; ++a) {
-            const int32_t lo1 = L.slab[2 * a][ss], hi1 = L.slab[2 * a + 1][ss];
-            own[2 * a] = (own[2 * a] < lo1) ? own[2 * a] : lo1;
-            own[2 * a + 1] = (own[2 * a + 1] > hi1) ? own[2 * a + 1] : hi1;
-          }
-          if (is_left) r = slast;
-          else l = c0 + ss;
-          mypatch = (mypatch == spatch) ? mypatch : kMixed;
-          const uint32_t ndl = L.delta[l - c0], ndr = L.delta[r - c0 + 1];
-          if (is_patch_root(mypatch, l, r, n, ndl, ndr)) {
-            b.patch_root[mypatch] = parent;
-            store_patch_box<true>(b, mypatch, own);
-          }
-          node = parent;
-          if (l == 0 && r == n - 1) {
-            *b.root = parent;
-            store_rootbox<true>(b, own);
-            alive = false;
-          } else {
-            const bool up_left = (l == 0) || (r != n - 1 && ndr < ndl);
-            half = 2u * (up_left ? r : l - 1) + (up_left ? 0u : 1u);
-          }
-          publish<true>(L, l - c0, r - c0, own, r, mypatch);
+          const bool up_left = (l == 0) || (r != n - 1 && ndr < ndl);
+          half = 2u * (up_left ? r : l - 1) + (up_left ? 0u : 1u);
         }
+        publish<true>(L, l - c0, own);
       }
     }
-    store_level32(b, L, c0, node, half, l - c0);
+    store_level32(b, L, c0, node, half, l - c0, r, mypatch);
   }
 }
 
@@ -1248,28 +1227,32 @@ __global__ __launch_bounds__(256) void k_slab_error(ElemInput in, const double* 
 
 // The fp32 leaf halves of a wave (slabs from the leaves' LDS slots, leaf id,
 // input index) stored as 16-byte pieces in address order: lane l of store j
-// writes piece q = k mod 7 of the wave's leaf k / 7 (k = 64 j + l), so the 64
-// lanes of one store cover about nine consecutive halves rather than 64
-// scattered ones.  half: the lane's record half (2 x parent + side), or kEnd
-// for a lane without a leaf.  Called by all 64 lanes of the wave.
+// writes piece q = k mod 8 of the wave's leaf k / 8 (k = 64 j + l), so the 64
+// lanes of one store cover eight consecutive halves rather than 64 scattered
+// ones.  Piece 7 of a right half holds nothing and is written so that
+// memory gets whole 64-byte sectors (2M triangles 296 -> 279 us, with the inner
+// nodes' below 275); that of a left half is the record's range.  half: the
+// lane's record half (2 x parent + side), or kEnd for a lane without a leaf.
+// Called by all 64 lanes of the wave.
 __device__ __forceinline__ void store_leaf_halves32(const BuildBufs& b, const ChunkLds<true>& L, uint32_t t,
                                                     uint32_t half, uint32_t e, uint32_t c0, uint64_t n) {
   int4* base = (int4*)b.rec32;
   const uint32_t lane = t & (kWave - 1), w0 = t - lane;
   const uint32_t leaf0 = (uint32_t)(n - 1) + c0 + w0;
 #pragma unroll
-  for (uint32_t j = 0; j < 7; ++j) {
+  for (uint32_t j = 0; j < 8; ++j) {
     const uint32_t k = kWave * j + lane;
-    const uint32_t i = k / 7u, q = k - 7u * i;
+    const uint32_t i = k >> 3, q = k & 7u;
     const uint32_t h = (uint32_t)__shfl((int)half, (int)i, kWave);
     const uint32_t ei = (uint32_t)__shfl((int)e, (int)i, kWave);
     const uint32_t sl = w0 + i;
     // piece q holds slabs 4q .. 4q+3; piece 6 slabs 24, 25, the leaf id and
-    // its input index
-    const int32_t x = L.slab[4 * q][sl], y = L.slab[4 * q + 1][sl];
-    const int32_t z = q < 6 ? L.slab[4 * q + 2][sl] : (int32_t)(leaf0 + i);
-    const int32_t w = q < 6 ? L.slab[4 * q + 3][sl] : (int32_t)ei;
-    if (h != kEnd) base[(uint64_t)h * 8u + q] = make_int4(x, y, z, w);
+    // its input index; piece 7 is not read
+    const uint32_t r0 = q < 7 ? 4 * q : 0;
+    const int32_t x = L.slab[r0][sl], y = L.slab[r0 + 1][sl];
+    const int32_t z = q < 6 ? L.slab[q < 6 ? r0 + 2 : 0][sl] : (int32_t)(leaf0 + i);
+    const int32_t w = q < 6 ? L.slab[q < 6 ? r0 + 3 : 0][sl] : (int32_t)ei;
+    if (h != kEnd && (q < 7 || (h & 1))) base[(uint64_t)h * 8u + q] = make_int4(x, y, z, w);
   }
 }
 
@@ -1289,7 +1272,7 @@ __global__ __launch_bounds__(kTreeChunk) void k_tree_leaves(ElemInput in, BuildB
 #pragma unroll
     for (int a = 0; a < kAxes; ++a) po[a] = b.origin[3 + a];
   }
-  L.cnt[t] = 0;
+  L.far[t] = 0;
   {
     // delta[c0 - 1 + t] for t in [0, 256], where the index is in [0, n - 2]
     const uint64_t di = (uint64_t)c0 + t;  // = (c0 - 1 + t) + 1
@@ -1324,9 +1307,6 @@ __global__ __launch_bounds__(kTreeChunk) void k_tree_leaves(ElemInput in, BuildB
     const bool single = patch_begin(b.splits, od, pk) == p && patch_end(b.splits, od, n, pk) == p + 1;
     if (single) b.patch_root[pk] = leaf;
     if constexpr (FP32) {
-      L.last[t] = p;
-      L.patch[t] = pk;
-      L.endslot[t] = t;
       // the leaf's half of its parent's record (the root's array if n = 1),
       // from its LDS slot, all its stores together; the slabs stay in
       // registers for the climb
@@ -1342,7 +1322,7 @@ __global__ __launch_bounds__(kTreeChunk) void k_tree_leaves(ElemInput in, BuildB
       double kd[kSlabs];
       element_kdop<KIND, NV>(in, e, kd);
       if (single) store_patch_box<false>(b, pk, kd);
-      publish<false>(L, t, t, kd, p, pk);
+      publish<false>(L, t, kd);
       if (n == 1) {
         *b.root = leaf;
         store_rootbox<false>(b, kd);
@@ -1356,13 +1336,13 @@ __global__ __launch_bounds__(kTreeChunk) void k_tree_leaves(ElemInput in, BuildB
   }
   __syncthreads();  // counters, deltas and leaf slots ready
   if constexpr (FP32) climb_chunk32(b, n, act && n > 1, p, p, pk, c0, c1, L, own);
-  else if (act && n > 1) climb_chunk<FP32>(b, n, p, p, pk, c0, c1, L, own);
+  else if (act && n > 1) climb_chunk64(b, n, p, p, pk, c0, c1, L);
   __syncthreads();
   // a first arrival whose sibling lies outside the chunk leaves its arrival word
-  if (c0 + t + 1 < c1 && L.cnt[t] == 1) {
+  if (c0 + t + 1 < c1 && L.far[t] != 0) {
     // (the far end's neighbour: left of a left child's first position, right
     // of a right child's last)
-    const uint32_t f = L.far[t] - c0;
+    const uint32_t f = L.far[t] - 1u - c0;
     b.counters[c0 + t] = arrival_word(c0 + f, L.delta[f <= t ? f : f + 1]);
   }
   if (t < 2) b.front_a[2 * chunk + t] = (t < L.nfront) ? L.front[t] : FrontNode{kEnd, kEnd, kEnd, 0u};
