@@ -1091,9 +1091,11 @@ __global__ __launch_bounds__(256) void k_narrow64s(TreeView q, TreeView t, int x
 // sized for it); kGeneric: any mix, chosen at run time.
 constexpr int kGeneric = -1;
 
-// blocks per re-check stripe (2,048 in all): each block strides over its
-// stripe's list, so a block stages many pairs per flush
-constexpr uint64_t kRecheckBlocksPerStripe = 32;
+// blocks per re-check stripe (512 in all): each block strides over its
+// stripe's list, so a block stages many pairs per flush (12.6M candidates of a
+// 2M-triangle mesh against itself: 409 us; with 32 / 16 / 6 / 4 blocks a stripe 567 /
+// 522 / 508 / 506; 54,612 hexes 42 us, 51 / 46 / 52 / 65)
+constexpr uint64_t kRecheckBlocksPerStripe = 8;
 
 template <int KIND, int NV>
 __global__ __launch_bounds__(256) void k_recheck(TreeView q, TreeView t, PairOut out) {
@@ -1101,11 +1103,24 @@ __global__ __launch_bounds__(256) void k_recheck(TreeView q, TreeView t, PairOut
   uint64_t* buf = s_buf[threadIdx.x / kWave];
   uint32_t fill = 0;
   if (blockIdx.x == 0 && threadIdx.x < kRecheckStripes) {
-    const unsigned long long c = out.rcount[(uint64_t)threadIdx.x * kRecheckStride];
-    atomicAdd(out.rtotal, c);
-    atomicMax(out.rtotal + 1, c);
-    if (out.visits) atomicAdd(out.visits, out.rcount[(uint64_t)threadIdx.x * kRecheckStride + 1]);
-    if (out.candidates) atomicAdd(out.candidates, out.rcount[(uint64_t)threadIdx.x * kRecheckStride + 2]);
+    // one wave: summed in registers (an addition per lane to these neighbouring
+    // words queued for 10 us, most of this kernel on short lists)
+    static_assert(kRecheckStripes == kWave, "a lane per stripe");
+    const unsigned long long* line = out.rcount + (uint64_t)threadIdx.x * kRecheckStride;
+    unsigned long long c = line[0], mx = c, v = line[1], k = line[2];
+    for (int o = kWave / 2; o > 0; o >>= 1) {
+      c += __shfl_xor(c, o, kWave);
+      v += __shfl_xor(v, o, kWave);
+      k += __shfl_xor(k, o, kWave);
+      const unsigned long long y = __shfl_xor(mx, o, kWave);
+      mx = y > mx ? y : mx;
+    }
+    if (threadIdx.x == 0) {
+      atomicAdd(out.rtotal, c);
+      atomicMax(out.rtotal + 1, mx);
+      if (out.visits) atomicAdd(out.visits, v);
+      if (out.candidates) atomicAdd(out.candidates, k);
+    }
   }
   const uint32_t stripe = blockIdx.x % kRecheckStripes;
   const uint32_t per = gridDim.x / kRecheckStripes;
