@@ -325,9 +325,9 @@ struct ClusterCut {
   uint32_t D, need;
 };
 
-// threshold of the histogram, computed by every block (256 bins in LDS)
+// threshold of the histogram, computed by every block of 256 threads, a bin each
 __device__ __forceinline__ ClusterCut cluster_cut(const uint32_t* __restrict__ hist, uint64_t c) {
-  __shared__ uint32_t h[256];
+  __shared__ uint32_t ws[4];
   __shared__ ClusterCut cut;
   uint32_t hv[kHistCopies];  // (all loads issued before the sum)
 #pragma unroll
@@ -335,17 +335,16 @@ __device__ __forceinline__ ClusterCut cluster_cut(const uint32_t* __restrict__ h
   uint32_t v = 0;
 #pragma unroll
   for (int c = 0; c < kHistCopies; ++c) v += hv[c];
-  h[threadIdx.x] = v;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    uint64_t cum = 0;
-    uint32_t d = 0;
-    for (; d < 255; ++d) {
-      if (cum + h[d] >= c) break;
-      cum += h[d];
-    }
-    cut = ClusterCut{d, (uint32_t)(c - cum)};
+  uint32_t incl = v;  // (all bins together count n - 1 < 2^30 boundaries)
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t x = (uint32_t)__shfl_up((int)incl, o, 64);
+    if ((int)lane_id() >= o) incl += x;
   }
+  if (lane_id() == 63) ws[threadIdx.x / 64] = incl;
+  __syncthreads();
+  for (uint32_t w = 0; w < threadIdx.x / 64; ++w) incl += ws[w];
+  const uint32_t before = incl - v;
+  if (incl >= c && (threadIdx.x == 0 || before < c)) cut = ClusterCut{threadIdx.x, (uint32_t)(c - before)};
   __syncthreads();
   return cut;
 }
@@ -354,17 +353,19 @@ __device__ __forceinline__ ClusterCut cluster_cut(const uint32_t* __restrict__ h
 __global__ __launch_bounds__(256) void k_cluster_count(const uint32_t* __restrict__ depth, uint64_t m,
                                                        const uint32_t* __restrict__ hist, uint64_t c,
                                                        uint32_t* __restrict__ counts) {
-  const ClusterCut cut = cluster_cut(hist, c);
   const uint64_t base = (uint64_t)blockIdx.x * kClusterTile;
-  uint32_t lt = 0, eq = 0;
+  uint32_t d[kClusterItems];  // (on their way while the threshold is found)
 #pragma unroll
   for (uint32_t k = 0; k < kClusterItems; ++k) {
     const uint64_t i = base + (uint64_t)k * 256 + threadIdx.x;
-    if (i < m) {
-      const uint32_t d = depth[i];
-      lt += d < cut.D;
-      eq += d == cut.D;
-    }
+    d[k] = i < m ? depth[i] : 0xffffffffu;  // (above every threshold)
+  }
+  const ClusterCut cut = cluster_cut(hist, c);
+  uint32_t lt = 0, eq = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < kClusterItems; ++k) {
+    lt += d[k] < cut.D;
+    eq += d[k] == cut.D;
   }
   // block sums: wave reductions, then LDS
   for (int o = 32; o > 0; o >>= 1) {
@@ -411,37 +412,70 @@ __global__ __launch_bounds__(1024) void k_cluster_scan(uint32_t* __restrict__ co
   }
 }
 
-// the taken boundaries in position order; slots c .. nsplits - 1 take n - 1
+// the taken boundaries in position order; slots c .. nsplits - 1 take n - 1.
+// The tile's depths are loaded together and its waves' counts exchanged once:
+// with a barrier and a load per row of 256, the 16 rows took 10 us.  `counts` are
+// the tiles' counts, or with `scanned` their exclusive sums: up to 256 tiles
+// every block adds up those before its own, a count per thread (a launch less).
 __global__ __launch_bounds__(256) void k_cluster_emit(const uint32_t* __restrict__ depth, uint64_t m,
                                                       const uint32_t* __restrict__ hist, uint64_t c,
-                                                      const uint32_t* __restrict__ offs, uint64_t nsplits,
-                                                      uint32_t* __restrict__ splits) {
-  const ClusterCut cut = cluster_cut(hist, c);
+                                                      const uint32_t* __restrict__ counts, int scanned,
+                                                      uint64_t nsplits, uint32_t* __restrict__ splits) {
   const uint64_t base = (uint64_t)blockIdx.x * kClusterTile;
-  __shared__ uint32_t wl[4], we[4];
-  uint32_t lt0 = offs[2 * blockIdx.x], eq0 = offs[2 * blockIdx.x + 1];
-  const uint32_t wv = threadIdx.x / 64;
+  __shared__ uint32_t wl[kClusterItems * 4], we[kClusterItems * 4];  // per wave of 64 boundaries, in order
+  uint32_t d[kClusterItems];
+#pragma unroll
   for (uint32_t k = 0; k < kClusterItems; ++k) {
     const uint64_t i = base + (uint64_t)k * 256 + threadIdx.x;
-    const uint32_t d = i < m ? depth[i] : 0xffffffffu;
-    const bool isl = i < m && d < cut.D, ise = i < m && d == cut.D;
-    const uint64_t ml = __ballot(isl), me = __ballot(ise);
+    d[k] = i < m ? depth[i] : 0xffffffffu;  // (above every threshold)
+  }
+  const uint32_t from = scanned ? blockIdx.x : threadIdx.x;
+  const bool mine = scanned ? threadIdx.x == 0 : threadIdx.x < blockIdx.x;
+  uint32_t lt0 = mine ? counts[2 * from] : 0u, eq0 = mine ? counts[2 * from + 1] : 0u;
+  __shared__ uint32_t s0[2][4];
+  for (int o = 32; o > 0; o >>= 1) {
+    lt0 += (uint32_t)__shfl_xor((int)lt0, o, 64);
+    eq0 += (uint32_t)__shfl_xor((int)eq0, o, 64);
+  }
+  if (lane_id() == 0) {
+    s0[0][threadIdx.x / 64] = lt0;
+    s0[1][threadIdx.x / 64] = eq0;
+  }
+  const ClusterCut cut = cluster_cut(hist, c);
+  const uint32_t wv = threadIdx.x / 64;
+#pragma unroll
+  for (uint32_t k = 0; k < kClusterItems; ++k) {
+    const uint64_t ml = __ballot(d[k] < cut.D), me = __ballot(d[k] == cut.D);
     if (lane_id() == 0) {
-      wl[wv] = (uint32_t)__popcll(ml);
-      we[wv] = (uint32_t)__popcll(me);
+      wl[4 * k + wv] = (uint32_t)__popcll(ml);
+      we[4 * k + wv] = (uint32_t)__popcll(me);
     }
-    __syncthreads();
-    uint32_t lb = lt0, eb = eq0;
-    for (uint32_t v = 0; v < wv; ++v) {
-      lb += wl[v];
-      eb += we[v];
+  }
+  __syncthreads();
+  lt0 = s0[0][0] + s0[0][1] + s0[0][2] + s0[0][3];
+  eq0 = s0[1][0] + s0[1][1] + s0[1][2] + s0[1][3];
+  // lane w of every wave: the taken boundaries before row-wave w of the tile
+  static_assert(kClusterItems * 4 == 64, "a lane per row and wave");
+  const uint32_t l0 = wl[lane_id()], e0 = we[lane_id()];
+  uint32_t li = l0, ei = e0;
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t x = (uint32_t)__shfl_up((int)li, o, 64), y = (uint32_t)__shfl_up((int)ei, o, 64);
+    if ((int)lane_id() >= o) {
+      li += x;
+      ei += y;
     }
-    const uint32_t lr = lb + (uint32_t)__popcll(ml & lanemask_lt());
-    const uint32_t er = eb + (uint32_t)__popcll(me & lanemask_lt());
-    if (isl || (ise && er < cut.need)) splits[lr + (er < cut.need ? er : cut.need)] = (uint32_t)i;
-    lt0 += wl[0] + wl[1] + wl[2] + wl[3];
-    eq0 += we[0] + we[1] + we[2] + we[3];
-    __syncthreads();
+  }
+  li += lt0 - l0;
+  ei += eq0 - e0;
+#pragma unroll
+  for (uint32_t k = 0; k < kClusterItems; ++k) {
+    const bool isl = d[k] < cut.D, ise = d[k] == cut.D;
+    const uint64_t ml = __ballot(isl), me = __ballot(ise);
+    if ((ml | me) == 0) continue;
+    const uint32_t lr = (uint32_t)__shfl((int)li, (int)(4 * k + wv), 64) + (uint32_t)__popcll(ml & lanemask_lt());
+    const uint32_t er = (uint32_t)__shfl((int)ei, (int)(4 * k + wv), 64) + (uint32_t)__popcll(me & lanemask_lt());
+    if (isl || (ise && er < cut.need))
+      splits[lr + (er < cut.need ? er : cut.need)] = (uint32_t)(base + (uint64_t)k * 256 + threadIdx.x);
   }
   if (blockIdx.x == 0) {
     const uint32_t fillv = (uint32_t)m;  // n - 1
@@ -1566,9 +1600,10 @@ hipError_t launch_cluster(const BuildBufs& b, uint64_t n, int bits, uint64_t nsp
     uint32_t* counts = b.depth_idx;  // 2 words per tile (n words available)
     hipLaunchKernelGGL(k_cluster_count, dim3((unsigned)tiles), dim3(256), 0, s, (const uint32_t*)b.depth0, m,
                        (const uint32_t*)hist, c, counts);
-    hipLaunchKernelGGL(k_cluster_scan, dim3(1), dim3(1024), 0, s, counts, (uint32_t)tiles);
+    const int scanned = tiles > 256;
+    if (scanned) hipLaunchKernelGGL(k_cluster_scan, dim3(1), dim3(1024), 0, s, counts, (uint32_t)tiles);
     hipLaunchKernelGGL(k_cluster_emit, dim3((unsigned)tiles), dim3(256), 0, s, (const uint32_t*)b.depth0, m,
-                       (const uint32_t*)hist, c, (const uint32_t*)counts, nsplits, b.splits);
+                       (const uint32_t*)hist, c, (const uint32_t*)counts, scanned, nsplits, b.splits);
     return hipGetLastError();
   }
   hipLaunchKernelGGL(k_cluster_select, dim3(1), dim3(1024), 0, s, (const uint32_t*)b.depth_idx, n, nsplits, b.splits);
