@@ -149,7 +149,7 @@ struct bvh_world_s {
   DevBuf s_kb, s_ka, s_va, s_vb, s_hist, s_ctl, s_lb;
   DevBuf prim_in, prim_out;  // host-memory staging of bvh_closest_point
   // bvh_max_variant_axis / bvh_sort_and_sweep: staging, sorted B, counts
-  DevBuf sw_ka, sw_kb, sw_ga, sw_gb, sw_bq, sw_bidx, sw_kbs, sw_bmax, sw_count, sw_total, sw_out, sw_part;
+  DevBuf sw_ka, sw_kb, sw_ga, sw_gb, sw_bq, sw_bidx, sw_kbs, sw_bmax, sw_tmax, sw_count, sw_total, sw_out, sw_part;
   LaunchShape shape;  // narrowphase launch shape (autotuned)
   // stream capture (batching form): the queries captured so far, with the
   // state a replay restores in their objects
@@ -2549,16 +2549,18 @@ bvh_status bvh_sort_and_sweep(bvh_world w, const double* pa, const double* ka, c
   BVH_TRY(w->sw_bidx.ensure(nb * 4));
   BVH_TRY(w->sw_kbs.ensure(nb * 26 * sizeof(double)));
   BVH_TRY(w->sw_bmax.ensure(nb * sizeof(double)));
+  BVH_TRY(w->sw_tmax.ensure((nb + 63) / 64 * sizeof(double)));
   BVH_TRY(w->sw_count.ensure(na * 4));
   BVH_TRY(w->sw_total.ensure(sizeof(unsigned long long)));
   HIP_TRY(launch_sweep_prepare(dkb, nb, axis, gmin, conv, w->sw_bq.as<uint32_t>(), w->sw_bidx.as<uint32_t>(), s));
   BVH_TRY(prim_sort<uint32_t>(w, w->sw_bq.as<uint32_t>(), w->sw_bidx.as<uint32_t>(), nb));
   HIP_TRY(launch_sweep_gather(dkb, w->sw_bidx.as<uint32_t>(), nb, axis, gmin, conv, w->sw_kbs.as<double>(),
-                              w->sw_bmax.as<double>(), s));
+                              w->sw_bmax.as<double>(), w->sw_tmax.as<double>(), s));
   a.na = na;
   a.nb = nb;
   a.kbs = w->sw_kbs.as<double>();
   a.bmax = w->sw_bmax.as<double>();
+  a.tmax = w->sw_tmax.as<double>();
   a.bq = w->sw_bq.as<uint32_t>();
   a.bidx = w->sw_bidx.as<uint32_t>();
   a.axis = axis;

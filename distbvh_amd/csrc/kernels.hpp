@@ -256,8 +256,9 @@ struct SweepArgs {
   const double* ka;            // A's k-DOPs, na x 26
   const uint64_t* ga;          // A's global ids (null: local indices)
   uint64_t na;
-  const double* kbs;           // B's k-DOPs in sorted order, nb x 26
+  const double* kbs;           // B's k-DOPs in sorted order, 26 planes of nb
   const double* bmax;          // B's scaled maxima on the axis, sorted order
+  const double* tmax;          // the largest of each 64 of them (+inf: one is NaN)
   const uint32_t* bq;          // B's truncated minima, sorted
   const uint32_t* bidx;        // sorted position -> B index
   const uint64_t* gb;          // B's global ids (null: local indices)
@@ -265,7 +266,7 @@ struct SweepArgs {
   int axis;
   double gmin, conv;
   uint32_t* count;             // per a: count (count pass), exclusive offset (write pass)
-  unsigned long long* total;   // zeroed before the count pass
+  unsigned long long* total;   // the counts' sum (count pass)
   uint64_t* out;               // 2 words per pair
 };
 // max_variant_axis: partials (variant_axis_partials() x 6 doubles), axis out
@@ -275,7 +276,8 @@ uint32_t variant_axis_partials();
 hipError_t launch_sweep_prepare(const double* kb, uint64_t nb, int axis, double gmin, double conv, uint32_t* bq,
                                 uint32_t* bidx, hipStream_t s);
 hipError_t launch_sweep_gather(const double* kb, const uint32_t* bidx, uint64_t nb, int axis, double gmin,
-                               double conv, double* kbs, double* bmax, hipStream_t s);
+                               double conv, double* kbs, double* bmax, double* tmax,
+                               hipStream_t s);
 hipError_t launch_sweep(const SweepArgs& a, bool write, hipStream_t s);
 // 26-DOPs of in.n polytopes of in.nv vertices (kPoly planes), n x 26
 hipError_t launch_element_kdops(const ElemInput& in, double* out, hipStream_t s);

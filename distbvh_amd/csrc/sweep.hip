@@ -10,9 +10,14 @@
 // and reports (a, b) when the two 26-DOPs overlap.
 //
 // The stop is the first sorted position whose minimum exceeds a's maximum,
-// i.e. an upper bound found by binary search; the visited range is then
-// walked 64 positions at a time by one wave per a, so each a's pairs come out
-// in B's sorted order, as the reference's callback sees them.  A count pass
+// i.e. an upper bound, searched 64 ways by the wave that sweeps a.  The range
+// before it is walked in tiles of 64 positions, in order, so each a's pairs
+// come out in B's sorted order, as the reference's callback sees them; a tile
+// whose largest scaled maximum lies below a's minimum holds only skipped b, and
+// one ballot finds the others among 64 tiles (of 8,192 x 8,192 sheet elements
+// six are left where 64 of the 128 were walked: 73 + 70 us for the two passes
+// instead of 120 + 102).  What a walked tile costs is its reads: the sorted k-DOPs
+// are planes, and x, y, z are tested first (35 + 34 us).  A count pass
 // and a write pass at per-a offsets (exclusive scan) make the output order
 // (a ascending, then sorted b) independent of scheduling.
 #include "device.hpp"
@@ -58,13 +63,22 @@ __global__ __launch_bounds__(kMomentBlock) void k_moments(const double* __restri
 
 // The block sums folded in block order, then var = s2 - s * s / n per axis
 // and the first axis of largest variance (kokkos.hpp:144-158).
-__global__ void k_variant_axis(const double* __restrict__ part, uint32_t nblocks, uint64_t n,
-                               int32_t* __restrict__ axis) {
+__global__ __launch_bounds__(256) void k_variant_axis(const double* __restrict__ part, uint32_t nblocks, uint64_t n,
+                                                      int32_t* __restrict__ axis) {
+  // the partials through LDS, then a lane per sum, in block order (one thread
+  // that loaded as it added took 15 us)
+  __shared__ double sp[kMomentBlocks * 6];
+  __shared__ double s[6];
+  for (uint32_t i = threadIdx.x; i < nblocks * 6; i += 256) sp[i] = part[i];
+  __syncthreads();
+  if (threadIdx.x < 6) {
+    double x = 0;
+#pragma unroll 8
+    for (uint32_t b = 0; b < nblocks; ++b) x = x + sp[b * 6 + threadIdx.x];
+    s[threadIdx.x] = x;
+  }
+  __syncthreads();
   if (threadIdx.x != 0) return;
-  double s[6] = {0, 0, 0, 0, 0, 0};
-  for (uint32_t b = 0; b < nblocks; ++b)
-#pragma unroll
-    for (int k = 0; k < 6; ++k) s[k] = s[k] + part[(uint64_t)b * 6 + k];
   double var[3];
 #pragma unroll
   for (int i = 0; i < 3; ++i) var[i] = s[3 + i] - s[i] * s[i] / (double)n;
@@ -85,38 +99,82 @@ __global__ __launch_bounds__(256) void k_sweep_quantize(const double* __restrict
   bidx[i] = (uint32_t)i;
 }
 
-// B's k-DOPs and scaled maxima in sorted order, so that the sweep reads
-// consecutive positions.
+// B's k-DOPs in sorted order, as 26 planes, and their scaled maxima; and the
+// largest scaled maximum of every 64 sorted positions.  A block per 64: its
+// rows come in through LDS and leave as plane segments, so that both sides are
+// whole lines.
 __global__ __launch_bounds__(256) void k_sweep_gather(const double* __restrict__ kb, const uint32_t* __restrict__ bidx,
                                                       uint64_t nb, int axis, double gmin, double conv,
-                                                      double* __restrict__ kbs, double* __restrict__ bmax) {
-  const uint64_t total = nb * 26;
-  for (uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; t < total;
-       t += (uint64_t)gridDim.x * blockDim.x) {
-    const uint64_t j = t / 26;
-    const int k = (int)(t - j * 26);
-    const double v = kb[(uint64_t)bidx[j] * 26 + k];
-    kbs[t] = v;
-    if (k == 2 * axis + 1) bmax[j] = (v - gmin) * conv;
+                                                      double* __restrict__ kbs, double* __restrict__ bmax,
+                                                      double* __restrict__ tmax) {
+  __shared__ double s[64][kSlabs + 1];
+  const uint64_t j0 = (uint64_t)blockIdx.x * 64;
+  const uint32_t cnt = nb - j0 < 64 ? (uint32_t)(nb - j0) : 64u;
+  for (uint32_t t = threadIdx.x; t < cnt * kSlabs; t += 256) {
+    const uint32_t j = t / kSlabs, k = t - j * kSlabs;
+    s[j][k] = kb[(uint64_t)bidx[j0 + j] * kSlabs + k];
+  }
+  __syncthreads();
+  const uint32_t j = threadIdx.x & 63;
+  if (j < cnt)
+    for (uint32_t k = threadIdx.x >> 6; k < kSlabs; k += 4) kbs[(uint64_t)k * nb + j0 + j] = s[j][k];
+  if (threadIdx.x < 64) {
+    double v = -__builtin_inf();
+    if (j < cnt) {
+      v = (s[j][2 * axis + 1] - gmin) * conv;
+      bmax[j0 + j] = v;
+    }
+    if (!(v == v)) v = __builtin_inf();  // a NaN is below nothing: its tile is walked
+    for (int o = 32; o > 0; o >>= 1) {
+      const double x = __shfl_xor(v, o, 64);
+      v = x > v ? x : v;
+    }
+    if (j == 0) tmax[blockIdx.x] = v;
   }
 }
 
-// The sweep of one element a of A by one wave: COUNT writes a's pair count
-// and adds it to the 64-bit total; WRITE writes the pairs at a's exclusive
-// offset.
+// The 64-bit sum of the counts: one addition a block, where one a wave of the
+// sweep queued for the word.
+__global__ __launch_bounds__(256) void k_sweep_total(const uint32_t* __restrict__ count, uint64_t na,
+                                                     unsigned long long* __restrict__ total) {
+  __shared__ unsigned long long s[4];
+  unsigned long long c = 0;
+  for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < na; i += (uint64_t)gridDim.x * 256) c += count[i];
+  for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
+  if (lane_id() == 0) s[threadIdx.x >> 6] = c;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    c = s[0] + s[1] + s[2] + s[3];
+    if (c) atomicAdd(total, c);
+  }
+}
+
+// Strict overlap on axes [A0, A1) of a's k-DOP with the k-DOP in planes of nb.
+template <int A0, int A1>
+__device__ __forceinline__ bool sweep_axes(const double* ak, const double* kb, uint64_t nb) {
+  bool o = true;
+#pragma unroll
+  for (int x = A0; x < A1; ++x)
+    o = o & (ak[2 * x] < kb[(uint64_t)(2 * x + 1) * nb]) & (kb[(uint64_t)(2 * x) * nb] < ak[2 * x + 1]);
+  return o;
+}
+
+// The sweep of one element a of A by one wave: COUNT writes a's pair count;
+// WRITE writes the pairs at a's exclusive offset.
 template <bool WRITE>
 __device__ __forceinline__ void sweep_one(const SweepArgs& a, uint64_t ai, int lane) {
   const double* ak = a.ka + ai * 26;
   const uint32_t amin = (uint32_t)float_to_uint((ak[2 * a.axis] - a.gmin) * a.conv);
   const uint32_t amax = (uint32_t)float_to_uint((ak[2 * a.axis + 1] - a.gmin) * a.conv);
   // the first sorted position whose minimum exceeds amax: the sweep's stop
+  // (64 probes a round: those at or below amax are the first c of them)
   uint64_t lo = 0, hi = a.nb;
   while (lo < hi) {
-    const uint64_t mid = (lo + hi) >> 1;
-    if (a.bq[mid] > amax)
-      hi = mid;
-    else
-      lo = mid + 1;
+    const uint64_t step = (hi - lo + 63) / 64, at = lo + (uint64_t)lane * step;
+    const uint64_t c = (uint64_t)__popcll(__ballot(at < hi && a.bq[at < hi ? at : lo] <= amax));
+    if (c == 0) break;  // position lo is above
+    if (lo + c * step < hi) hi = lo + c * step;
+    lo += (c - 1) * step + 1;
   }
   const uint64_t ub = lo;
   uint32_t cnt = 0;
@@ -126,13 +184,25 @@ __device__ __forceinline__ void sweep_one(const SweepArgs& a, uint64_t ai, int l
     base = a.count[ai];
     gid_a = a.ga ? a.ga[ai] : ai;
   }
-  for (uint64_t j0 = 0; j0 < ub; j0 += 64) {
-    const uint64_t j = j0 + lane;
+  uint64_t t0 = 0, tiles = 0;  // tiles to walk among the 64 from t0 - 64 on
+  for (;;) {
+    while (tiles == 0 && t0 * 64 < ub) {
+      const uint64_t t = t0 + lane;
+      tiles = __ballot(t * 64 < ub && !(a.tmax[t * 64 < ub ? t : t0] < (double)amin));
+      t0 += 64;
+    }
+    if (tiles == 0) break;
+    const uint64_t j = (t0 - 64 + (uint64_t)__builtin_ctzll(tiles)) * 64 + lane;
+    tiles &= tiles - 1;
     bool hit = false;
     if (j < ub) {
       // skipped while b lies below a (bmax < amin, fp64 against the integer)
-      if (!(a.bmax[j] < (double)amin)) hit = overlap(ak, a.kbs + j * 26);
+      hit = !(a.bmax[j] < (double)amin);
+      // x, y and z first: the other axes are read if these leave a lane
+      hit = hit & sweep_axes<0, 3>(ak, a.kbs + j, a.nb);
     }
+    if (__ballot(hit) == 0) continue;
+    if (j < ub) hit = hit & sweep_axes<3, kAxes>(ak, a.kbs + j, a.nb);
     const uint64_t m = __ballot(hit);
     if constexpr (WRITE) {
       if (hit) {
@@ -146,10 +216,7 @@ __device__ __forceinline__ void sweep_one(const SweepArgs& a, uint64_t ai, int l
     cnt += (uint32_t)__popcll(m);
   }
   if constexpr (!WRITE) {
-    if (lane == 0) {
-      a.count[ai] = cnt;
-      atomicAdd(a.total, (unsigned long long)cnt);
-    }
+    if (lane == 0) a.count[ai] = cnt;
   }
 }
 
@@ -199,7 +266,7 @@ hipError_t launch_variant_axis(const double* ca, uint64_t na, const double* cb, 
   if (blocks > kMomentBlocks) blocks = kMomentBlocks;
   if (blocks == 0) blocks = 1;
   hipLaunchKernelGGL(k_moments, dim3((uint32_t)blocks), dim3(kMomentBlock), 0, s, ca, na, cb, nb, part);
-  hipLaunchKernelGGL(k_variant_axis, dim3(1), dim3(64), 0, s, part, (uint32_t)blocks, n, axis);
+  hipLaunchKernelGGL(k_variant_axis, dim3(1), dim3(256), 0, s, part, (uint32_t)blocks, n, axis);
   return hipGetLastError();
 }
 
@@ -214,12 +281,10 @@ hipError_t launch_sweep_prepare(const double* kb, uint64_t nb, int axis, double 
 }
 
 hipError_t launch_sweep_gather(const double* kb, const uint32_t* bidx, uint64_t nb, int axis, double gmin,
-                               double conv, double* kbs, double* bmax, hipStream_t s) {
+                               double conv, double* kbs, double* bmax, double* tmax, hipStream_t s) {
   if (nb == 0) return hipSuccess;
-  uint64_t blocks = (nb * 26 + 255) / 256;
-  if (blocks > 65536) blocks = 65536;
-  hipLaunchKernelGGL(k_sweep_gather, dim3((uint32_t)blocks), dim3(256), 0, s, kb, bidx, nb, axis, gmin,
-                     conv, kbs, bmax);
+  hipLaunchKernelGGL(k_sweep_gather, dim3((uint32_t)((nb + 63) / 64)), dim3(256), 0, s, kb, bidx, nb, axis, gmin,
+                     conv, kbs, bmax, tmax);
   return hipGetLastError();
 }
 
@@ -227,10 +292,14 @@ hipError_t launch_sweep(const SweepArgs& a, bool write, hipStream_t s) {
   if (a.na == 0) return hipSuccess;
   uint64_t blocks = (a.na + 3) / 4;
   if (blocks > 65536) blocks = 65536;
-  if (write)
+  if (write) {
     hipLaunchKernelGGL(k_sweep<true>, dim3((uint32_t)blocks), dim3(256), 0, s, a);
-  else
+  } else {
     hipLaunchKernelGGL(k_sweep<false>, dim3((uint32_t)blocks), dim3(256), 0, s, a);
+    uint64_t sum = (a.na + 2047) / 2048;
+    if (sum > 64) sum = 64;
+    hipLaunchKernelGGL(k_sweep_total, dim3((uint32_t)sum), dim3(256), 0, s, (const uint32_t*)a.count, a.na, a.total);
+  }
   return hipGetLastError();
 }
 

@@ -180,3 +180,28 @@ def test_element_kdops(torch_cuda, nv, eps):
         assert np.array_equal(w.element_kdops(verts, eps), exp)
         assert np.array_equal(w.element_kdops(to_cuda(verts), eps).cpu().numpy(), exp)
         assert w.element_kdops(verts[:, :, :0]).shape == (0, 26)
+
+
+@pytest.mark.parametrize("na,nb", [(1, 63), (3, 64), (70, 65), (130, 4096), (130, 4097), (60, 8193), (2500, 300), (9, 70000)])
+def test_sweep_windows(torch_cuda, na, nb):
+    """Sizes around a tile of 64 positions and 64 tiles: short elements, a few
+    that span everything (every tile is walked for them, and their tiles for
+    every a), one with NaN slabs."""
+    rng = np.random.default_rng(na + nb)
+
+    def kdops(n, wide):
+        c, h = rng.random((n, 13)), rng.random((n, 13)) * 0.4 + 0.01
+        k = np.stack([c - h, c + h], axis=2)
+        c0 = rng.random(n)
+        k[:, 0] = np.stack([c0, c0 + 2.0 / nb], axis=1)
+        k[rng.integers(0, n, wide), 0] = [-0.5, 1.5]
+        return np.ascontiguousarray(k.reshape(n, 26))
+
+    ka, kb = kdops(na, na // 50), kdops(nb, 2)
+    if nb > 100:
+        kb[nb // 2] = np.nan
+    pa, pb = _patch(ka), _patch(np.nan_to_num(kb))
+    ga, gb = np.arange(na, dtype=np.uint64) + 7, np.arange(nb, dtype=np.uint64) + 11
+    exp = O.sort_and_sweep(pa, ka, ga, pb, kb, gb, 0)
+    with CollisionWorld(1) as w:
+        assert np.array_equal(w.sort_and_sweep(pa, ka, ga, pb, kb, gb, 0), exp)
