@@ -64,7 +64,7 @@ def kernel_bytes(stage, n, npairs, n_other, fp32=False, elem_bytes=72):
 
 # stage -> the kernel whose measured HBM traffic the roofline reports
 STAGE_KERNEL = {"tree": ("k_tree_leaves<0, 3, false>", "k_tree_leaves<0, 3, true>"),
-                "sort": ("k_sort_pass<unsigned long>", "k_sort_pass<unsigned long>")}
+                "sort": ("k_sort_pass<unsigned long, true>", "k_sort_pass<unsigned long, true>")}
 
 
 def stage_kernel(stage, fp32, launch):
@@ -73,7 +73,7 @@ def stage_kernel(stage, fp32, launch):
     the launch batch: one record in scalar registers, or K staged in LDS)."""
     if stage == "narrowphase":
         if fp32:
-            return "k_narrow32<false, false>"
+            return "k_narrow32<false, false, 0>"
         b = launch.get("batch", 1) if launch else 1
         return "k_narrow64s<false, false>" if b == 1 else "k_narrow64<false, %d, false>" % b
     return STAGE_KERNEL.get(stage, (None, None))[1 if fp32 else 0]
