@@ -1011,47 +1011,84 @@ __device__ __forceinline__ uint32_t arrive(const BuildBufs& b, uint64_t n, uint3
   return (is_left ? r + 1 : far) - c0;
 }
 
-// Phase-1 climb inside the chunk [c0, c1) from node [l, r] of patch
-// `mypatch`, whose slabs are in LDS slot l - c0 and in its half of its
-// parent's record.  Arrivals are LDS atomics whose fences order LDS only, so
-// a level costs LDS latency.  The second arriver forms the parent's slabs
-// from the two children's LDS slots, so no slabs are carried from one level
-// to the next (which keeps the register count down); record halves go to
-// global memory with stores that nothing in this kernel waits for.
-__device__ __forceinline__ void climb_chunk64(const BuildBufs& b, uint64_t n, uint32_t l, uint32_t r, uint32_t mypatch,
-                                              uint32_t c0, uint32_t c1, ChunkLds<false>& L) {
+// The fp64 halves of a wave's nodes, stored as 16-byte pieces in address order:
+// the lanes with a node (`half` = 2 x parent + side, else kEnd; slabs in LDS slot
+// `sl`) are ranked in lane order in the wave's part of L.order, and lane l of
+// store j writes piece k mod 13 of the node of rank k / 13 (k = 64 j + l).  Stored by
+// each lane for itself, a piece at a time, the 64 lanes of a store hit as many
+// records (524k triangles 130 -> 121 us).  Called by all lanes of the wave.
+__device__ __forceinline__ void store_halves64(const BuildBufs& b, ChunkLds<false>& L, uint32_t half, uint32_t sl) {
+  const uint64_t mask = __ballot(half != kEnd);
+  if (mask == 0) return;
+  double2* base = (double2*)b.rec64;
+  const uint32_t lane = lane_id(), w0 = threadIdx.x - lane;
+  if (half != kEnd) L.order[w0 + (uint32_t)__popcll(mask & lanemask_lt())] = (uint8_t)lane;
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  constexpr uint32_t kPieces = kSlabs / 2, kRecPieces = sizeof(Rec64) / 16;
+  const uint32_t pieces = kPieces * (uint32_t)__popcll(mask);
+  for (uint32_t k0 = 0; k0 < pieces; k0 += kWave) {  // wave-uniform
+    const uint32_t k = k0 + lane;
+    const uint32_t i = k < pieces ? k / kPieces : 0u, q = k - i * kPieces;
+    const int src = (int)L.order[w0 + i];
+    const uint32_t h = (uint32_t)__shfl((int)half, src, kWave);
+    const uint32_t s = (uint32_t)__shfl((int)sl, src, kWave);
+    if (k < pieces)
+      base[(uint64_t)(h >> 1) * kRecPieces + (h & 1u) * kPieces + q] = make_double2(L.slab[2 * q][s], L.slab[2 * q + 1][s]);
+  }
+}
+
+// The fp64 phase-1 climb inside the chunk [c0, c1), wave-synchronous as the fp32
+// one (climb_chunk32); alive: the lane holds leaf l = r, whose slabs are in its
+// LDS slot and in its half of its parent's record.  The slabs of a node are formed
+// from its children's slots, so none are carried from one level to the next (which
+// keeps the register count down).
+__device__ __forceinline__ void climb_chunk64(const BuildBufs& b, uint64_t n, bool alive, uint32_t l, uint32_t r,
+                                              uint32_t mypatch, uint32_t c0, uint32_t c1, ChunkLds<false>& L) {
   Rec64* recs = b.rec64;
-  for (;;) {
-    uint32_t parent, far;
-    bool is_left;
-    const uint32_t ss = arrive<false>(b, n, l, r, mypatch, c0, c1, L, parent, is_left, far);
-    if (ss == kEnd) return;
-    const uint32_t ms = l - c0;
-    double kd[kSlabs];
+  while (__ballot(alive) != 0) {
+    uint32_t half = kEnd;
+    if (alive) {
+      uint32_t parent, far;
+      bool is_left;
+      const uint32_t ss = arrive<false>(b, n, l, r, mypatch, c0, c1, L, parent, is_left, far);
+      if (ss == kEnd) {
+        alive = false;
+      } else {
+        const uint32_t ms = l - c0;
+        double kd[kSlabs];
 #pragma unroll
-    for (int a = 0; a < kAxes; ++a) {
-      const double lo0 = L.slab[2 * a][ms], lo1 = L.slab[2 * a][ss];
-      const double hi0 = L.slab[2 * a + 1][ms], hi1 = L.slab[2 * a + 1][ss];
-      kd[2 * a] = (lo0 < lo1) ? lo0 : lo1;
-      kd[2 * a + 1] = (hi0 > hi1) ? hi0 : hi1;
+        for (int a = 0; a < kAxes; ++a) {
+          const double lo0 = L.slab[2 * a][ms], lo1 = L.slab[2 * a][ss];
+          const double hi0 = L.slab[2 * a + 1][ms], hi1 = L.slab[2 * a + 1][ss];
+          kd[2 * a] = (lo0 < lo1) ? lo0 : lo1;
+          kd[2 * a + 1] = (hi0 > hi1) ? hi0 : hi1;
+        }
+        if (L.delta[parent - c0 + 1] >= 128) mypatch = kMixed;
+        if (is_left) r = far;
+        else l = far;
+        rec_set_range(recs[parent], l, r, mypatch);
+        const uint32_t ndl = L.delta[l - c0], ndr = L.delta[r - c0 + 1];
+        if (is_patch_root(mypatch, l, r, n, ndl, ndr)) {
+          b.patch_root[mypatch] = parent;
+          store_patch_box<false>(b, mypatch, kd);
+        }
+        if (l == 0 && r == n - 1) {
+          *b.root = parent;
+          store_rootbox<false>(b, kd);
+          alive = false;
+        } else {
+          const bool up_left = (l == 0) || (r != n - 1 && ndr < ndl);
+          const uint32_t up = up_left ? r : l - 1;
+          half = 2u * up + (up_left ? 0u : 1u);
+          recs[up].child[half & 1u] = parent;
+          recs[up].elem[half & 1u] = kEnd;
+          publish<false>(L, l - c0, kd);
+        }
+      }
     }
-    if (L.delta[parent - c0 + 1] >= 128) mypatch = kMixed;
-    if (is_left) r = far;
-    else l = far;
-    rec_set_range(recs[parent], l, r, mypatch);
-    const uint32_t ndl = L.delta[l - c0], ndr = L.delta[r - c0 + 1];
-    if (is_patch_root(mypatch, l, r, n, ndl, ndr)) {
-      b.patch_root[mypatch] = parent;
-      store_patch_box<false>(b, mypatch, kd);
-    }
-    if (l == 0 && r == n - 1) {
-      *b.root = parent;
-      store_rootbox<false>(b, kd);
-      return;
-    }
-    const bool up_left = (l == 0) || (r != n - 1 && ndr < ndl);
-    rec_store_half<false>(b, up_left ? r : l - 1, up_left ? 0 : 1, kd, parent, kEnd);
-    publish<false>(L, l - c0, kd);
+    store_halves64(b, L, half, l - c0);
   }
 }
 
@@ -1360,17 +1397,21 @@ __global__ __launch_bounds__(kTreeChunk) void k_tree_leaves(ElemInput in, BuildB
       if (n == 1) {
         *b.root = leaf;
         store_rootbox<false>(b, kd);
-      } else {
-        rec_store_half<false>(b, parent, side, kd, leaf, e);
+      } else {  // (the slabs: the wave together, below)
+        b.rec64[parent].child[side] = leaf;
+        b.rec64[parent].elem[side] = e;
       }
     }
   }
   if constexpr (FP32) {
     if (n > 1) store_leaf_halves32(b, L, t, act ? 2 * parent + (uint32_t)side : kEnd, e, c0, n);
   }
+  if constexpr (!FP32) {
+    if (n > 1) store_halves64(b, L, act ? 2 * parent + (uint32_t)side : kEnd, t);
+  }
   __syncthreads();  // counters, deltas and leaf slots ready
   if constexpr (FP32) climb_chunk32(b, n, act && n > 1, p, p, pk, c0, c1, L, own);
-  else if (act && n > 1) climb_chunk64(b, n, p, p, pk, c0, c1, L);
+  else climb_chunk64(b, n, act && n > 1, p, p, pk, c0, c1, L);
   __syncthreads();
   // a first arrival whose sibling lies outside the chunk leaves its arrival word
   if (c0 + t + 1 < c1 && L.far[t] != 0) {
