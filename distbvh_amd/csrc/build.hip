@@ -10,7 +10,7 @@
 //      -> k_morton (+ digit histograms of the sort)
 //  * radix_sorter, util/sort.hpp:75-144 -> sort.hip
 //  * morton_cluster splits, split/cluster.hpp:143-168
-//      -> k_cluster_depth + one 8-bit sort pass + k_cluster_select
+//      -> k_cluster_depth + k_cluster_count / _scan / _emit
 //  * patches (collision_object.cpp:134-141) and the tree
 //      -> k_delta + k_tree (Apetrei-style bottom-up build: each leaf climbs,
 //         the second child to reach a parent merges both children's slabs)

@@ -187,8 +187,8 @@ __device__ __forceinline__ uint32_t xcd_group_tile(uint32_t b, uint32_t nb, uint
 // slabs live in its parent's record (the root's in a separate array).
 // fp32 form: 256 B, read with scalar loads; fp64 form: 448 B, staged through
 // LDS by a wave-wide vector load.
-// Rec32: two 128-byte halves, one per child, each written as seven 16-byte
-// stores (slabs, child id, element) by the child that completes: a half is
+// Rec32: two 128-byte halves, one per child, each written in 16-byte
+// pieces (slabs, child id, element) by the child that completes: a half is
 // the child's ordered fp32 slab images (104 B), its node id and, for a leaf,
 // its input index; half 0 also holds this node's range and patch (one 16-byte
 // store by the node's completer).

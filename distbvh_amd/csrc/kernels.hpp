@@ -104,8 +104,8 @@ struct BuildBufs {
   uint8_t* delta;          // n-1
   uint32_t* patch_of_pos;  // n
   uint32_t* patch_of_input;// n
-  // n-1 arrival words: 0 before any child arrives, then the first arriver's
-  // far end + 1 (high word) and its patch (low word)
+  // n-1 arrival words: 0, or for a child whose sibling arrives in a later
+  // launch its far end + 1 (from bit 8 on) and the split height beyond it
   unsigned long long* counters;
   uint32_t* patch_root;    // od
   uint32_t* root;          // 1
@@ -332,9 +332,9 @@ struct PairOut {
 constexpr uint32_t kRecheckStripes = 64;
 constexpr uint32_t kRecheckStride = 16;  // counter words: one 128-byte line per stripe
 
-// launch shape of the narrowphase (tuned by the autotuner): threads per
-// block (64, 128 or 256), whether blocks are remapped so each XCD walks a
-// contiguous range of query tiles, and the fp64 walk's batch: 1 = one
+// launch shape of the narrowphase (tuned by the autotuner): the fp64 walk's
+// threads per block (64, 128 or 256; the fp32 walk's blocks are single waves),
+// whether neighbouring queries walk on one XCD, and the fp64 walk's batch: 1 = one
 // record per visit in scalar registers (k_narrow64s), 2 or 4 = that many
 // records per memory round trip loaded into LDS (k_narrow64; 2 by default,
 // the fastest on dense contact).  The fp32 walk always takes one record in

@@ -321,7 +321,8 @@ __device__ __forceinline__ void load_query32(const TreeView& q, const TreeView& 
 // or a run of such items.  The cross-patch walk is split: where meshes of
 // uneven sizes meet, a coarse element overlaps thousands of a fine mesh's, and
 // its wave alone (7,700 visits among 213 on average over 512 meshes of
-// lognormal size) held the launch for 4,577 us.  Split, it takes 1,465 + 1,092;
+// lognormal size) held the launch for 4,577 us.  Split, it took 1,465 + 1,092
+// (and takes 1,215 + 1,060 by the order of the waves and the early out);
 // with 128 or 64 visits before the split, or 32 or 128 leaves an item, 2,536 to
 // 2,661 us.  Evenly loaded walks lose by it (contact of 2 x 2M triangles 1,158
 // -> 1,271 us: the split's registers cost every visit) and stay whole.

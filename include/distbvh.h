@@ -450,7 +450,7 @@ typedef struct bvh_tuning {
 bvh_status bvh_autotune(bvh_object o, bvh_object other, bvh_tuning *best);
 /* Sets / reads the world's narrowphase launch shape (batch, block_size,
  * xcd_remap of a bvh_tuning; the other fields are ignored / zero).  Default:
- * batch 1, block 256, remap on.  No reference counterpart. */
+ * batch 2, block 256, remap on.  No reference counterpart. */
 bvh_status bvh_set_launch(bvh_world w, const bvh_tuning *shape);
 bvh_status bvh_get_launch(bvh_world w, bvh_tuning *shape);
 
