@@ -662,8 +662,11 @@ __global__ __launch_bounds__(kWave) void k_narrow32_batch(const BatchQuery* __re
   }
   const BatchQuery& e = bq[lo];
   if (b - e.block0 >= e.blocks) return;
-  walk32<false, false, kWalkWhole>(e.q, e.t, tile - 4 * e.block0, kWave, 0, 0, e.out, inner, L.buf, L.rbuf, L.stack,
-                                   nullptr, blockIdx.x % kRecheckStripes);
+  // (the stripe by the wave's number in its query: the blocks of one query's
+  // waves, 8 apart within a turn, would reach half the stripes or fewer)
+  const uint32_t wave = tile - 4 * e.block0;
+  walk32<false, false, kWalkWhole>(e.q, e.t, wave, kWave, 0, 0, e.out, inner, L.buf, L.rbuf, L.stack, nullptr,
+                                   wave % kRecheckStripes);
 }
 
 // Strict overlap of the lane's query slabs q with one box b whose 26 slabs
