@@ -4,6 +4,7 @@ expected ones throughout."""
 import numpy as np
 import pytest
 
+import oracle as O
 from distbvh_amd import CollisionWorld
 from helpers import sort_pairs, to_cuda
 
@@ -48,3 +49,52 @@ def test_batch_fills_every_stripe(n, precision):
             assert o.result_stats()["rechecked_pairs"] == copies * n
             assert np.array_equal(sort_pairs(o.pairs()), want)
         assert after == before
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("seed", [1, 2, 3])
+def test_cross_patch_replays_fill_the_same_stripes(seed, precision):
+    """A captured cross-patch step whose walk leaves subtrees to its second
+    launch, most of its re-check candidates in a few of them: 32 waves of large
+    spheres, each with its tops at one of 32 heights, over a sheet of small ones
+    in blocks at those heights (within a few fp32 ulps of touching, or well
+    inside, or missed).  The eager step sized the list, so every replay on the
+    same data fits, in whatever order the subtrees are written."""
+    from distbvh_amd import GIVEN
+    levels, side, size = 32, 64, 64.0
+    na, nb = 64 * levels, side * side
+    rng = np.random.default_rng(seed)
+    g, r, step = np.repeat(np.arange(levels), 64), 0.25 / side, 2.0 ** -5
+    big = np.stack([0.5 + 0.02 * g + 0.001 * rng.random(na), 0.5 + 0.001 * rng.random(na), g * step - size,
+                    np.full(na, size)])
+    gx, gy = np.meshgrid(np.arange(side), np.arange(side))
+    level = rng.permutation(levels)[(gy // 8 * 8 + gx // 8) % levels]
+    z = level * step + r + 4e-6 * (2.0 * rng.random(gx.shape) - 1.0)
+    small = np.stack([(gx + 0.5).reshape(-1) / side, (gy + 0.5).reshape(-1) / side, z.reshape(-1), np.full(nb, r)])
+    data = np.concatenate([big, small], axis=1)
+    kd, _ = O.elements_sphere(data)
+    want = sort_pairs(O.brute_pairs(kd[:na], kd[na:]))
+    want[:, 1] += np.uint64(na)
+    buf = to_cuda(np.ascontiguousarray(data))
+    with CollisionWorld(2, precision=precision) as w:
+        o = w.create_collision_object()
+        o.set_patch_offsets([na])
+
+        def step_():
+            o.set_entity_data_sphere(buf, split_algorithm=GIVEN)
+            o.init_broadphase()
+            o.self_collision_cross_patch()
+
+        step_()
+        assert np.array_equal(sort_pairs(o.pairs()), want)
+        # (the blocks at a wave's own height are its candidates)
+        assert o.result_stats()["rechecked_pairs"] > na * nb // levels // 2
+        with w.capture() as graph:
+            step_()
+        try:
+            for _ in range(40):
+                graph.launch()
+                assert o.result_count() == len(want)
+            assert np.array_equal(sort_pairs(o.pairs()), want)
+        finally:
+            graph.close()
