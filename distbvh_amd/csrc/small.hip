@@ -6,7 +6,8 @@
 // bounds, codes and boundaries stay in registers and LDS between them.  As
 // launches of their own these stages cost an object of 512 triangles ten
 // launches and their gaps, about 90 us of which 40 were the kernels; as one
-// launch they take 20 us.  One CU's memory and sorting rate sets the upper end
+// launch they take 20 us (with up to some hundred patches; what is cleared for each
+// patch is below).  One CU's memory and sorting rate sets the upper end
 // of the range: at 8,192 triangles the launch takes 60 us and a contact step of
 // two such objects 820 us, 804 as separate launches.
 #include "device.hpp"
@@ -71,7 +72,7 @@ __device__ __forceinline__ void element_bounds(const ElemInput& in, uint32_t e, 
 }  // namespace
 
 template <typename K, int ITEMS>
-__global__ __launch_bounds__(kSmallBlock) void k_build_small(ElemInput in, BuildBufs b) {
+__global__ __launch_bounds__(kSmallBlock) void k_build_small(ElemInput in, BuildBufs b, int clear_k64) {
   constexpr int kWaves = kSmallBlock / 64;
   constexpr int kPasses = sizeof(K);
   __shared__ SortBlockLds<K, ITEMS> L;
@@ -86,7 +87,7 @@ __global__ __launch_bounds__(kSmallBlock) void k_build_small(ElemInput in, Build
 
   // what later stages expect cleared
   for (uint64_t i = tid; i < b.od; i += kSmallBlock) b.patch_root[i] = kEnd;
-  if (b.rec64)
+  if (clear_k64)
     for (uint64_t i = tid; i < b.od * kSlabs; i += kSmallBlock) b.patch_k64[i] = (i & 1) ? 0ull : ~0ull;
   if (tid < 4) b.status[tid] = 0;
   if (tid == 0) *b.root = kEnd;
@@ -288,21 +289,32 @@ __global__ __launch_bounds__(kSmallBlock) void k_build_small(ElemInput in, Build
 }
 
 constexpr uint64_t kBuildSmallMax = 4 * kSmallBlock;
+// Patches up to which the one workgroup also clears the patch slabs of a build
+// with fp64 records (208 bytes each); above, a launch of its own does.  Build of
+// one sphere, cleared here / by a launch: 64 patches 80 / 88 us, 2,048 86 / 85,
+// 4,096 90 / 84, 16,384 126 / 86.
+constexpr uint64_t kClearSmallMax = 2048;
 bool build_is_small(uint64_t n) { return n > 0 && n <= kBuildSmallMax; }
 
 template <typename K>
-static void build_small(const ElemInput& in, const BuildBufs& b, hipStream_t s) {
+static void build_small(const ElemInput& in, const BuildBufs& b, int clear_k64, hipStream_t s) {
   const dim3 g(1), t(kSmallBlock);
-  if (in.n <= 1 * kSmallBlock) hipLaunchKernelGGL((k_build_small<K, 1>), g, t, 0, s, in, b);
-  else if (in.n <= 2 * kSmallBlock) hipLaunchKernelGGL((k_build_small<K, 2>), g, t, 0, s, in, b);
-  else hipLaunchKernelGGL((k_build_small<K, 4>), g, t, 0, s, in, b);
+  if (in.n <= 1 * kSmallBlock) hipLaunchKernelGGL((k_build_small<K, 1>), g, t, 0, s, in, b, clear_k64);
+  else if (in.n <= 2 * kSmallBlock) hipLaunchKernelGGL((k_build_small<K, 2>), g, t, 0, s, in, b, clear_k64);
+  else hipLaunchKernelGGL((k_build_small<K, 4>), g, t, 0, s, in, b, clear_k64);
 }
 
 hipError_t launch_build_small(const ElemInput& in, const BuildBufs& b, int bits, hipStream_t s) {
   if (!build_is_small(in.n) || in.nv < 1 || b.od < 1 || !in.data) return hipErrorInvalidValue;
   if (in.kind == kSnapshot && !in.centroids) return hipErrorInvalidValue;
-  if (bits == 63) build_small<uint64_t>(in, b, s);
-  else build_small<uint32_t>(in, b, s);
+  int clear_k64 = b.rec64 != nullptr;
+  if (clear_k64 && b.od > kClearSmallMax) {
+    const hipError_t e = launch_patch_k64_init(b.patch_k64, b.od, s);
+    if (e != hipSuccess) return e;
+    clear_k64 = 0;
+  }
+  if (bits == 63) build_small<uint64_t>(in, b, clear_k64, s);
+  else build_small<uint32_t>(in, b, clear_k64, s);
   return hipGetLastError();
 }
 
