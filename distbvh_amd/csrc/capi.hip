@@ -2610,13 +2610,15 @@ bvh_status bvh_autotune(bvh_object o, bvh_object other, bvh_tuning* best) {
   b.ms = -1.0;
   bvh_status st = BVH_OK;
   uint32_t k = 0;
-  // the fp32 walk takes one record per round trip (scalar registers)
-  const int nbatch = o->fp32 ? 1 : 3;
+  // the fp32 walk takes one record per round trip (scalar registers) and is
+  // launched in blocks of one wave: only its remap is timed, each time stands
+  // for the three block sizes, and the world keeps its block size
+  const int nbatch = o->fp32 ? 1 : 3, nblock = o->fp32 ? 1 : 3;
   for (int ki = 0; ki < nbatch && st == BVH_OK; ++ki)
-    for (int bi = 0; bi < 3 && st == BVH_OK; ++bi)
+    for (int bi = 0; bi < nblock && st == BVH_OK; ++bi)
       for (int xi = 0; xi < 2 && st == BVH_OK; ++xi) {
         w->shape.batch = o->fp32 ? keep_shape.batch : kBatch[ki];
-        w->shape.block = kBlock[bi];
+        w->shape.block = o->fp32 ? keep_shape.block : kBlock[bi];
         w->shape.xcd_remap = xi == 1;
         st = run_query(o, other, self, true, cross);  // sizes the buffers
         double t = 0.0;
@@ -2629,8 +2631,12 @@ bvh_status bvh_autotune(bvh_object o, bvh_object other, bvh_tuning* best) {
           (void)hipEventElapsedTime(&f, e0, e1);
           t = (r == 0 || f < t) ? f : t;
         }
-        if (k < 24) b.tried_ms[k] = t;
-        ++k;
+        if (o->fp32) {
+          for (int b3 = 0; b3 < 3; ++b3) b.tried_ms[2 * b3 + xi] = t;
+        } else if (k < 24) {
+          b.tried_ms[k] = t;
+        }
+        k += o->fp32 ? 3 : 1;
         if (st == BVH_OK && (b.ms < 0.0 || t < b.ms)) {
           b.ms = t;
           b.batch = w->shape.batch;

@@ -434,17 +434,20 @@ typedef struct bvh_tuning {
   uint32_t batch;       /* fp64 walk: 1 = one record per visit in scalar registers, 2 (default)
                            or 4 = that many records per memory round trip loaded into LDS */
   uint32_t block_size;  /* fp64 walk: threads per block, 64, 128 or 256 (the fp32 walk: one wave) */
-  uint32_t xcd_remap;   /* 1: neighbouring queries walk on one XCD, the XCDs take turns */
-  uint32_t tried;       /* configurations timed (entries of tried_ms) */
+  uint32_t xcd_remap;   /* 1: neighbouring queries walk on one XCD, the XCDs take turns
+                           (a batch's fp32 walk always, its fp64 walk never) */
+  uint32_t tried;       /* settings covered (entries of tried_ms) */
   double ms;            /* best query time */
   double tried_ms[24];  /* in the order batch (1, 2, 4) x block (64, 128, 256) x remap (off, on) */
 } bvh_tuning;
 /* Times the query o x other (self collision when o == other, cross-patch if
  * that was o's last query) over the batch
- * (1, 2, 4; fp64 form only: the fp32 walk takes one record per round trip),
- * block size (64, 128, 256) and XCD remap (off, on), best of 3 runs each,
- * keeps the fastest setting for the world and leaves that query's results in
- * o.  The pair set does not depend on the setting.
+ * (1, 2, 4), block size (64, 128, 256) and XCD remap (off, on), best of 3 runs
+ * each, keeps the fastest setting for the world and leaves that query's results
+ * in o.  The walk over fp32 records has neither a batch nor a block size: it is
+ * timed with the remap off and on, tried_ms holds these two times for each
+ * block size, and the world's batch and block size stay.  The pair set does
+ * not depend on the setting.
  * (No reference counterpart: the walk here is wave-wide and record-based,
  * and these are its tuning parameters.) */
 bvh_status bvh_autotune(bvh_object o, bvh_object other, bvh_tuning *best);

@@ -299,3 +299,21 @@ def test_cross_patch_graph_replays(torch_cuda):
                 assert o.digest() == pair_digest(wp)
         finally:
             g.close()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_autotune_leaves_what_the_fp32_walk_ignores(torch_cuda, precision):
+    """The walk over fp32 records runs one wave a block whatever the block size:
+    the tuner times it with the remap off and on, each time standing for the three
+    block sizes, and keeps the world's block size and batch."""
+    a, b = W.wavy_sheets(64)
+    with CollisionWorld(16, precision=precision) as w:
+        oa = gpu_object(w, "poly", a, device=True)
+        ob = gpu_object(w, "poly", b, device=True)
+        for batch, block in ((2, 256), (4, 64)):
+            w.set_launch(batch=batch, block_size=block, xcd_remap=False)
+            t = oa.autotune(ob)
+            assert (t["batch"], t["block_size"]) == (batch, block)
+            assert t["tried_ms"][:2] == t["tried_ms"][2:4] == t["tried_ms"][4:]
+            assert t["ms"] == min(t["tried_ms"]) == t["tried_ms"][int(t["xcd_remap"])]
+            assert w.launch() == {"batch": batch, "block_size": block, "xcd_remap": t["xcd_remap"]}
