@@ -83,11 +83,13 @@ struct DevBuf {
     p = nullptr;
     bytes = 0;
   }
-  bvh_status ensure(size_t want) {
+  // first_counts = false: captured work gets by without this buffer, so that
+  // its first allocation leaves graphs launchable
+  bvh_status ensure(size_t want, bool first_counts = true) {
     if (want <= bytes && p) return BVH_OK;
     if (t_capturing)
       return fail(BVH_E_STATE, "a device buffer would grow inside a capture: run the step once before capturing");
-    gen->fetch_add(1);
+    if (p || first_counts) gen->fetch_add(1);
     if (p) {
       (void)hipFree(p);
       p = nullptr;
@@ -378,6 +380,9 @@ static bvh_status copy_out(void* dst, const void* src, size_t bytes, uint32_t me
   return BVH_OK;
 }
 
+// first size of the fp32 walk's re-check and split lists
+static uint64_t split_list_bytes(const bvh_object_s* o) { return std::max<uint64_t>(1u << 16, o->in.n) * 8; }
+
 static bvh_status object_alloc(bvh_object_s* o) {
   const uint64_t n = o->in.n;
   const uint64_t od = o->w->od;
@@ -417,6 +422,8 @@ static bvh_status object_alloc(bvh_object_s* o) {
     BVH_TRY(o->rootbox32.ensure(kSlabs * sizeof(int32_t)));
     BVH_TRY(o->frame.ensure(16 * sizeof(double)));
     BVH_TRY(o->patch_box32.ensure(od * kSlabs * sizeof(int32_t)));
+    // (a split list grows here, with the buffers that end the graphs anyway)
+    if (o->items.p) BVH_TRY(o->items.ensure(split_list_bytes(o)));
   } else {
     BVH_TRY(o->rec64.ensure((n1 > 1 ? n1 - 1 : 1) * sizeof(Rec64)));
     BVH_TRY(o->rootbox64.ensure(kSlabs * sizeof(double)));
@@ -1049,13 +1056,14 @@ static bvh_status grow_query_lists(bvh_object_s* o) {
   return BVH_OK;
 }
 
-// The fp32 walk's lists at their first sizes.  The split list is there from the
-// first query of any kind, so that a capture finds it.
-static bvh_status first_query_lists(bvh_object_s* o) {
+// The fp32 walk's lists at their first sizes.  The split list comes with the
+// first eager cross-patch query; a step captured before walks without one.
+static bvh_status first_query_lists(bvh_object_s* o, bool cross) {
   if (!o->fp32) return BVH_OK;
-  const uint64_t bytes = std::max<uint64_t>(1u << 16, o->in.n) * 8;
+  const uint64_t bytes = split_list_bytes(o);
   BVH_TRY(o->recheck.ensure(bytes));
-  return o->items.ensure(bytes);
+  if (!cross || o->w->capturing) return BVH_OK;
+  return o->items.ensure(bytes, false);
 }
 
 static bvh_status run_query(bvh_object_s* o, bvh_object_s* other, bool self, bool narrow = true, bool cross = false) {
@@ -1070,7 +1078,7 @@ static bvh_status run_query(bvh_object_s* o, bvh_object_s* other, bool self, boo
   BVH_TRY(o->ppairs.ensure(std::max<uint64_t>(1024, 4 * w->od) * 8));
   if (narrow) {
     BVH_TRY(ensure_pairs(o, std::max<uint64_t>(1u << 20, 8 * o->in.n)));
-    BVH_TRY(first_query_lists(o));
+    BVH_TRY(first_query_lists(o, self && cross));
   }
   if (w->capturing) {
     BVH_TRY(launch_query(o, other, self, narrow, cross));
@@ -1116,7 +1124,7 @@ static bvh_status run_query_batch(bvh_object_s* const* os, bvh_object_s* const* 
     BVH_TRY(o->count.ensure(kCntTotal * sizeof(unsigned long long)));
     BVH_TRY(o->ppairs.ensure(std::max<uint64_t>(1024, 4 * w->od) * 8));
     BVH_TRY(ensure_pairs(o, std::max<uint64_t>(1u << 20, 8 * o->in.n)));
-    BVH_TRY(first_query_lists(o));
+    BVH_TRY(first_query_lists(o, false));
   }
   // (a batch ends synchronized, unless it failed)
   if (w->bq_busy) HIP_TRY(hipStreamSynchronize(s));

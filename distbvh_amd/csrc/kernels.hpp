@@ -323,7 +323,8 @@ struct PairOut {
   unsigned long long* rcount;
   unsigned long long* rtotal;
   // fp32 cross-patch walk: the split list (subtrees that a wave leaves to a
-  // second launch) and its length, which may pass icap
+  // second launch; icap 0: none, every wave walks its own) and its length,
+  // which may pass icap
   uint64_t* items;
   uint64_t icap;
   unsigned long long* icount;

@@ -1382,9 +1382,10 @@ hipError_t launch_narrowphase(const TreeView& q, const TreeView& t, int leaf_siz
     const int32_t inner = kInnerUlps;
     const dim3 g(waves), bl(kWave);
     if (self == 2) {
-      if (!out.items || !out.icount) return hipErrorInvalidValue;
+      if ((out.icap && !out.items) || !out.icount) return hipErrorInvalidValue;
       hipLaunchKernelGGL((k_narrow32<true, true, kWalkTop>), g, bl, 0, s, q, t, xcd, qper, out, inner);
-      hipLaunchKernelGGL((k_narrow32_items<true, true>), dim3(kItemBlocks), bl, 0, s, q, t, qper, out, inner);
+      if (out.icap)
+        hipLaunchKernelGGL((k_narrow32_items<true, true>), dim3(kItemBlocks), bl, 0, s, q, t, qper, out, inner);
     } else if (self) {
       hipLaunchKernelGGL((k_narrow32<true, false>), g, bl, 0, s, q, t, xcd, qper, out, inner);
     } else {

@@ -98,3 +98,52 @@ def test_cross_patch_replays_fill_the_same_stripes(seed, precision):
             assert np.array_equal(sort_pairs(o.pairs()), want)
         finally:
             graph.close()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_split_list_comes_with_the_first_cross_patch_query(precision):
+    """Only a cross-patch query allocates the split list (65,536 entries at
+    least).  Its first one leaves earlier graphs launchable, and a cross-patch step
+    captured before it walks without a list: same pairs."""
+    from distbvh_amd import GIVEN
+    rng = np.random.default_rng(7)
+    na, nb = 700, 3000
+    data = np.concatenate([rng.random((3, na + nb)), rng.random((1, na + nb)) * 0.02])
+    data[0, na:] += 2.0  # apart but for every 40th of the first patch
+    data[3, :na:40] = 6.0
+    (kd, _) = O.elements_sphere(data)
+    own = sort_pairs(O.brute_self(kd))
+    cross = own[(own[:, 0] < na) & (own[:, 1] >= na)]
+    assert 0 < len(cross) < len(own)
+    buf = to_cuda(np.ascontiguousarray(data))
+    with CollisionWorld(2, precision=precision) as w:
+        o = w.create_collision_object()
+        o.set_patch_offsets([na])
+
+        def step(query):
+            o.set_entity_data_sphere(buf, split_algorithm=GIVEN)
+            o.init_broadphase()
+            query()
+
+        graphs = []
+        try:
+            step(o.self_collision)
+            assert np.array_equal(sort_pairs(o.pairs()), own)
+            for query, want in ((o.self_collision, own), (o.self_collision_cross_patch, cross)):
+                with w.capture() as graph:
+                    step(query)
+                graphs.append((graph, want))
+            before = o.device_bytes()
+            step(o.self_collision)
+            assert o.device_bytes() == before
+            step(o.self_collision_cross_patch)
+            assert o.device_bytes() == before + 65536 * 8
+            assert np.array_equal(sort_pairs(o.pairs()), cross)
+            for _ in range(3):
+                for graph, want in graphs:
+                    graph.launch()
+                    assert o.result_count() == len(want)
+                    assert np.array_equal(sort_pairs(o.pairs()), want)
+        finally:
+            for graph, _ in graphs:
+                graph.close()
