@@ -1238,28 +1238,35 @@ __global__ __launch_bounds__(256) void k_records(const uint64_t* __restrict__ pa
 // element's two dependent loads in the chain, took 1,703 us on 32 patches of
 // 4,096 triangles on average; this takes 45 us.
 constexpr uint32_t kCentroidItems = 4;
-constexpr uint32_t kCentroidChunk = 256 * kCentroidItems;
-__global__ __launch_bounds__(256) void k_patch_centroids(const double* __restrict__ planes,
-                                                         const double* __restrict__ caos,
-                                                         const uint32_t* __restrict__ perm,
-                                                         const uint32_t* __restrict__ splits, uint64_t n,
-                                                         uint64_t od, double* __restrict__ out) {
-  __shared__ double buf[2][3][kCentroidChunk];
-  const uint64_t k = blockIdx.x;
-  const uint32_t b = (k == 0) ? 0u : splits[k - 1];
-  const uint32_t e = (k == od - 1) ? (uint32_t)n : splits[k];
-  const uint32_t t = threadIdx.x;
-  if (e <= b) {  // an empty patch
-    if (t < 3) out[3 * k + t] = 0.0;
-    return;
-  }
-  const uint32_t cnt = e - b, nchunk = (cnt + kCentroidChunk - 1) / kCentroidChunk;
+template <uint32_t BLOCK>
+struct CentroidLds {
+  static constexpr uint32_t chunk = BLOCK * kCentroidItems;
+  double v[2][3][chunk];
+};
+// positions of patch k
+__device__ __forceinline__ void patch_range(const uint32_t* splits, uint64_t n, uint64_t od, uint64_t k, uint32_t& b,
+                                            uint32_t& e) {
+  b = (k == 0) ? 0u : splits[k - 1];
+  e = (k == od - 1) ? (uint32_t)n : splits[k];
+}
+__device__ __forceinline__ double centroid_coord(const double* planes, const double* caos, uint64_t n, uint32_t src,
+                                                 uint32_t c) {
+  return planes ? planes[(uint64_t)c * n + src] : caos[3 * (uint64_t)src + c];
+}
+
+// one patch of cnt > 0 elements from position b on, by the whole block
+template <uint32_t BLOCK>
+__device__ __forceinline__ void block_centroid(const double* __restrict__ planes, const double* __restrict__ caos,
+                                               const uint32_t* __restrict__ perm, uint64_t n, uint64_t k, uint32_t b,
+                                               uint32_t cnt, double* __restrict__ out, CentroidLds<BLOCK>& L) {
+  constexpr uint32_t kChunk = CentroidLds<BLOCK>::chunk;
+  const uint32_t t = threadIdx.x, nchunk = (cnt + kChunk - 1) / kChunk;
   uint32_t src[kCentroidItems];
   double v[kCentroidItems][3];
   auto load_src = [&](uint32_t chunk) {
 #pragma unroll
     for (uint32_t j = 0; j < kCentroidItems; ++j) {
-      const uint32_t i = chunk * kCentroidChunk + j * 256 + t;
+      const uint32_t i = chunk * kChunk + j * BLOCK + t;
       src[j] = i < cnt ? perm[b + i] : kEnd;
     }
   };
@@ -1267,30 +1274,89 @@ __global__ __launch_bounds__(256) void k_patch_centroids(const double* __restric
 #pragma unroll
     for (uint32_t j = 0; j < kCentroidItems; ++j)
 #pragma unroll
-      for (int c = 0; c < 3; ++c)
-        v[j][c] = src[j] == kEnd ? 0.0 : (planes ? planes[(uint64_t)c * n + src[j]] : caos[3 * (uint64_t)src[j] + c]);
+      for (int c = 0; c < 3; ++c) v[j][c] = src[j] == kEnd ? 0.0 : centroid_coord(planes, caos, n, src[j], c);
   };
   load_src(0);
   load_val();
   load_src(1);
   double s = 0.0;
   for (uint32_t q = 0; q < nchunk; ++q) {
-    double(*cur)[kCentroidChunk] = buf[q & 1];
+    double(*cur)[kChunk] = L.v[q & 1];
 #pragma unroll
     for (uint32_t j = 0; j < kCentroidItems; ++j)
 #pragma unroll
-      for (int c = 0; c < 3; ++c) cur[c][j * 256 + t] = v[j][c];
+      for (int c = 0; c < 3; ++c) cur[c][j * BLOCK + t] = v[j][c];
     load_val();
     load_src(q + 2);
     // one barrier per chunk: the chunk staged next goes to the other buffer,
     // whose adds ended before every thread's arrival here
     __syncthreads();
     if (t < 3) {
-      const uint32_t left = cnt - q * kCentroidChunk;
-      s = ordered_sum(cur[t], left < kCentroidChunk ? left : kCentroidChunk, s);
+      const uint32_t left = cnt - q * kChunk;
+      s = ordered_sum(cur[t], left < kChunk ? left : kChunk, s);
     }
   }
   if (t < 3) out[3 * k + t] = s / (double)cnt;
+}
+
+__global__ __launch_bounds__(256) void k_patch_centroids(const double* __restrict__ planes,
+                                                         const double* __restrict__ caos,
+                                                         const uint32_t* __restrict__ perm,
+                                                         const uint32_t* __restrict__ splits, uint64_t n,
+                                                         uint64_t od, double* __restrict__ out) {
+  __shared__ CentroidLds<256> L;
+  const uint64_t k = blockIdx.x;
+  uint32_t b, e;
+  patch_range(splits, n, od, k, b, e);
+  if (e <= b) {  // an empty patch
+    if (threadIdx.x < 3) out[3 * k + threadIdx.x] = 0.0;
+    return;
+  }
+  block_centroid<256>(planes, caos, perm, n, k, b, e - b, out, L);
+}
+
+// Many patches of few elements: 16 patches a wave, four lanes each, of which
+// three add a coordinate straight from memory, kFewBatch loads together.  A
+// patch of more than kFewElems elements is left to the wave as a whole.  The
+// wave's patches are gridDim.x apart, so that large neighbours are not one
+// wave's.
+constexpr uint32_t kFewPatches = 16;
+constexpr uint32_t kFewElems = 128;
+constexpr uint32_t kFewBatch = 8;
+__global__ __launch_bounds__(kWave) void k_patch_centroids_few(const double* __restrict__ planes,
+                                                               const double* __restrict__ caos,
+                                                               const uint32_t* __restrict__ perm,
+                                                               const uint32_t* __restrict__ splits, uint64_t n,
+                                                               uint64_t od, double* __restrict__ out) {
+  __shared__ CentroidLds<kWave> L;
+  const uint32_t c = threadIdx.x & 3;
+  const uint64_t k = (uint64_t)(threadIdx.x >> 2) * gridDim.x + blockIdx.x;
+  uint32_t b = 0, e = 0;
+  if (k < od) patch_range(splits, n, od, k, b, e);
+  const uint32_t cnt = e > b ? e - b : 0u;
+  if (k < od && cnt <= kFewElems && c < 3) {
+    double s = 0.0;
+    for (uint32_t i = 0; i < cnt; i += kFewBatch) {
+      uint32_t src[kFewBatch];
+      double v[kFewBatch];
+#pragma unroll
+      for (uint32_t j = 0; j < kFewBatch; ++j) src[j] = i + j < cnt ? perm[b + i + j] : kEnd;
+#pragma unroll
+      for (uint32_t j = 0; j < kFewBatch; ++j) v[j] = src[j] == kEnd ? 0.0 : centroid_coord(planes, caos, n, src[j], c);
+#pragma unroll
+      for (uint32_t j = 0; j < kFewBatch; ++j)
+        if (i + j < cnt) s = s + v[j];
+    }
+    out[3 * k + c] = cnt ? s / (double)cnt : 0.0;
+  }
+  uint64_t large = __ballot(c == 0 && cnt > kFewElems);
+  while (large) {  // (uniform)
+    const int l = __builtin_ctzll(large);
+    large &= large - 1;
+    block_centroid<kWave>(planes, caos, perm, n, (uint64_t)(l >> 2) * gridDim.x + blockIdx.x,
+                          (uint32_t)__shfl((int)b, l, kWave), (uint32_t)__shfl((int)cnt, l, kWave), out, L);
+    __syncthreads();  // L is free again
+  }
 }
 
 // Order-independent digest of a pair list: the sum and the xor of two
@@ -1519,11 +1585,22 @@ hipError_t launch_digest(const uint64_t* pairs, uint64_t count, unsigned long lo
   return hipGetLastError();
 }
 
+// Where the patches are many and small, a block each is mostly the cost of its
+// launch: the whole call that packs them takes, with a block a patch / four lanes
+// a patch, 63 / 26 us for 131,072 elements in 16,384 patches, 80 / 43 for a million in
+// 16,384, 34 / 27 for 131,072 in 4,096 and 30 / 30 in 2,048 (an average of 64),
+// but 27 / 86 in 512 and 49 / 84 for a million in 4,096.
+constexpr uint64_t kFewPatchesMin = 1024;
+constexpr uint64_t kFewAverage = 64;
 hipError_t launch_patch_centroids(const double* planes, const double* caos, const uint32_t* perm,
                                   const uint32_t* splits, uint64_t n, uint64_t od, double* out, hipStream_t s) {
   if (od == 0) return hipSuccess;
   if (!out || (n && ((!planes && !caos) || !perm)) || (od > 1 && !splits)) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_patch_centroids, dim3((unsigned)od), dim3(256), 0, s, planes, caos, perm, splits, n, od, out);
+  if (od >= kFewPatchesMin && n <= kFewAverage * od)
+    hipLaunchKernelGGL(k_patch_centroids_few, dim3((unsigned)((od + kFewPatches - 1) / kFewPatches)), dim3(kWave), 0, s,
+                       planes, caos, perm, splits, n, od, out);
+  else
+    hipLaunchKernelGGL(k_patch_centroids, dim3((unsigned)od), dim3(256), 0, s, planes, caos, perm, splits, n, od, out);
   return hipGetLastError();
 }
 

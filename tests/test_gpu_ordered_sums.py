@@ -50,6 +50,61 @@ def test_patch_centroids_at_chunk_edges(kind):
         assert np.array_equal(got[k]["centroid"], want), (k, m)
 
 
+@pytest.mark.parametrize("kind", ["sphere", "snapshot"])
+@pytest.mark.parametrize("od,extra", [(512, 0), (1024, 0), (2048, 0), (2048, 70), (16384, 0)])
+def test_centroids_of_many_patches(od, extra, kind):
+    """Patches of few elements (four lanes each from 1,024 patches on, while they
+    hold at most 64 elements on average), at the sizes where a lane's batches end,
+    with large ones side by side, first, last and a block's number of patches apart."""
+    rng = np.random.default_rng(od + extra)
+    sizes = rng.choice([0, 0, 1, 2, 7, 8, 9, 15, 16, 17, 40], size=od) + extra
+    for k, m in {0: 128, 1: 129, 2: 255, 3: 256, 4: 257, 5: 700, od // 16: 130, od // 2: 127, od // 2 + od // 16: 300,
+                 od - 2: 2000, od - 1: 129}.items():
+        sizes[k] = m
+    n = int(sizes.sum())
+    c = rng.normal(size=(3, n)) * 10.0 ** rng.integers(-3, 4, size=n) + np.array([[1e3], [-2e3], [0.0]])
+    with CollisionWorld(od) as w:
+        o = w.create_collision_object()
+        o.set_patch_offsets(np.cumsum(sizes)[:-1])
+        if kind == "sphere":
+            o.set_entity_data_sphere(to_cuda(np.concatenate([c, np.full((1, n), 0.5)])), split_algorithm=GIVEN)
+        else:
+            kd = np.repeat(rng.normal(size=(n, 13)), 2, axis=1)
+            kd[:, 1::2] += 1.0
+            o.set_entity_data_snapshot(to_cuda(kd), to_cuda(c.T), split_algorithm=GIVEN)
+        got = o.local_patches()
+    off = np.concatenate([[0], np.cumsum(sizes)])
+    for k, m in enumerate(sizes):
+        want = _ordered_mean(c[:, off[k]:off[k + 1]]) if m else np.zeros(3)
+        assert got[k]["size"] == m
+        assert np.array_equal(got[k]["centroid"], want), (k, m)
+
+
+def test_packing_time_does_not_follow_the_patches():
+    """Packing 16,384 patches of one element takes about as long as 512 patches
+    of 32 (25 against 24 us; 56 with a block for each patch)."""
+    import time
+    n, best = 16384, {512: 1e9, 16384: 1e9}
+    data = to_cuda(np.concatenate([np.random.default_rng(1).random((3, n)), np.full((1, n), 0.01)]))
+    worlds = {od: CollisionWorld(od) for od in best}
+    try:
+        objs = {od: w.create_collision_object() for od, w in worlds.items()}
+        for od, o in objs.items():
+            o.set_patch_offsets(np.arange(1, od) * (n // od))
+            o.set_entity_data_sphere(data, split_algorithm=GIVEN)
+            o.init_broadphase()
+        for _ in range(200):
+            for od, o in objs.items():
+                t = time.perf_counter()
+                o.pack_patches(device=True)
+                worlds[od].synchronize()
+                best[od] = min(best[od], time.perf_counter() - t)
+    finally:
+        for w in worlds.values():
+            w.close()
+    assert best[16384] < 1.5 * best[512], best
+
+
 def _split_line(kind, n, rng):
     """x of n points whose mean is one of them, so that the rounded sum decides."""
     k = np.arange(n) - (n - 1) // 2
