@@ -612,11 +612,11 @@ __device__ __forceinline__ void walk32(const TreeView& q, const TreeView& t, uin
   recheck_flush(rbuf, rfill, out, rstripe);
   sink += pf;
   asm volatile("; record prefetch sink %0" ::"v"(sink));  // keeps the prefetch loads
-  // the counts go to a stripe's line, and k_recheck adds the lines up; those of
-  // items to any, so that neighbours don't queue (512-mesh step 3,368 -> 3,345 us)
+  // the counts go to a stripe's line, the block's (neighbours on one line queue:
+  // those of items by their own wave's took the 512-mesh step from 3,345 to
+  // 3,368 us), and k_recheck adds the lines up
   if (lane == 0) {
-    const uint32_t ls = MODE == kWalkItems ? blockIdx.x % kRecheckStripes : rstripe;
-    unsigned long long* line = out.rcount + (uint64_t)ls * kRecheckStride;
+    unsigned long long* line = out.rcount + (uint64_t)(blockIdx.x % kRecheckStripes) * kRecheckStride;
     atomicAdd(line + 1, (unsigned long long)(MODE == kWalkItems ? total : steps));
     atomicAdd(line + 2, (unsigned long long)ncand);
   }
