@@ -3,16 +3,16 @@
 //
 // Stage map (reference file:line -> kernel):
 //  * per-element 26-DOP + centroid, kdop.hpp:238-288 / TestCommon.hpp:62-73
-//      -> k_prep (centroid, cardinal bounds), k_tree (slabs, in sorted order)
+//      -> k_prep (centroid, cardinal bounds), k_tree_leaves (slabs, in sorted order)
 //  * compute_bounds(min_inv_diag), contact_entity.hpp:136-148
-//      -> k_prep block reduction + last-block finalize
+//      -> k_prep block partials + k_prep_final
 //  * morton(view, bounds, codes), contact_entity.hpp:157-191, hash.hpp
 //      -> k_morton (+ digit histograms of the sort)
 //  * radix_sorter, util/sort.hpp:75-144 -> sort.hip
 //  * morton_cluster splits, split/cluster.hpp:143-168
 //      -> k_cluster_depth + k_cluster_count / _scan / _emit
 //  * patches (collision_object.cpp:134-141) and the tree
-//      -> k_delta + k_tree (Apetrei-style bottom-up build: each leaf climbs,
+//      -> k_delta + k_tree_leaves / k_tree_up (Apetrei-style bottom-up build: each leaf climbs,
 //         the second child to reach a parent merges both children's slabs)
 //
 // The tree is the binary radix tree of the augmented keys
@@ -722,8 +722,9 @@ __device__ __forceinline__ bool is_patch_root(uint32_t patch, uint32_t l, uint32
 }
 
 // leaves per phase-1 workgroup (and the growth factor of the upper phases):
-// 128 leaves keep the phase-1 LDS at 30 KB, three workgroups per CU (measured:
-// 612 us per 2M-triangle tree instead of 653 at 256)
+// with 128, phase 1 takes 14 KB of LDS over fp32 records (eleven workgroups a CU
+// by it) and 28 KB over fp64 ones (five).  Measured with 30 KB: 612 us per
+// 2M-triangle tree instead of 653 at 256 leaves; 64 were slower too
 constexpr uint32_t kTreeChunk = kTreeLeafChunk;
 
 // LDS of an upper phase's workgroup: per thread (slot) the node it has
@@ -959,13 +960,13 @@ __global__ void k_patch_k64_init(unsigned long long* pk64, uint64_t count) {
 // written to its first position's slot, which only the thread that has just read
 // it overwrites.  far[j] is the far end of the first child to arrive at internal
 // node c0 + j, plus one (0: none yet).  What else a sibling needs to know follows
-// from it, so the slabs are most of this: 14.6 KB (fp32), 11 chunks a CU.
+// from it, so the slabs are most of this: 14.2 KB (fp32), 11 chunks a CU.
 template <bool FP32>
 struct ChunkLds {
   SlabT<FP32> slab[kSlabs][kTreeChunk + 1];  // SoA, rows padded: conflict-free stores, and column reads
   uint32_t far[kTreeChunk];
   uint8_t delta[kTreeChunk + 1];  // delta[c0 - 1 + j]
-  uint8_t order[kTreeChunk];      // fp32 climb: per wave, the lanes that formed a node at this level
+  uint8_t order[kTreeChunk];      // ordered stores: per wave, the lanes that formed a node at this level
   FrontNode front[2];
   uint32_t nfront;
 };
@@ -1136,7 +1137,7 @@ __device__ __forceinline__ void store_level32(const BuildBufs& b, ChunkLds<true>
   }
 }
 
-// The fp32 phase-1 climb (climb_chunk's steps), wave-synchronous: every lane
+// The fp32 phase-1 climb, wave-synchronous: every lane
 // of the wave runs each level, lanes whose climb has ended idle, so that the
 // level's record stores go out together (store_level32).  alive: the lane
 // holds leaf l = r (its slabs in own and in its LDS slot).
@@ -1345,7 +1346,7 @@ __global__ __launch_bounds__(kTreeChunk) void k_tree_leaves(ElemInput in, BuildB
   }
   L.far[t] = 0;
   {
-    // delta[c0 - 1 + t] for t in [0, 256], where the index is in [0, n - 2]
+    // delta[c0 - 1 + t] for t in [0, kTreeChunk], where the index is in [0, n - 2]
     const uint64_t di = (uint64_t)c0 + t;  // = (c0 - 1 + t) + 1
     L.delta[t] = (di >= 1 && di - 1 < n - 1) ? b.delta[di - 1] : 0;
     if (t == 0) {

@@ -1107,12 +1107,12 @@ static bvh_status run_query(bvh_object_s* o, bvh_object_s* other, bool self, boo
   return BVH_OK;
 }
 
-// Several object pairs o[i] x other[i] in one coalesced step: their counters
-// cleared and patch broadphases run per pair, then every element
-// narrowphase in one launch (k_narrow64_batch / k_narrow32_batch), then one synchronization
-// for all their counters.  A pair whose lists overflowed runs again on its
-// own with grown buffers.  The fp32-outward forms add one re-check launch per
-// pair after the walk.
+// Several object pairs o[i] x other[i] in one coalesced step: all their counters
+// cleared in one launch, every element narrowphase in one (k_narrow64_batch /
+// k_narrow32_batch), their counts written to the host by one, and one
+// synchronization.  Patch pairs are computed when asked for.  A pair whose lists
+// overflowed runs again on its own with grown buffers.  The fp32-outward forms
+// add one re-check launch per pair after the walk.
 static bvh_status run_query_batch(bvh_object_s* const* os, bvh_object_s* const* others, uint64_t k) {
   bvh_world w = os[0]->w;
   hipStream_t s = w->stream;

@@ -368,10 +368,6 @@ struct BatchQuery {
   uint32_t block0;
   uint32_t blocks;
 };
-// the pair walks of nq queries (no self) in one launch of `blocks` blocks of 256
-// threads (the fp32-outward walk: four of one wave each); bq in device memory; batch 2 or 4 for the
-// walk over fp64 records.  The fp32-outward forms leave their re-check
-// lists to launch_recheck_query, one launch per query.
 // na, nb and nc 8-byte words of device memory (at most 64, 8-byte aligned), one
 // run after the other, into host (pinned, device-accessible) memory
 hipError_t launch_readback(const void* a, int na, const void* b, int nb, const void* c, int nc,
@@ -383,6 +379,10 @@ hipError_t launch_batch_clear(const BatchQuery* bq, uint32_t nq, uint32_t words,
 constexpr uint32_t kReadbackWords = 16;
 hipError_t launch_batch_readback(const BatchQuery* bq, uint32_t nq, int ncount, unsigned long long* host,
                                  hipStream_t s);
+// the pair walks of nq queries (no self) in one launch of `blocks` blocks of 256
+// threads (the fp32-outward walk: four of one wave each); bq in device memory; batch 2 or 4 for the
+// walk over fp64 records.  The fp32-outward forms leave their re-check
+// lists to launch_recheck_query, one launch per query.
 hipError_t launch_narrowphase_batch(const BatchQuery* bq, uint32_t nq, uint32_t blocks, int batch, int form,
                                     hipStream_t s);
 hipError_t launch_recheck_query(const TreeView& q, const TreeView& t, const PairOut& out, hipStream_t s);

@@ -254,7 +254,7 @@ __device__ __forceinline__ void recheck_flush(uint64_t* buf, uint32_t& fill, con
 // the start of a self walk meets more than its end.  With 1,024 queries in turn
 // the 2 x 2M walk takes 933 us instead of 1,038 (931 / 947 with 4,096 / 16,384 in
 // a row), the 512-mesh walk 1,215 instead of 1,259 (1,256 / 1,310), the 2 x 524k
-// walk over fp64 records 568 instead of 612; tiles that share lines still run on
+// walk over fp64 records 433 instead of 474; tiles that share lines still run on
 // one XCD.
 constexpr uint32_t kXcdQueries = 1024;
 
@@ -322,7 +322,7 @@ __device__ __forceinline__ void load_query32(const TreeView& q, const TreeView& 
 // uneven sizes meet, a coarse element overlaps thousands of a fine mesh's, and
 // its wave alone (7,700 visits among 213 on average over 512 meshes of
 // lognormal size) held the launch for 4,577 us.  Split, it took 1,465 + 1,092
-// (and takes 1,215 + 1,060 by the order of the waves and the early out);
+// (and takes 1,215 + 1,020 by the order of the waves and the early out);
 // with 128 or 64 visits before the split, or 32 or 128 leaves an item, 2,536 to
 // 2,661 us.  Evenly loaded walks lose by it (contact of 2 x 2M triangles 1,158
 // -> 1,271 us: the split's registers cost every visit) and stay whole.

@@ -33,8 +33,11 @@ namespace dbvh {
 // and the digit runs written are twice as long.  Per 8-bit pass of u64 keys
 // with payloads, narrow / wide: 54,612 keys 9.1 / 13.8 us, 524,288 13.7 / 17.3,
 // 2,097,152 25.0 / 23.4, 12,000,017 104.9 / 81.3 (one shape of 256 threads x
-// 16 keys: 13.3, 18.0, 28.8, 118.7): the line lies between the last two of
-// these sizes where the wide one wins.
+// 16 keys: 13.3, 18.0, 28.8, 118.7).  The line is where whole sorts cross, for
+// both key widths, with and without payload (narrow / wide, us): u64 pairs 202 /
+// 214 at 1,048,576 keys, 226 / 227 at 1,500,000, 242 / 228 at 1,650,000; u64 keys
+// 187 / 193, 215 / 216, 228 / 218; u32 pairs 118 / 127, 133 / 136, 141 / 137; u32
+// keys 110 / 116, 123 / 124, 133 / 127.
 template <bool WIDE>
 struct SortShape {
   static constexpr int block = WIDE ? 512 : 1024;

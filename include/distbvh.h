@@ -143,7 +143,10 @@ bvh_status bvh_synchronize(bvh_world w);
 bvh_status bvh_world_stream(bvh_world w, void **stream);
 /* Per-stage device times (ms) recorded (BVH_FLAG_TIMING) since the previous
  * call of this function, in call order; reading clears the record (at most
- * 512 stages are kept).  names[i] gets a static string. */
+ * 512 stages are kept).  names[i] gets a static string.  A world that records
+ * times builds every object in separate launches; another builds an object of
+ * at most 4,096 elements (clustering) in one launch up to its tree, so that the
+ * sum of these times is more than such a build takes there. */
 bvh_status bvh_stage_times(bvh_world w, const char **names, double *ms, size_t cap, size_t *count);
 
 /* ---- collision object (collision_object.hpp:55-283) --------------------------- */
